@@ -295,6 +295,15 @@ Launch current_launch(dice_hip_context *ctx, int mode) {
   }
   const int max_groups = (ctx->n + L.waves_per_group - 1) / L.waves_per_group;
   if (L.groups > max_groups) L.groups = max_groups > 0 ? max_groups : 1;
+  L.num_cus = ctx->num_cus;
+  // the wide kernel's window: the largest subset with the interpolation's
+  // support and a few pixels of stretch, up to 56 KB (larger windows fall back
+  // to taps from the image there)
+  const long long ws = ctx->max_side + 10;
+  L.wide_floats = (int)std::min<long long>(ws * ws, 14336);
+  // square subsets whose window would outgrow a wave's slot even compressed by a fifth
+  const long long small = (long long)(0.8 * ctx->S) + 1;
+  L.wide_only = ctx->S > 0 && small * small > L.lds_floats_per_wave ? 1 : 0;
   L.lane_simplex = ctx->max_count <= dice_hip::kLaneSimplexMaxPixels ? std::max(ctx->max_count, 1) : 0;
   return L;
 }

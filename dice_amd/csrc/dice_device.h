@@ -25,8 +25,10 @@
 //             (at most ceil(N/64) pixels each) that are added across lanes in
 //             FP64 through an LDS transpose; the 6x6 system is solved in FP64
 //             with one row per lane.  No barriers: a wave synchronises itself.
-//             A subset whose window does not fit the slot is handed over to the
-//             PLAIN kernel (overflow list) and restarted there.
+//             A subset whose window does not fit the slot is handed over
+//             (overflow list) and restarted in the third shape.
+//   TEAM    : a workgroup per subset with the window in LDS and PLAIN's FP64
+//             sums (correlate_wide_kernel).
 #pragma once
 #include "dice_kernels.h"
 
@@ -128,6 +130,7 @@ __device__ __forceinline__ int opaque_lane(int lane) {
 struct WaveGroup {
   int lane;
   static constexpr int kSize = kWave;
+  static constexpr bool kWindow = true;
   __device__ __forceinline__ int rank() const { return opaque_lane(lane); }
   __device__ __forceinline__ void sync() const {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -154,6 +157,7 @@ constexpr int kMaxRed = 40;
 struct BlockGroup {
   lds_double *red;
   static constexpr int kSize = kPlainThreads;
+  static constexpr bool kWindow = false;
   __device__ __forceinline__ int rank() const { return threadIdx.x; }
   __device__ __forceinline__ void sync() const { __syncthreads(); }
   template <int K>
@@ -190,6 +194,62 @@ struct BlockGroup {
     __syncthreads();
     int r = ri[0];
     for (int k = 1; k < kPlainThreads / kWave; ++k) r = take_min ? min(r, ri[k]) : max(r, ri[k]);
+    __syncthreads();
+    return r;
+  }
+  __device__ __forceinline__ int imin(int v) const { return ired(v, true); }
+  __device__ __forceinline__ int imax(int v) const { return ired(v, false); }
+};
+
+// A workgroup of NT threads with the deformed window in LDS (correlate_wide_kernel).
+// red: LDS scratch of NT / 64 x kTeamRed doubles.
+constexpr int kTeamRed = 32;
+template <int NT>
+struct TeamGroup {
+  lds_double *red;
+  static constexpr int kSize = NT;
+  static constexpr bool kWindow = true;
+  static constexpr int kWaves = NT / kWave;
+  __device__ __forceinline__ int rank() const { return opaque_lane((int)threadIdx.x); }
+  __device__ __forceinline__ void sync() const { __syncthreads(); }
+  template <int K>
+  __device__ __forceinline__ void sum(double (&v)[K]) const {
+    static_assert(K <= kTeamRed, "reduction too wide");
+    const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double s = wave_sum(v[k]);
+      if (l == 0) red[w * kTeamRed + k] = s;
+    }
+    __syncthreads();
+    // lane k of every wave adds total k (all waves the same values), then v_readlane
+    double t = 0.0;
+    if (l < K)
+#pragma unroll
+      for (int q = 0; q < kWaves; ++q) t += red[q * kTeamRed + l];
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = lane_value(t, k);
+    __syncthreads();
+  }
+  template <int K>
+  __device__ __forceinline__ void bcast0(double (&v)[K]) const {
+    static_assert(K <= kTeamRed, "broadcast too wide");
+    if (threadIdx.x == 0)
+#pragma unroll
+      for (int k = 0; k < K; ++k) red[k] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = red[k];
+    __syncthreads();
+  }
+  __device__ __forceinline__ int ired(int v, bool take_min) const {
+    const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
+    int s = take_min ? wave_min(v) : wave_max(v);
+    __attribute__((address_space(3))) int *ri = reinterpret_cast<__attribute__((address_space(3))) int *>(red);
+    if (l == 0) ri[w] = s;
+    __syncthreads();
+    int r = ri[0];
+    for (int k = 1; k < kWaves; ++k) r = take_min ? min(r, ri[k]) : max(r, ri[k]);
     __syncthreads();
     return r;
   }
@@ -575,8 +635,16 @@ constexpr int kOverflow = -1000;
 
 // ------------------------------------------------------ subset solver ---
 template <typename T, typename G, int INTERP, bool DEFGRAD>
+struct Solver;
+template <typename T, int INTERP, int NT>
+__device__ __forceinline__ int team_simplex(Solver<T, TeamGroup<NT>, INTERP, false> &s, Affine &A, int &iters);
+
+template <typename T, typename G, int INTERP, bool DEFGRAD>
 struct Solver {
   static constexpr bool kIsWave = G::kSize == kWave;
+  // a workgroup that stages the deformed window in LDS; a window that does not
+  // fit leaves win_ok false, and the taps come from the image
+  static constexpr bool kTeam = !kIsWave && G::kWindow;
   const KParams kp;
   const DImage ref;
   const DImage def;
@@ -610,6 +678,7 @@ struct Solver {
   // a workgroup's LDS tables for the objective of subsets of at most
   // kLaneSimplexMaxPixels pixels (3 kLaneSimplexMaxPixels floats), or null
   lds_float *small_tab = nullptr;
+  lds_float *nm_tab = nullptr;  // kTeam: team_simplex's vertex table and point (kNmFloats + 8 floats)
   bool forced;  // Nelder-Mead only
   float meanF;
   float en[6];  // 1 for enabled parameters
@@ -834,7 +903,7 @@ struct Solver {
     const float tx = ddx - flx, ty = ddy - fly;
     const int ix = cx - def.ox + (int)flx;
     const int iy = cy - def.oy + (int)fly;
-    if constexpr (kIsWave) {
+    if (kIsWave || (kTeam && win_ok)) {
       // window origin and pitch are scalar; kept pixels index the window with
       // non-negative offsets below 2^24
       if (INTERP == 0) return bilinear_sum(win + (__umul24(iy - wy0, wpitch) + (ix - wx0)), wpitch, tx, ty);
@@ -891,6 +960,10 @@ struct Solver {
     // image coordinates through wx0, wy0, wpitch)
     if (win_ok && x0 >= wx0 && x1 < wx0 + wpitch && y0 >= wy0 && y1 < wy0 + wrows) return true;
     if (ww * hh > win_cap) {
+      if constexpr (kTeam) {
+        win_ok = false;
+        return true;  // the taps come from the image
+      }
       if (hand_over) overflow = true;
       return false;
     }
@@ -920,14 +993,16 @@ struct Solver {
     const auto *P = Pix<T>::ptr(def.pix) + y0 * def.w + x0;
     const float inv = 1.0f / (float)ww_s;
     const int tot = ww_s * hh_s;
-    if constexpr (kIsWave && std::is_same<T, float>::value) {
+    if constexpr ((kIsWave || kTeam) && std::is_same<T, float>::value) {
       // direct global -> LDS loads (global_load_lds_dword): the 64 lanes of one
       // load fill 64 consecutive floats of the slot, so window element k =
       // 64 j + lane comes from batch j.  No VGPRs hold the data and every batch
-      // is in flight before the single wait.
-      const int lane = grp.rank();
+      // is in flight before the single wait.  (A workgroup's waves take the
+      // batches in turn.)
+      const int lane = kIsWave ? grp.rank() : (int)(threadIdx.x % kWave);
+      const int first = kIsWave ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave) * kWave);
 #pragma unroll 4
-      for (int k0 = 0; k0 < tot; k0 += kWave) {
+      for (int k0 = first; k0 < tot; k0 += G::kSize) {
         const int k = k0 + lane;
         if (k < tot) {
           const int r = (int)(((float)k + 0.5f) * inv);
@@ -971,7 +1046,7 @@ struct Solver {
   // Window covering the warped subset bbox (+ interpolation support and a
   // 1-px rounding margin) at parameters A.
   __device__ __forceinline__ bool stage_affine(const Affine &A, bool ring = true) {
-    if constexpr (!kIsWave) {
+    if constexpr (!kIsWave && !kTeam) {
       (void)A;
       (void)ring;
       return true;
@@ -1098,6 +1173,79 @@ struct Solver {
       for (int k = 0; k < 6; ++k) acc[27 + k] += rd[k];
       acc[33] += (double)Gv;
       acc[34] += 1.0;
+    });
+    grp.sum(acc);
+  }
+
+  // correlate_wide_kernel: the sums over the active pixels that every step's H
+  // and sigma follow from, added in FP64: sum(phi phi^T) (a full 6 x 6 at
+  // pers[0, 36)), sum(phi) (pers[36, 42)), sum(gx^2) and sum(gy^2) of the float
+  // squares (pers[kWideSg, +2)), and the mean reference intensity (meanF).
+  static constexpr int kWideSg = 44;
+  __device__ __forceinline__ void precompute_wide() {
+    double acc[31];
+#pragma unroll
+    for (int k = 0; k < 31; ++k) acc[k] = 0.0;
+    for_pixels([&](int x, int y, bool a) {
+      if (!a) return;
+      float F, gx, gy;
+      ref_pixel(x - ref.ox, y - ref.oy, F, gx, gy);
+      const double dx = (double)(x - cx), dy = (double)(y - cy), dgx = gx, dgy = gy;
+      const double ph[6] = {dgx, dgy, dx * dgx, dy * dgx, dx * dgy, dy * dgy};
+      int h = 0;
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+#pragma unroll
+        for (int l = k; l < 6; ++l) { acc[h] = fma(ph[k], ph[l], acc[h]); ++h; }
+#pragma unroll
+      for (int k = 0; k < 6; ++k) acc[21 + k] += ph[k];
+      acc[27] += (double)F;
+      acc[28] += 1.0;
+      acc[29] += (double)(gx * gx);
+      acc[30] += (double)(gy * gy);
+    });
+    grp.sum(acc);
+    meanF = acc[28] > 0.0 ? (float)(acc[27] / acc[28]) : 0.0f;
+    if (grp.rank() == 0) {
+      int h = 0;
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+#pragma unroll
+        for (int l = k; l < 6; ++l) {
+          pers[6 * k + l] = acc[h];
+          pers[6 * l + k] = acc[h];
+          ++h;
+        }
+#pragma unroll
+      for (int k = 0; k < 6; ++k) pers[36 + k] = acc[21 + k];
+      pers[kWideSg] = acc[29];
+      pers[kWideSg + 1] = acc[30];
+    }
+    grp.sync();
+  }
+
+  // One Gauss-Newton pass of correlate_wide_kernel, every active pixel kept:
+  // sum(gmf r) over the residual rows (6) and sum(G), the terms of
+  // accumulate_gn_block, added in FP64.
+  __device__ __forceinline__ void accumulate_gn_wide(const Affine &A, float shift, double (&acc)[7]) {
+#pragma unroll
+    for (int k = 0; k < 7; ++k) acc[k] = 0.0;
+    for_pixels_ref([&](auto inside, int x, int y, bool a) {
+      if (!a) return;
+      // the reference loads first: they are in flight during the interpolation
+      float Fv, gx, gy;
+      ref_pixel<decltype(inside)::value>(x - ref.ox, y - ref.oy, Fv, gx, gy);
+      const float dx = (float)(x - cx), dy = (float)(y - cy);
+      float ox, oy;
+      A.disp(dx, dy, ox, oy);
+      const float Gv = sample(ox, oy);
+      const float Gx = A.c * gx - A.s * gy, Gy = A.s * gx + A.c * gy;
+      float r[6];
+      A.residual(dx, dy, Gx, Gy, r);
+      const double gmf = (double)((Gv - shift) - (Fv - meanF));
+#pragma unroll
+      for (int k = 0; k < 6; ++k) acc[k] = fma(gmf, (double)(r[k] * en[k]), acc[k]);
+      acc[6] += (double)Gv;
     });
     grp.sum(acc);
   }
@@ -1424,7 +1572,7 @@ struct Solver {
       }
     }
     bool every = false;  // BATCHED: every active pixel is kept (no per-pixel guard test)
-    if constexpr (kIsWave) every = all_kept(A);
+    if constexpr (kIsWave || kTeam) every = all_kept(A);
     if (every) {
       gamma_sums_every<false>(A, acc);
     } else {
@@ -2043,19 +2191,28 @@ struct Solver {
   // Rows of M over phi = (gx, gy, dx gx, dy gx, dx gy, dy gy): u (c, -s, 0, 0, 0, 0),
   // v (s, c, 0, 0, 0, 0), theta (0, 0, -g, -ey1, ex1, g), ex (0, 0, 1, 0, 0, 0),
   // ey (0, 0, 0, 0, 0, 1), gxy (0, 0, 0, 1, 1, 0).
-  __device__ __forceinline__ void fast_system(const Affine &A, double corr, double (&H)[6][6], double (&q)[6]) const {
+  // (M t)_r for a vector t over phi
+  __device__ __forceinline__ static double fast_row(const Affine &A, int r, const double (&t)[6]) {
     const double c = A.c, sn = A.s, ex1 = 1.0 + (double)A.p[3], ey1 = 1.0 + (double)A.p[4], g = A.p[5];
-    // (M t)_r for a vector t over phi
-    auto apply = [&](int r, const double (&t)[6]) -> double {
-      switch (r) {
-        case 0: return c * t[0] - sn * t[1];
-        case 1: return sn * t[0] + c * t[1];
-        case 2: return ex1 * t[4] - ey1 * t[3] + g * (t[5] - t[2]);
-        case 3: return t[2];
-        case 4: return t[5];
-        default: return t[3] + t[4];
-      }
-    };
+    switch (r) {
+      case 0: return c * t[0] - sn * t[1];
+      case 1: return sn * t[0] + c * t[1];
+      case 2: return ex1 * t[4] - ey1 * t[3] + g * (t[5] - t[2]);
+      case 3: return t[2];
+      case 4: return t[5];
+      default: return t[3] + t[4];
+    }
+  }
+  template <class V>
+  __device__ __forceinline__ static void fast_rows(const Affine &A, V &&v, double (&out)[6]) {
+    double t[6];
+#pragma unroll
+    for (int l = 0; l < 6; ++l) t[l] = v(l);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) out[i] = fast_row(A, i, t);
+  }
+  __device__ __forceinline__ void fast_matrix(const Affine &A, double (&H)[6][6]) const {
+    auto apply = [&](int r, const double (&t)[6]) { return fast_row(A, r, t); };
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
       double t[6];  // S m_j (S is symmetric: row k of S against row j of M)
@@ -2072,11 +2229,10 @@ struct Solver {
         H[j][i] = H[i][j];
       }
     }
-    double v[6];
-#pragma unroll
-    for (int l = 0; l < 6; ++l) v[l] = pers[kPersistPass + l] - corr * pers[36 + l];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) q[i] = apply(i, v);
+  }
+  __device__ __forceinline__ void fast_system(const Affine &A, double corr, double (&H)[6][6], double (&q)[6]) const {
+    fast_matrix(A, H);
+    fast_rows(A, [&](int l) { return pers[kPersistPass + l] - corr * pers[36 + l]; }, q);
   }
   // Identity rows and columns and a zero gradient for disabled parameters (the
   // same solution as the reference's reduced N x N system), and the LM term.
@@ -2364,7 +2520,30 @@ struct Solver {
       if (!stage_affine(A)) return kOverflow;
       float du[6];
       float meanG;
-      if constexpr (!kIsWave) {
+      if constexpr (kTeam) {
+        // every pixel kept (else the PLAIN kernel takes the subset): H = M S M^T
+        // from the per-subset sums, q from the pass (see fast_system)
+        if (!all_kept(A)) return kOverflow;
+        last_fast = true;
+        double acc[7];
+        accumulate_gn_wide(A, shift, acc);
+        const double cnt = (double)n_def_active;
+        meanG = cnt > 0.0 ? (float)(acc[6] / cnt) : 0.0f;
+        const double corr = (double)meanG - (double)shift;
+        double H[6][6], q[6], sr[6];
+        fast_matrix(A, H);
+        fast_rows(A, [&](int l) { return (double)pers[36 + l]; }, sr);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) q[k] = acc[k] - corr * sr[k];
+        finish_system(H, q);
+        const float cond = cond2x2(H[0][0], H[0][1], H[0][1], H[1][1]);
+        if (grp.rank() == 0) fields[(size_t)F_CONDITION * nsub + gid] = cond;
+        if (cond > 1.0e12f) return HESSIAN_SINGULAR;
+        double dd[6];
+        if (!ldlt_update6(H, q, dd)) return kOverflow;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) du[k] = wave_uniform_f((float)dd[k]);
+      } else if constexpr (!kIsWave) {
         double acc[35];
         accumulate_gn_block(A, shift, acc);
         const double cnt = acc[34];
@@ -2519,7 +2698,7 @@ struct Solver {
   // BATCHED window for the shifted positions did not fit.
   __device__ __forceinline__ bool uncertainty(const Affine &A, double *fields, int nsub, int gid) {
     const float u = A.p[0], v = A.p[1];
-    if constexpr (kIsWave) {
+    if constexpr (kIsWave || kTeam) {
       // window covering the subset bbox shifted by (u, v), Keys support and a
       // 1-px margin for the rounding of x + u
       const int fu = (int)floorf(u), fv = (int)floorf(v);
@@ -2544,7 +2723,8 @@ struct Solver {
       keys_weights(v - (float)fv, wyu);
     }
     bool e_in_win = false;
-    if constexpr (kIsWave)
+    const bool in_win = kIsWave || (kTeam && win_ok);
+    if (in_win)
       e_in_win = wx0 <= bx0 - ref.ox && wx0 + wpitch > bx1 - ref.ox && wy0 <= by0 - ref.oy &&
                  wy0 + wrows > by1 - ref.oy;
     for_pixels([&](int x, int y, bool a) {
@@ -2554,7 +2734,7 @@ struct Solver {
       float refv, gx, gy;
       ref_pixel(rx, ry, refv, gx, gy);
       float sub_r;
-      if constexpr (kIsWave) {
+      if (in_win) {
         if (uniform_w)
           sub_r = keys_sum(win + (__umul24(ry + fv - 2 - wy0, wpitch) + (rx + fu - 2 - wx0)), wpitch, wxu, wyu) - refv;
         else
@@ -2565,7 +2745,7 @@ struct Solver {
       const bool inb = rx >= 0 && ry >= 0 && rx <= def.w - 2 && ry <= def.h - 2;
       float e = 0.0f;
       if (inb) {
-        if constexpr (kIsWave) {
+        if (in_win) {
           // the unshifted pixel from the window when the window holds the subset bbox
           e = e_in_win ? (float)win[__umul24(ry - wy0, wpitch) + (rx - wx0)] : Pix<T>::at(def.pix, ry * def.w + rx);
         } else {
@@ -2867,7 +3047,8 @@ struct Solver {
       // BATCHED: the bbox and its 1-px ring staged in LDS when it fits (the
       // mask taps of the interior pixels then come from the window)
       bool in_lds = false;
-      if constexpr (kIsWave) in_lds = stage(min_x - ox - 1, max_x - ox, min_y - oy - 1, max_y - oy, false);
+      if constexpr (kIsWave || kTeam)
+        in_lds = stage(min_x - ox - 1, max_x - ox, min_y - oy - 1, max_y - oy, false) && (kIsWave || win_ok);
       const bool fdiv = tot < (1 << 20);  // (k + 0.5) / bw in float is exact below this size
       const float inv = 1.0f / (float)bw;
       const auto *P = Pix<T>::ptr(def.pix);
@@ -2908,7 +3089,7 @@ struct Solver {
   // Objective::sigma (DICe_Objective.cpp:150-184) with the subset state of the
   // last warp (parameters p_state) and the final parameters A.
   __device__ __forceinline__ float sigma(const float p_state[6], const Affine &A, float &noise) {
-    if constexpr (kFast) {
+    if constexpr (kFast || kTeam) {
       if (last_fast && (S > 0 || n_def_active > 0)) {
         // the last warp kept every active pixel: the gradient sums are
         // sum(phi phi^T)[0][0] and [1][1], the kept bbox is the bbox of the
@@ -2916,7 +3097,8 @@ struct Solver {
         if (S > 0) noise = noise_std_dev(bx0, bx1, by0, by1, A.p[0], A.p[1]);
         else noise = noise_std_dev(min(cx, abx0), max(cx, abx1), min(cy, aby0), max(cy, aby1), A.p[0], A.p[1]);
         if (noise < 0.0f) return -1.0f;
-        const float sgx = (float)uniform(pers[0]), sgy = (float)uniform(pers[7]);
+        const float sgx = (float)uniform(kTeam ? pers[kWideSg] : pers[0]);
+        const float sgy = (float)uniform(kTeam ? pers[kWideSg + 1] : pers[7]);
         const float sg = sgx > sgy ? sgy : sgx;
         return sg > 0.0f ? (float)sqrt(2.0 * (double)noise * (double)noise / (double)sg) : -1.0f;
       }
@@ -3049,7 +3231,7 @@ struct Solver {
   // nm: per-subset Nelder-Mead results of simplex_groups_kernel for this pass
   // (SIMPLEX_OPT only), or null to run the simplex here.  NM_ONLY: the
   // instantiation holds no simplex (and so needs far fewer registers); a
-  // subset without a result goes to ov_list, and the PLAIN kernel runs its
+  // subset without a result goes to ov_list, and correlate_wide_kernel runs its
   // simplex.
   template <bool SIMPLEX_OPT, bool NM_ONLY = false>
   __device__ __forceinline__ void run(const DSubsets &ss, int gid, double *fields, int pass, int *fb_list,
@@ -3081,6 +3263,8 @@ struct Solver {
     int iters = -1;
     if constexpr (!SIMPLEX_OPT && kFast) {
       precompute_phi();  // and meanF
+    } else if constexpr (!SIMPLEX_OPT && kTeam) {
+      precompute_wide();  // and meanF
     } else if (!SIMPLEX_OPT) {
       // mean of the reference subset over defined-active pixels (DICe_Objective.cpp:464)
       double acc[2] = {0.0, 0.0};
@@ -3122,6 +3306,8 @@ struct Solver {
         corr = __float_as_int(r[7]);
       } else if constexpr (NM_ONLY) {
         corr = kOverflow;
+      } else if constexpr (kTeam) {
+        corr = team_simplex(*this, A, iters);
       } else {
         corr = simplex(A, iters);
       }
@@ -3331,6 +3517,7 @@ struct Items {
 // the lane and samples the images from global memory (no LDS window).
 struct LaneGroup {
   static constexpr int kSize = 1;
+  static constexpr bool kWindow = false;
   __device__ __forceinline__ int rank() const { return 0; }
   __device__ __forceinline__ void sync() const {}
   template <int K>
@@ -3383,6 +3570,10 @@ struct LaneSimplex {
   __device__ __forceinline__ void start(const DSubsets &ss, int gid, const double *fields) {
     s.set_subset(ss, gid);
     s.init_params(A, fields, ss.n, gid);
+    begin();
+  }
+  // ... with the initial point in A.p
+  __device__ __forceinline__ void begin() {
     if (writer) {
 #pragma unroll
       for (int j = 0; j < 6; ++j) nm[49 + j] = A.p[j];
@@ -3552,6 +3743,117 @@ struct LaneSimplex {
   }
 };
 
+// Simplex::minimize for one subset on a workgroup with the window in LDS: all
+// waves evaluate the objective, wave 0 runs LaneSimplex's bookkeeping (once, not
+// in every wave) and publishes the next point.  The reference sums of the
+// objective do not change while every pixel is kept, so they are formed once.
+// On exit A.p holds the last evaluated point, as after Solver::simplex.
+template <typename T, int INTERP, int NT>
+__device__ __forceinline__ int team_simplex(Solver<T, TeamGroup<NT>, INTERP, false> &s, Affine &A, int &iters) {
+  lds_float *const nm = s.nm_tab, *const out = nm + kNmFloats;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  LaneSimplex<T, INTERP, true> m(s.kp, s.ref, s.def, nm, threadIdx.x == 0);
+  if (wave == 0) {
+    m.A = A;
+    m.begin();
+  }
+  const bool small = s.n <= kLaneSimplexMaxPixels;
+  double rsum[2] = {0.0, 0.0};  // sum r, sum r^2 over the active pixels
+  if (!small) {
+    s.for_pixels([&](int x, int y, bool a) {
+      if (!a) return;
+      const double r = s.ref_value(x - s.ref.ox, y - s.ref.oy);
+      rsum[0] += r;
+      rsum[1] = fma(r, r, rsum[1]);
+    });
+    s.grp.sum(rsum);
+  }
+  s.grp.sync();
+  while (true) {
+    A.prepare();
+    float g = 0.0f;
+    int active;
+    float contrast;
+    if (small) {
+      g = s.gamma_eval(A, active, contrast);
+    } else {
+      s.stage_affine(A);
+      double acc[6] = {0, 0, 0, 0, 0, 0};  // n, sd, sdd, sr, srr, sdr
+      lds_double *const red = s.grp.red;
+      const bool every = s.all_kept(A);
+      auto reduce = [&](int k) {
+        const double t = wave_sum(acc[k]);
+        if (lane == 0) red[wave * kTeamRed + k] = t;
+      };
+      if (every) {
+        s.for_pixels_ref([&](auto inside, int x, int y, bool a) {
+          if (!a) return;
+          const double r = s.template ref_value<decltype(inside)::value>(x - s.ref.ox, y - s.ref.oy);
+          float ox, oy;
+          A.disp((float)(x - s.cx), (float)(y - s.cy), ox, oy);
+          const double d = s.sample(ox, oy);
+          acc[1] += d;
+          acc[2] = fma(d, d, acc[2]);
+          acc[5] = fma(d, r, acc[5]);
+        });
+        reduce(1);
+        reduce(2);
+        reduce(5);
+      } else {
+        s.for_pixels([&](int x, int y, bool a) {
+          if (!a) return;
+          const double r = s.ref_value(x - s.ref.ox, y - s.ref.oy);
+          float ox, oy;
+          A.disp((float)(x - s.cx), (float)(y - s.cy), ox, oy);
+          if (!s.kept(ox, oy)) return;
+          const double d = s.sample(ox, oy);
+          acc[0] += 1.0;
+          acc[1] += d;
+          acc[2] = fma(d, d, acc[2]);
+          acc[3] += r;
+          acc[4] = fma(r, r, acc[4]);
+          acc[5] = fma(d, r, acc[5]);
+        });
+#pragma unroll
+        for (int k = 0; k < 6; ++k) reduce(k);
+      }
+      __syncthreads();
+      if (wave == 0) {
+        double t = 0.0;
+        if (lane < 6)
+#pragma unroll
+          for (int q = 0; q < NT / kWave; ++q) t += red[q * kTeamRed + lane];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) acc[k] = lane_value(t, k);
+        if (every) {
+          acc[0] = (double)s.n_def_active;
+          acc[3] = rsum[0];
+          acc[4] = rsum[1];
+        }
+        g = s.gamma_of(acc, active, contrast);
+      }
+    }
+    if (wave == 0) {
+      int it = 0;
+      const int st = m.step(g, it);
+      if (lane == 0) {
+#pragma unroll
+        for (int j = 0; j < 6; ++j) out[j] = m.A.p[j];
+        out[6] = __int_as_float(it);
+        out[7] = __int_as_float(st);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 6; ++j) A.p[j] = wave_uniform_f(out[j]);
+    const int st = __float_as_int(wave_uniform_f(out[7]));
+    if (st >= 0) {
+      iters = __float_as_int(wave_uniform_f(out[6]));
+      return st;
+    }
+  }
+}
+
 // BATCHED Nelder-Mead iterations for small subsets, 64 / W per wave: each row
 // of W lanes (16, or 8 when no subset has more than kNarrowSimplexMaxPixels
 // pixels) owns one subset, runs LaneSimplex's state machine in all of its
@@ -3565,9 +3867,9 @@ struct LaneSimplex {
 // of them hold LaneSimplex's vertex table); a point whose footprint leaves the
 // window restages it.  A point whose window does not fit the slot reads its
 // taps from the image (bilinear) or ends the row's work on the subset with
-// status kNmNoResult (Keys): the epilogue kernel hands such a subset to the
-// PLAIN kernel, which runs its simplex (in the same summation order, so with
-// the same result).  Rows that finish a subset write its result to
+// status kNmNoResult (Keys): the epilogue kernel hands such a subset to
+// correlate_wide_kernel, which runs its simplex (in the same summation order, so
+// with the same result).  Rows that finish a subset write its result to
 // nm_out and take the next items: one atomic per wave and refill, the rows
 // numbered by their rank in the ballot.  A row whose item index is past the
 // end stays idle, and the wave exits when all of its rows are idle: every
@@ -3730,6 +4032,93 @@ __global__ __launch_bounds__(kPlainThreads) void correlate_plain_kernel(KParams 
   for (int k = blockIdx.x; k < total; k += gridDim.x)
     s.template run<SIMPLEX_OPT>(ss, items.at(k), fields, pa.pass, pa.fb_list, pa.fb_count, nullptr, nullptr,
                                 pa.nm_result);
+}
+
+// Work claims of a workgroup over the eight item ranges (see
+// correlate_batched_kernel): the next item, or -1 when every range is
+// exhausted.  Every thread calls it; next: one LDS int.
+struct BlockClaims {
+  int *counter;
+  int total, range, visited;
+  __device__ __forceinline__ BlockClaims(int *c, int n)
+      : counter(c), total(n), range((int)(blockIdx.x % kWorkRanges)), visited(0) {}
+  __device__ __forceinline__ int take(int *next) {
+    while (visited < kWorkRanges) {
+      const int lo = (int)((long long)total * range / kWorkRanges);
+      const int hi = (int)((long long)total * (range + 1) / kWorkRanges);
+      if (threadIdx.x == 0) *next = atomicAdd(counter + range * kCounterStride, 1);
+      __syncthreads();
+      const int k = __builtin_amdgcn_readfirstlane(*next) + lo;
+      __syncthreads();
+      if (k < hi) return k;
+      range = range + 1 == kWorkRanges ? 0 : range + 1;
+      ++visited;
+    }
+    return -1;
+  }
+};
+
+// The subsets whose window outgrew a BATCHED wave's slot (or all of them when
+// the subset side says so in advance, pa.count_all): one workgroup of NT
+// threads per subset, in PLAIN's arithmetic -- FP64 sums -- with the deformed
+// window in LDS (cap floats).  Gauss-Newton takes the subsets whose pixels
+// are all kept, and hands the others to pa.ov_list for the PLAIN kernel.
+// PLAIN is bound by its taps: 36 scattered loads per pixel and pass through
+// the CU's one texture-address unit.  From LDS the kernel is bound by VALU issue
+// (84 % of the quad-cycles at four waves per SIMD), so the sums per pixel count:
+// Gauss-Newton adds q and sum(G) only (7 FP64 adds instead of 35) and takes H
+// from the per-subset S.  2,280 subsets of 75 x 75 (1500 x 1100, six
+// parameters): 1.49 -> 0.44 ms per frame; 8,000 polygons of 200-3000 px, half of
+// them too large for a slot: 1.91 -> 0.84 ms.  NT = 1024 when there is at most
+// one subset per CU (a subset's latency is then what counts): six 61 x 61
+// subsets by Nelder-Mead 0.99 -> 0.78 ms, bookkeeping in one wave only.
+// Registers: four waves per SIMD with some spills beat two without (0.53 against
+// 0.59 ms, and 0.95 against 1.08 ms for the polygons, measured with an earlier
+// reduction).
+#ifndef DICE_WIDE_WPE
+#define DICE_WIDE_WPE 4
+#endif
+template <typename T, int INTERP, bool SIMPLEX_OPT, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT > 512 ? 4 : DICE_WIDE_WPE))) void correlate_wide_kernel(
+    KParams kp, DImage ref, DImage def, DSubsets ss, double *fields, PassArgs pa, int cap) {
+  extern __shared__ float lds[];
+  __shared__ double red[NT / kWave * kTeamRed];
+  __shared__ double pers[48];
+  __shared__ float small_tab[3 * kLaneSimplexMaxPixels];
+  __shared__ float nm_tab[kNmFloats + 8];
+  __shared__ int next;
+  const Items items{pa.items, pa.item_count, ss.order};
+  const int total = items.total(ss.n);
+  if ((int)blockIdx.x >= total) return;
+  using G = TeamGroup<NT>;
+  Solver<T, G, INTERP, false> s(kp, ref, def, G{(lds_double *)red}, (lds_float *)lds, cap);
+  s.pers = (lds_double *)pers;
+  s.small_tab = (lds_float *)small_tab;
+  s.nm_tab = (lds_float *)nm_tab;
+  BlockClaims claims(pa.counter, total);
+#pragma unroll 1
+  for (int k = claims.take(&next); k >= 0; k = claims.take(&next)) {
+    const int gid = items.at(k);
+    if (pa.count_all && threadIdx.x == 0) atomicAdd(pa.count_all, 1);
+    s.template run<SIMPLEX_OPT>(ss, gid, fields, pa.pass, pa.fb_list, pa.fb_count, pa.ov_list, pa.ov_count,
+                                pa.nm_result);
+  }
+}
+
+template <typename T, int INTERP, bool SX>
+hipError_t launch_wide_variant(const Launch &L, const KParams &kp, const DImage &ref, const DImage &def,
+                               const DSubsets &subs, double *fields, const PassArgs &pa, hipStream_t stream) {
+  const size_t shm = (size_t)L.wide_floats * sizeof(float);
+  if (subs.n <= L.num_cus) {
+    // at most one subset per CU: its latency counts, so every SIMD gets four waves of it
+    hipLaunchKernelGGL((correlate_wide_kernel<T, INTERP, SX, 1024>), dim3(subs.n), dim3(1024), shm, stream, kp, ref,
+                       def, subs, fields, pa, L.wide_floats);
+  } else {
+    const int groups = subs.n < 4 * L.num_cus ? subs.n : 4 * L.num_cus;
+    hipLaunchKernelGGL((correlate_wide_kernel<T, INTERP, SX, 256>), dim3(groups), dim3(256), shm, stream, kp, ref, def,
+                       subs, fields, pa, L.wide_floats);
+  }
+  return hipGetLastError();
 }
 
 // BATCHED: persistent waves pull items from work counters until every range
@@ -3904,7 +4293,7 @@ hipError_t launch_variant(const Launch &L, const KParams &kp, const DImage &ref,
   // two waves per SIMD and spills nothing (built for the Gauss-Newton kernel
   // with reference gradients, the large-conformal-subset case)
   // the epilogue of simplex_groups_kernel's results: the variant without a
-  // simplex (the subsets it has no result for go to the PLAIN kernel)
+  // simplex (the subsets it has no result for go to correlate_wide_kernel)
   if constexpr (SX && !DEFGRAD) {
     if (pa.nm_result && pa.ov_list) {
       hipLaunchKernelGGL((correlate_batched_kernel<T, INTERP, DEFGRAD, SX, DICE_BATCHED_WAVES_PER_EU, true>),

@@ -132,6 +132,9 @@ struct Launch {
   int lane_simplex;            // batched: 0, or the most pixels of a subset (<= kLaneSimplexMaxPixels):
                                // Nelder-Mead passes run rows of 8 or 16 lanes per subset first
                                // (simplex_groups_kernel)
+  int wide_floats;             // batched: LDS window of correlate_wide_kernel
+  int wide_only;               // batched: no subset's window can fit a wave's slot
+  int num_cus;
 };
 
 // Subsets of at most this many pixels run the Nelder-Mead iterations of the
@@ -161,6 +164,7 @@ struct PassArgs {
   int *ov_list, *ov_count;
   int *counter;                // BATCHED work counters, kWorkRanges of them kCounterStride ints apart (zeroed before the launch)
   const float *nm_result;      // Nelder-Mead passes: per-subset results of simplex_groups_kernel, or null
+  int *count_all;              // correlate_wide_kernel taking every subset: the overflow count they add to, or null
 };
 
 // Differentiation path (forward gamma / adjoint) of one launch.
@@ -180,15 +184,23 @@ struct GammaArgs {
 constexpr int kWorkRanges = 8;
 constexpr int kCounterStride = 32;  // ints
 constexpr int kWorkCounterInts = kWorkRanges * kCounterStride;
-// Header of the work area: the range counters, then (on the next line) the
-// fallback count and the overflow counts of pass 0 and pass 1.
-constexpr int kWorkHeader = kWorkCounterInts + kCounterStride;
-constexpr int kWorkFbCount = kWorkCounterInts, kWorkOv0Count = kWorkCounterInts + 1,
-              kWorkOv1Count = kWorkCounterInts + 2;
-constexpr int kWorkLaneCount = kWorkCounterInts + 3;  // work counter of simplex_groups_kernel
+// Header of the work area: a set of range counters for each work-stealing
+// launch of a correlation (lean, then batched and wide of pass 0 and of pass
+// 1), so that one fill at the start clears them all, then (on the next line)
+// the fallback count and the overflow counts of pass 0 and pass 1.
+constexpr int kWorkSets = 5;
+constexpr int kWorkSetLean = 0, kWorkSetBatched = 1, kWorkSetWide = 2;  // of pass 0; pass 1: + 2
+constexpr int kWorkCounts = kWorkSets * kWorkCounterInts;
+constexpr int kWorkHeader = kWorkCounts + kCounterStride;
+constexpr int kWorkFbCount = kWorkCounts, kWorkOv0Count = kWorkCounts + 1, kWorkOv1Count = kWorkCounts + 2;
+constexpr int kWorkLaneCount = kWorkCounts + 3;  // work counters of simplex_groups_kernel (pass 0, pass 1)
 // count of the lean pass's hand-over list, which lives in the storage of the pass-1
 // overflow list (pass 1 starts after pass 0 has finished with it)
-constexpr int kWorkLeanCount = kWorkCounterInts + 4;
+constexpr int kWorkLeanCount = kWorkCounts + 5;
+// counts of the subsets correlate_wide_kernel hands to the PLAIN kernel in pass 0 and pass 1; the
+// lists live in the storage of the other pass's overflow list (the hand-over list of the lean
+// pass, which shares pass 1's, has been worked off by then)
+constexpr int kWorkWideCount = kWorkCounts + 6;
 
 // Device ints of the work area of launch_correlate: the header, the fallback
 // and overflow lists (n each), the Nelder-Mead results (kNmStride per subset).

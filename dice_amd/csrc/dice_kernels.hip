@@ -20,6 +20,10 @@ hipError_t launch_gn_lean(int, int, const Launch &, const KParams &, const DImag
                           double *, const PassArgs &, hipStream_t);
 hipError_t launch_simplex_batched(int, int, int, const Launch &, const KParams &, const DImage &, const DImage &,
                                   const DSubsets &, double *, const PassArgs &, hipStream_t);
+hipError_t launch_gn_wide(int, int, const Launch &, const KParams &, const DImage &, const DImage &, const DSubsets &,
+                          double *, const PassArgs &, hipStream_t);
+hipError_t launch_simplex_wide(int, int, const Launch &, const KParams &, const DImage &, const DImage &,
+                               const DSubsets &, double *, const PassArgs &, hipStream_t);
 
 namespace {
 using dev::ldpix;
@@ -659,81 +663,96 @@ hipError_t launch_reset_listed(const int *list, const int *count, const double *
 }
 
 // One optimizer pass over `items` (nullptr: all subsets).  BATCHED mode runs the
-// persistent kernel, then the PLAIN kernel over the subsets it handed over.
-// A Nelder-Mead pass with L.lane_simplex first runs the iterations in rows of 8
-// or 16 lanes per subset (results in nm); the persistent kernel then does the
-// checks and the epilogue of each subset around them, and hands any subset
-// that kernel left with kNmNoResult to the PLAIN kernel, which runs its simplex.
+// persistent kernel, then correlate_wide_kernel over the subsets whose window
+// outgrew a wave's slot, then (Gauss-Newton) the PLAIN kernel over what that one
+// leaves.  A Nelder-Mead pass with L.lane_simplex first runs the iterations in
+// rows of 8 or 16 lanes per subset (results in nm); the persistent kernel then
+// does the checks and the epilogue of each subset around them, and hands any
+// subset that kernel left with kNmNoResult to correlate_wide_kernel, which runs
+// its simplex.  When no subset's window can fit a wave's slot (L.wide_only),
+// correlate_wide_kernel takes every item at once.
+// work: the header, then the fallback list and the overflow lists of pass 0 and
+// pass 1 (n each); the caller has cleared the header.
 static hipError_t launch_pass(bool simplex, int storage, const Launch &L, const KParams &kp, const DImage &ref,
-                              const DImage &def, const DSubsets &subs, double *fields, PassArgs pa, int *ov_list,
-                              int *ov_count, float *nm, hipStream_t stream, int *lean_list = nullptr) {
+                              const DImage &def, const DSubsets &subs, double *fields, PassArgs pa, int *work,
+                              hipStream_t stream) {
   const int defgrad = simplex ? 0 : kp.def_grads;
+  const size_t n = (size_t)subs.n;
   PassLauncher plain = simplex ? launch_simplex_plain : launch_gn_plain;
   pa.nm_result = nullptr;
+  pa.count_all = nullptr;
   if (L.mode == 0) {
     pa.ov_list = pa.ov_count = nullptr;
     return plain(storage, kp.interp, defgrad, L, kp, ref, def, subs, fields, pa, stream);
   }
+  int *const ov0 = work + kWorkHeader + n, *const ov1 = ov0 + n;
+  int *const ov_list = pa.pass == 0 ? ov0 : ov1, *const ov_count = work + kWorkOv0Count + pa.pass;
+  int *const other = pa.pass == 0 ? ov1 : ov0;  // free once the lean hand-overs have been worked off
+  auto set = [&](int which) { return work + (which + 2 * pa.pass) * kWorkCounterInts; };
   PassLauncher batched = simplex ? launch_simplex_batched : launch_gn_batched;
   hipError_t e;
-  // Gauss-Newton pass 0 of square subsets with none of the options the lean
-  // kernel leaves out: the lean kernel takes every subset first and hands the
-  // others (and those that leave its common case) to the general kernel
-  if (!simplex && pa.pass == 0 && subs.S > 0 && !subs.mbox && !kp.def_grads &&
-      kp.momentum == 0.0f && kp.init_gamma_thr == -1.0 && !kp.has_forced && kp.en_rot && kp.en_normal &&
-      kp.en_shear && kp.lm_alpha <= 0.0f && lean_list) {
-    e = launch_zero_ints(pa.counter, kWorkCounterInts, stream);
+  const bool wide_only = L.wide_only && !defgrad;
+  if (!wide_only) {
+    // Gauss-Newton pass 0 of square subsets with none of the options the lean
+    // kernel leaves out: the lean kernel takes every subset first and hands the
+    // others (and those that leave its common case) to the general kernel
+    if (!simplex && pa.pass == 0 && subs.S > 0 && !subs.mbox && !kp.def_grads && kp.momentum == 0.0f &&
+        kp.init_gamma_thr == -1.0 && !kp.has_forced && kp.en_rot && kp.en_normal && kp.en_shear &&
+        kp.lm_alpha <= 0.0f) {
+      PassArgs pl = pa;
+      pl.counter = work + kWorkSetLean * kWorkCounterInts;
+      pl.ov_list = other;
+      pl.ov_count = work + kWorkLeanCount;
+      e = launch_gn_lean(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
+      if (e != hipSuccess) return e;
+      pa.items = pl.ov_list;
+      pa.item_count = pl.ov_count;
+    }
+    if (simplex && L.lane_simplex) {
+      float *nm = reinterpret_cast<float *>(work + kWorkHeader + 3 * n);
+      e = launch_simplex_lanes(storage, kp.interp, L.lane_simplex, kp, ref, def, subs, fields, pa, nm,
+                               work + kWorkLaneCount + pa.pass, stream);
+      if (e != hipSuccess) return e;
+      pa.nm_result = nm;
+    }
+    pa.counter = set(kWorkSetBatched);
+    pa.ov_list = ov_list;
+    pa.ov_count = ov_count;
+    e = batched(storage, kp.interp, defgrad, L, kp, ref, def, subs, fields, pa, stream);
     if (e != hipSuccess) return e;
-    PassArgs pl = pa;
-    pl.ov_list = lean_list;
-    pl.ov_count = pa.counter + kWorkLeanCount;
-    e = launch_gn_lean(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
-    if (e != hipSuccess) return e;
-    pa.items = lean_list;
-    pa.item_count = pa.counter + kWorkLeanCount;
+    pa.items = ov_list;
+    pa.item_count = ov_count;
   }
-  if (simplex && L.lane_simplex) {
-    int *lane_counter = pa.counter + kWorkLaneCount;
-    e = launch_zero_ints(lane_counter, 1, stream);
-    if (e != hipSuccess) return e;
-    e = launch_simplex_lanes(storage, kp.interp, L.lane_simplex, kp, ref, def, subs, fields, pa, nm, lane_counter,
-                             stream);
-    if (e != hipSuccess) return e;
-    pa.nm_result = nm;
+  if (!defgrad) {
+    pa.counter = set(kWorkSetWide);
+    pa.ov_list = other;
+    pa.ov_count = work + kWorkWideCount + pa.pass;
+    pa.count_all = wide_only ? ov_count : nullptr;
+    e = (simplex ? launch_simplex_wide : launch_gn_wide)(storage, kp.interp, L, kp, ref, def, subs, fields, pa,
+                                                         stream);
+    if (e != hipSuccess || simplex) return e;
+    pa.items = pa.ov_list;
+    pa.item_count = pa.ov_count;
   }
-  e = launch_zero_ints(pa.counter, kWorkCounterInts, stream);
-  if (e != hipSuccess) return e;
-  pa.ov_list = ov_list;
-  pa.ov_count = ov_count;
-  e = batched(storage, kp.interp, defgrad, L, kp, ref, def, subs, fields, pa, stream);
-  if (e != hipSuccess) return e;
-  PassArgs po = pa;
-  po.items = ov_list;
-  po.item_count = ov_count;
-  po.ov_list = po.ov_count = nullptr;
-  return plain(storage, kp.interp, defgrad, L, kp, ref, def, subs, fields, po, stream);
+  pa.ov_list = pa.ov_count = pa.count_all = nullptr;
+  return plain(storage, kp.interp, defgrad, L, kp, ref, def, subs, fields, pa, stream);
 }
 
 hipError_t launch_correlate(const Launch &L, int storage, const KParams &kp, const DImage &ref, const DImage &def,
                             const DSubsets &subs, double *fields, int *work, hipStream_t stream, const int *items,
                             const int *item_count) {
   if (subs.n <= 0) return hipSuccess;
-  // work: the header (range counters, fallback and overflow counts), then the
-  // fallback list and the overflow lists of pass 0 and pass 1 (n each)
-  const size_t n = (size_t)subs.n;
-  int *fb_list = work + kWorkHeader, *ov0 = fb_list + n, *ov1 = fb_list + 2 * n;
-  float *nm = reinterpret_cast<float *>(fb_list + 3 * n);
+  int *fb_list = work + kWorkHeader;
   hipError_t e = launch_zero_ints(work, kWorkHeader, stream);
   if (e != hipSuccess) return e;
   const bool simplex_first = kp.opt == 0 || kp.opt == 3;
-  PassArgs pa{0, items, items ? item_count : nullptr, fb_list, work + kWorkFbCount, nullptr, nullptr, work, nullptr};
-  e = launch_pass(simplex_first, storage, L, kp, ref, def, subs, fields, pa, ov0, work + kWorkOv0Count, nm, stream,
-                  ov1);
+  PassArgs pa{0, items, items ? item_count : nullptr, fb_list, work + kWorkFbCount, nullptr, nullptr, work, nullptr,
+              nullptr};
+  e = launch_pass(simplex_first, storage, L, kp, ref, def, subs, fields, pa, work, stream);
   // the second pass: the fallback optimizer, or Nelder-Mead for the forced subsets of a Gauss-Newton pass
   if (e != hipSuccess || !(kp.opt == 3 || kp.opt == 4 || (kp.has_forced && !simplex_first))) return e;
-  PassArgs pb{1, fb_list, work + kWorkFbCount, nullptr, nullptr, nullptr, nullptr, work, nullptr};
-  return launch_pass(!simplex_first, storage, L, kp, ref, def, subs, fields, pb, ov1, work + kWorkOv1Count, nm,
-                     stream);
+  PassArgs pb{1, fb_list, work + kWorkFbCount, nullptr, nullptr, nullptr, nullptr, work, nullptr, nullptr};
+  return launch_pass(!simplex_first, storage, L, kp, ref, def, subs, fields, pb, work, stream);
 }
 
 hipError_t launch_gradients(int storage, const void *pix, int w, int h, float *gx, float *gy, int smooth,

@@ -256,7 +256,7 @@ int dice_hip_neighbor_rounds(dice_hip_context *ctx);
  * stream): counts[0] subsets handed to the fallback optimizer pass
  * (GRADIENT_BASED_THEN_SIMPLEX / SIMPLEX_THEN_GRADIENT_BASED), counts[1] and
  * counts[2] subsets whose deformed window outgrew the BATCHED wave's LDS slot in
- * the primary and the fallback pass and were solved by the PLAIN kernel.  No
+ * the primary and the fallback pass and were solved by a workgroup each.  No
  * counterpart in the reference: a diagnostic of this library's launches. */
 int dice_hip_pass_counts(dice_hip_context *ctx, int *counts);
 
