@@ -43,6 +43,8 @@ namespace dev {
 // and global_load (HBM) with immediate offsets instead of flat accesses.
 typedef __attribute__((address_space(3))) float lds_float;
 typedef __attribute__((address_space(3))) double lds_double;
+typedef float float4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) float4v lds_float4;
 typedef __attribute__((address_space(1))) const float gfloat;
 typedef __attribute__((address_space(1))) const uint16_t gu16;
 typedef __attribute__((address_space(1))) const int gint;
@@ -131,6 +133,8 @@ struct WaveGroup {
   int lane;
   static constexpr int kSize = kWave;
   static constexpr bool kWindow = true;
+  static constexpr bool kHandOver = true;
+  static constexpr bool kTight = false;
   __device__ __forceinline__ int rank() const { return opaque_lane(lane); }
   __device__ __forceinline__ void sync() const {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -152,12 +156,20 @@ struct WaveGroup {
   __device__ __forceinline__ int imax(int v) const { return wave_max(v); }
 };
 
+// One wavefront whose slot holds fewer floats (win_phys) than the window that
+// still counts as fitting (win_cap): only the ring around the window suffers.
+struct TightWave : WaveGroup {
+  static constexpr bool kTight = true;
+};
+
 // A 256-thread workgroup.  red: LDS scratch of 4 * kMaxRed doubles.
 constexpr int kMaxRed = 40;
 struct BlockGroup {
   lds_double *red;
   static constexpr int kSize = kPlainThreads;
   static constexpr bool kWindow = false;
+  static constexpr bool kHandOver = false;
+  static constexpr bool kTight = false;
   __device__ __forceinline__ int rank() const { return threadIdx.x; }
   __device__ __forceinline__ void sync() const { __syncthreads(); }
   template <int K>
@@ -203,12 +215,14 @@ struct BlockGroup {
 
 // A workgroup of NT threads with the deformed window in LDS (correlate_wide_kernel).
 // red: LDS scratch of NT / 64 x kTeamRed doubles.
-constexpr int kTeamRed = 32;
+constexpr int kTeamRed = 36;
 template <int NT>
 struct TeamGroup {
   lds_double *red;
   static constexpr int kSize = NT;
   static constexpr bool kWindow = true;
+  static constexpr bool kHandOver = false;  // a window that does not fit: taps from the image
+  static constexpr bool kTight = false;
   static constexpr int kWaves = NT / kWave;
   __device__ __forceinline__ int rank() const { return opaque_lane((int)threadIdx.x); }
   __device__ __forceinline__ void sync() const { __syncthreads(); }
@@ -229,6 +243,25 @@ struct TeamGroup {
       for (int q = 0; q < kWaves; ++q) t += red[q * kTeamRed + l];
 #pragma unroll
     for (int k = 0; k < K; ++k) v[k] = lane_value(t, k);
+    __syncthreads();
+  }
+  // The sums in LDS instead (to, K doubles), for every thread after the call.
+  template <int K>
+  __device__ __forceinline__ void sum_to(const double (&v)[K], lds_double *to) const {
+    static_assert(K <= kTeamRed, "reduction too wide");
+    const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double s = wave_sum(v[k]);
+      if (l == 0) red[w * kTeamRed + k] = s;
+    }
+    __syncthreads();
+    if (w == 0 && l < K) {
+      double t = 0.0;
+#pragma unroll
+      for (int q = 0; q < kWaves; ++q) t += red[q * kTeamRed + l];
+      to[l] = t;
+    }
     __syncthreads();
   }
   template <int K>
@@ -255,6 +288,11 @@ struct TeamGroup {
   }
   __device__ __forceinline__ int imin(int v) const { return ired(v, true); }
   __device__ __forceinline__ int imax(int v) const { return ired(v, false); }
+};
+
+// The waves of a workgroup on one subset in a wave's arithmetic (correlate_crew_kernel).
+struct CrewGroup : TeamGroup<256> {
+  static constexpr bool kHandOver = true;  // a window that does not fit a wave's slot: as in a wave
 };
 
 // float element i (i < 2^30) of a global array through a 32-bit byte offset
@@ -630,6 +668,10 @@ __device__ __forceinline__ float cond2x2(double h00, double h01, double h10, dou
   return c;
 }
 
+#ifndef DICE_CREW_ADD
+#define DICE_CREW_ADD(gmf, gv, g1, p) ((p) + (g1))
+#endif
+
 // Status of a wave that handed its subset over (never stored in a field).
 constexpr int kOverflow = -1000;
 
@@ -645,6 +687,12 @@ struct Solver {
   // a workgroup that stages the deformed window in LDS; a window that does not
   // fit leaves win_ok false, and the taps come from the image
   static constexpr bool kTeam = !kIsWave && G::kWindow;
+  // the waves of the group, this wave's number and the lane in it
+  static constexpr int kNW = G::kSize >= kWave ? G::kSize / kWave : 1;
+  __device__ __forceinline__ static int wid() {
+    return kNW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  }
+  __device__ __forceinline__ static int lid() { return opaque_lane((int)(threadIdx.x % kWave)); }
   const KParams kp;
   const DImage ref;
   const DImage def;
@@ -682,6 +730,12 @@ struct Solver {
   bool forced;  // Nelder-Mead only
   float meanF;
   float en[6];  // 1 for enabled parameters
+  // Tables of correlate_trans_kernel / correlate_crew_kernel (LDS, square
+  // subsets, row-major): the interpolated values (n floats), per row of the
+  // subset its six y weights and its window row (8 floats each), and (crew) the
+  // reference values and gradients F, gx, gy (n floats each).
+  lds_float *gtab = nullptr, *ytab = nullptr, *rtab = nullptr;
+  int win_phys = 0;  // G::kTight
 
   __device__ __forceinline__ Solver(const KParams &k, const DImage &r, const DImage &d, G g, lds_float *w, int cap)
       : kp(k), ref(r), def(d), grp(g), win(w), win_cap(kFast ? cap - kPersistFloats : cap), wx0(0), wy0(0),
@@ -774,10 +828,13 @@ struct Solver {
   // a translation); the last S mod 32 columns R at a time, 64 / R rows per
   // step.  Each lane keeps one column per strip and steps down its rows:
   // f(x, y, dx, dy, o) with (dx, dy) = (x - cx, y - cy) and o the reference
-  // pixel offset (y - ref.oy) * ref.w + x - ref.ox.
-  template <class F>
+  // pixel offset (y - ref.oy) * ref.w + x - ref.ox.  The waves of a workgroup
+  // share the rows; SHARE false: every wave walks the whole subset.
+  template <bool SHARE = true, class F>
   __device__ __forceinline__ void for_strips(F &&f) const {
-    const int lane = grp.rank();
+    const int lane = lid();
+    constexpr int nw = SHARE ? kNW : 1;
+    const int w = SHARE ? wid() : 0;
     const int x0 = cx - hw, y0 = cy - hw;
     const int nfull = S >> 5;
     auto column = [&](int x, int r0, int step) {
@@ -793,13 +850,13 @@ struct Solver {
       }
     };
 #pragma unroll 1
-    for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), lane >> 5, 2);
+    for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), (lane >> 5) + 2 * w, 2 * nw);
     const int R = S & 31;
     if (R) {
       const int rows = kWave / R;
       // lane / R in float: exact for lane < 64 and R < 32
       const int lr = (int)(((float)lane + 0.5f) / (float)R), lc = lane - lr * R;
-      if (lr < rows) column(x0 + (nfull << 5) + lc, lr, rows);
+      if (lr < rows) column(x0 + (nfull << 5) + lc, lr + rows * w, rows * nw);
     }
   }
   // reference intensity and gradients at pixel offset o of the reference image
@@ -897,13 +954,15 @@ struct Solver {
   // Deformed intensity at x' = cx + ddx, y' = cy + ddy (interior interpolant of
   // interpolate_keys_fourth_all / interpolate_bilinear_all, DICe_Image.cpp:392-425,
   // 832-883).  Only called for kept pixels, so all taps lie inside the image
-  // and, in BATCHED mode, inside the staged window.
+  // and, in BATCHED mode, inside the staged window.  IN_WINDOW: the caller has
+  // tested win_ok (kTeam).
+  template <bool IN_WINDOW = false>
   __device__ __forceinline__ float sample(float ddx, float ddy) const {
     const float flx = floorf(ddx), fly = floorf(ddy);
     const float tx = ddx - flx, ty = ddy - fly;
     const int ix = cx - def.ox + (int)flx;
     const int iy = cy - def.oy + (int)fly;
-    if (kIsWave || (kTeam && win_ok)) {
+    if (kIsWave || (kTeam && (G::kHandOver || IN_WINDOW || win_ok))) {
       // window origin and pitch are scalar; kept pixels index the window with
       // non-negative offsets below 2^24
       if (INTERP == 0) return bilinear_sum(win + (__umul24(iy - wy0, wpitch) + (ix - wx0)), wpitch, tx, ty);
@@ -959,10 +1018,13 @@ struct Solver {
     // staged that contains this one serves it (the taps are read at their
     // image coordinates through wx0, wy0, wpitch)
     if (win_ok && x0 >= wx0 && x1 < wx0 + wpitch && y0 >= wy0 && y1 < wy0 + wrows) return true;
-    if (ww * hh > win_cap) {
+    const int room = G::kTight ? min(win_phys, win_cap) : win_cap;
+    if (ww * hh > room) {
       if constexpr (kTeam) {
-        win_ok = false;
-        return true;  // the taps come from the image
+        if constexpr (!G::kHandOver) {
+          win_ok = false;
+          return true;  // the taps come from the image
+        }
       }
       if (hand_over) overflow = true;
       return false;
@@ -972,14 +1034,14 @@ struct Solver {
     // by a fraction of a pixel, are usually inside this one
     {
       int e = ring ? 2 : 0;
-      while (e > 0 && (ww + 2 * e) * (hh + 2 * e) > win_cap) --e;
+      while (e > 0 && (ww + 2 * e) * (hh + 2 * e) > room) --e;
       x0 = max(x0 - e, 0);
       y0 = max(y0 - e, 0);
       x1 = min(x1 + e, def.w - 1);
       y1 = min(y1 + e, def.h - 1);
       // an odd pitch where there is room: the 32 words of a column that a
       // half-wave reads at 32 consecutive rows then fall in 32 different banks
-      if (((x1 - x0 + 1) & 1) == 0 && (x1 - x0 + 2) * (y1 - y0 + 1) <= win_cap) {
+      if (((x1 - x0 + 1) & 1) == 0 && (x1 - x0 + 2) * (y1 - y0 + 1) <= room) {
         if (x1 + 1 < def.w) ++x1;
         else if (x0 > 0) --x0;
       }
@@ -1029,6 +1091,14 @@ struct Solver {
   // parameters A: the map is affine, so they are taken at the bbox corners.
   __device__ __forceinline__ void warp_bounds(const Affine &A, float &lo_x, float &hi_x, float &lo_y,
                                               float &hi_y) const {
+    if constexpr (G::kTight) {
+      // a translation (correlate_trans_kernel): disp is p + (dx, dy)
+      lo_x = A.p[0] + ((float)bx0 - (float)cx);
+      hi_x = A.p[0] + ((float)bx1 - (float)cx);
+      lo_y = A.p[1] + ((float)by0 - (float)cy);
+      hi_y = A.p[1] + ((float)by1 - (float)cy);
+      return;
+    }
     lo_x = 1e30f, hi_x = -1e30f, lo_y = 1e30f, hi_y = -1e30f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1147,15 +1217,7 @@ struct Solver {
   __device__ __forceinline__ void accumulate_gn_block(const Affine &A, float shift, double (&acc)[35]) {
 #pragma unroll
     for (int k = 0; k < 35; ++k) acc[k] = 0.0;
-    for_pixels([&](int x, int y, bool a) {
-      if (!a) return;
-      const float dx = (float)(x - cx), dy = (float)(y - cy);
-      float ox, oy;
-      A.disp(dx, dy, ox, oy);
-      if (!kept(ox, oy)) return;
-      const float Gv = sample(ox, oy);
-      float Fv, Gx, Gy;
-      gn_ref(A, x - ref.ox, y - ref.oy, ox, oy, Fv, Gx, Gy);
+    auto add = [&](float dx, float dy, float Gv, float Fv, float Gx, float Gy) {
       float r[6];
       A.residual(dx, dy, Gx, Gy, r);
       double rd[6];
@@ -1173,81 +1235,68 @@ struct Solver {
       for (int k = 0; k < 6; ++k) acc[27 + k] += rd[k];
       acc[33] += (double)Gv;
       acc[34] += 1.0;
-    });
-    grp.sum(acc);
+    };
+    bool done = false;
+    if constexpr (kTeam && !DEFGRAD) {
+      if (last_fast && win_ok && ref_in && (S > 0 ? cx - hw >= 0 && cy - hw >= 0 : pk != nullptr)) {
+        // every active pixel is kept, its taps are in the window and its
+        // reference pixel in the image: one loop without those tests
+        auto inner = [&](float dx, float dy, int o) {
+          float Fv, gx, gy;
+          ref_at(o, Fv, gx, gy);
+          float ox, oy;
+          A.disp(dx, dy, ox, oy);
+          const float Gv = sample<true>(ox, oy);
+          add(dx, dy, Gv, Fv, A.c * gx - A.s * gy, A.s * gx + A.c * gy);
+        };
+        if (S > 0) {
+          for_strips([&](int, int, float dx, float dy, int o) { inner(dx, dy, o); });
+        } else {
+          for_pixels([&](int x, int y, bool a) {
+            if (a) inner((float)(x - cx), (float)(y - cy), (y - ref.oy) * ref.w + x - ref.ox);
+          });
+        }
+        done = true;
+      }
+    }
+    if (!done)
+      for_pixels([&](int x, int y, bool a) {
+        if (!a) return;
+        const float dx = (float)(x - cx), dy = (float)(y - cy);
+        float ox, oy;
+        A.disp(dx, dy, ox, oy);
+        if (!kept(ox, oy)) return;
+        const float Gv = sample(ox, oy);
+        float Fv, Gx, Gy;
+        gn_ref(A, x - ref.ox, y - ref.oy, ox, oy, Fv, Gx, Gy);
+        add(dx, dy, Gv, Fv, Gx, Gy);
+      });
+    if constexpr (kTeam) grp.sum_to(acc, pers + kWideTot);
+    else grp.sum(acc);
   }
+  static constexpr int kWideTot = 2;  // kTeam: the 35 totals in pers (fewer registers than a copy per thread)
 
-  // correlate_wide_kernel: the sums over the active pixels that every step's H
-  // and sigma follow from, added in FP64: sum(phi phi^T) (a full 6 x 6 at
-  // pers[0, 36)), sum(phi) (pers[36, 42)), sum(gx^2) and sum(gy^2) of the float
-  // squares (pers[kWideSg, +2)), and the mean reference intensity (meanF).
-  static constexpr int kWideSg = 44;
+  // correlate_wide_kernel: the mean reference intensity over the active pixels
+  // (meanF) and the sums of sigma() when every one is kept, sum(gx^2) and
+  // sum(gy^2) of the float squares (pers[0, 2)).
   __device__ __forceinline__ void precompute_wide() {
-    double acc[31];
-#pragma unroll
-    for (int k = 0; k < 31; ++k) acc[k] = 0.0;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for_pixels([&](int x, int y, bool a) {
       if (!a) return;
       float F, gx, gy;
       ref_pixel(x - ref.ox, y - ref.oy, F, gx, gy);
-      const double dx = (double)(x - cx), dy = (double)(y - cy), dgx = gx, dgy = gy;
-      const double ph[6] = {dgx, dgy, dx * dgx, dy * dgx, dx * dgy, dy * dgy};
-      int h = 0;
-#pragma unroll
-      for (int k = 0; k < 6; ++k)
-#pragma unroll
-        for (int l = k; l < 6; ++l) { acc[h] = fma(ph[k], ph[l], acc[h]); ++h; }
-#pragma unroll
-      for (int k = 0; k < 6; ++k) acc[21 + k] += ph[k];
-      acc[27] += (double)F;
-      acc[28] += 1.0;
-      acc[29] += (double)(gx * gx);
-      acc[30] += (double)(gy * gy);
+      acc[0] += (double)F;
+      acc[1] += 1.0;
+      acc[2] += (double)(gx * gx);
+      acc[3] += (double)(gy * gy);
     });
     grp.sum(acc);
-    meanF = acc[28] > 0.0 ? (float)(acc[27] / acc[28]) : 0.0f;
+    meanF = acc[1] > 0.0 ? (float)(acc[0] / acc[1]) : 0.0f;
     if (grp.rank() == 0) {
-      int h = 0;
-#pragma unroll
-      for (int k = 0; k < 6; ++k)
-#pragma unroll
-        for (int l = k; l < 6; ++l) {
-          pers[6 * k + l] = acc[h];
-          pers[6 * l + k] = acc[h];
-          ++h;
-        }
-#pragma unroll
-      for (int k = 0; k < 6; ++k) pers[36 + k] = acc[21 + k];
-      pers[kWideSg] = acc[29];
-      pers[kWideSg + 1] = acc[30];
+      pers[0] = acc[2];
+      pers[1] = acc[3];
     }
     grp.sync();
-  }
-
-  // One Gauss-Newton pass of correlate_wide_kernel, every active pixel kept:
-  // sum(gmf r) over the residual rows (6) and sum(G), the terms of
-  // accumulate_gn_block, added in FP64.
-  __device__ __forceinline__ void accumulate_gn_wide(const Affine &A, float shift, double (&acc)[7]) {
-#pragma unroll
-    for (int k = 0; k < 7; ++k) acc[k] = 0.0;
-    for_pixels_ref([&](auto inside, int x, int y, bool a) {
-      if (!a) return;
-      // the reference loads first: they are in flight during the interpolation
-      float Fv, gx, gy;
-      ref_pixel<decltype(inside)::value>(x - ref.ox, y - ref.oy, Fv, gx, gy);
-      const float dx = (float)(x - cx), dy = (float)(y - cy);
-      float ox, oy;
-      A.disp(dx, dy, ox, oy);
-      const float Gv = sample(ox, oy);
-      const float Gx = A.c * gx - A.s * gy, Gy = A.s * gx + A.c * gy;
-      float r[6];
-      A.residual(dx, dy, Gx, Gy, r);
-      const double gmf = (double)((Gv - shift) - (Fv - meanF));
-#pragma unroll
-      for (int k = 0; k < 6; ++k) acc[k] = fma(gmf, (double)(r[k] * en[k]), acc[k]);
-      acc[6] += (double)Gv;
-    });
-    grp.sum(acc);
   }
 
   // BATCHED: FP32 products and per-lane partial sums, FP64 totals in LDS.
@@ -1600,11 +1649,11 @@ struct Solver {
   // (acc[0], the count, is left to the caller: the defined-active count).
   template <bool LEAN>
   __device__ __forceinline__ void gamma_sums_every(const Affine &A, double (&acc)[6]) {
-    auto body = [&](float dx, float dy, float rv) {
+    auto body = [&](float dx, float dy, float rv, auto in_window) {
       const double r = rv;
       float ox, oy;
       A.disp(dx, dy, ox, oy);
-      const double d = sample(ox, oy);
+      const double d = sample<decltype(in_window)::value>(ox, oy);
       acc[1] += d;
       acc[2] += d * d;
       acc[3] += r;
@@ -1612,12 +1661,19 @@ struct Solver {
       acc[5] += d * r;
     };
     if constexpr (LEAN) {
-      for_strips([&](int, int, float dx, float dy, int o) { body(dx, dy, Pix<T>::at_u(ref.pix, (unsigned)o)); });
+      for_strips([&](int, int, float dx, float dy, int o) {
+        body(dx, dy, Pix<T>::at_u(ref.pix, (unsigned)o), std::false_type{});
+      });
+    } else if (kTeam && win_ok && S > 0 && ref_in && cx - hw >= 0 && cy - hw >= 0) {
+      for_strips([&](int, int, float dx, float dy, int o) {
+        body(dx, dy, Pix<T>::at_u(ref.pix, (unsigned)o), std::true_type{});
+      });
     } else {
       for_pixels_ref([&](auto inside, int x, int y, bool a) {
         if (!a) return;
         // the reference load first: it is in flight during the interpolation
-        body((float)(x - cx), (float)(y - cy), ref_value<decltype(inside)::value>(x - ref.ox, y - ref.oy));
+        body((float)(x - cx), (float)(y - cy), ref_value<decltype(inside)::value>(x - ref.ox, y - ref.oy),
+             std::false_type{});
       });
     }
   }
@@ -2191,28 +2247,19 @@ struct Solver {
   // Rows of M over phi = (gx, gy, dx gx, dy gx, dx gy, dy gy): u (c, -s, 0, 0, 0, 0),
   // v (s, c, 0, 0, 0, 0), theta (0, 0, -g, -ey1, ex1, g), ex (0, 0, 1, 0, 0, 0),
   // ey (0, 0, 0, 0, 0, 1), gxy (0, 0, 0, 1, 1, 0).
-  // (M t)_r for a vector t over phi
-  __device__ __forceinline__ static double fast_row(const Affine &A, int r, const double (&t)[6]) {
+  __device__ __forceinline__ void fast_system(const Affine &A, double corr, double (&H)[6][6], double (&q)[6]) const {
     const double c = A.c, sn = A.s, ex1 = 1.0 + (double)A.p[3], ey1 = 1.0 + (double)A.p[4], g = A.p[5];
-    switch (r) {
-      case 0: return c * t[0] - sn * t[1];
-      case 1: return sn * t[0] + c * t[1];
-      case 2: return ex1 * t[4] - ey1 * t[3] + g * (t[5] - t[2]);
-      case 3: return t[2];
-      case 4: return t[5];
-      default: return t[3] + t[4];
-    }
-  }
-  template <class V>
-  __device__ __forceinline__ static void fast_rows(const Affine &A, V &&v, double (&out)[6]) {
-    double t[6];
-#pragma unroll
-    for (int l = 0; l < 6; ++l) t[l] = v(l);
-#pragma unroll
-    for (int i = 0; i < 6; ++i) out[i] = fast_row(A, i, t);
-  }
-  __device__ __forceinline__ void fast_matrix(const Affine &A, double (&H)[6][6]) const {
-    auto apply = [&](int r, const double (&t)[6]) { return fast_row(A, r, t); };
+    // (M t)_r for a vector t over phi
+    auto apply = [&](int r, const double (&t)[6]) -> double {
+      switch (r) {
+        case 0: return c * t[0] - sn * t[1];
+        case 1: return sn * t[0] + c * t[1];
+        case 2: return ex1 * t[4] - ey1 * t[3] + g * (t[5] - t[2]);
+        case 3: return t[2];
+        case 4: return t[5];
+        default: return t[3] + t[4];
+      }
+    };
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
       double t[6];  // S m_j (S is symmetric: row k of S against row j of M)
@@ -2229,10 +2276,11 @@ struct Solver {
         H[j][i] = H[i][j];
       }
     }
-  }
-  __device__ __forceinline__ void fast_system(const Affine &A, double corr, double (&H)[6][6], double (&q)[6]) const {
-    fast_matrix(A, H);
-    fast_rows(A, [&](int l) { return pers[kPersistPass + l] - corr * pers[36 + l]; }, q);
+    double v[6];
+#pragma unroll
+    for (int l = 0; l < 6; ++l) v[l] = pers[kPersistPass + l] - corr * pers[36 + l];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) q[i] = apply(i, v);
   }
   // Identity rows and columns and a zero gradient for disabled parameters (the
   // same solution as the reference's reduced N x N system), and the LM term.
@@ -2329,7 +2377,8 @@ struct Solver {
     // these fixed weights: each lane keeps the row sums of its column for the
     // six window rows under its current pixel and, stepping down two rows, adds
     // the sums of two new rows (the same products and order as keys_sum)
-    const int lane = grp.rank();
+    const int lane = lid(), w = wid();
+    const int ra = S * w / kNW, rb = S * (w + 1) / kNW;  // this wave's rows
     const int x0 = cx - hw, y0 = cy - hw;
     auto rowsum = [&](const auto *p) {
       float rs = p[0] * wxu[0];
@@ -2342,7 +2391,9 @@ struct Solver {
       ref_at(o, refv, gx, gy);
       unc_terms(u, v, gx, gy, interp - refv, *e - refv, pt);
     };
-    auto column = [&](int x, int r0, int step) {
+    auto column = [&](int x, int r0) {
+      if (kNW > 1 && r0 >= rb) return;
+      constexpr int step = 2;
       const int rx = x - ref.ox, ry0 = y0 + r0 - ref.oy;
       int o = ry0 * ref.w + rx;
       const int ostep = step * ref.w;
@@ -2358,9 +2409,9 @@ struct Solver {
         // loads without a branch and they overlap the arithmetic
         const lds_float *tlast = win + (__umul24(wrows - 1, wpitch) + (rx + fu - 2 - wx0));
         float F0 = 0.0f, gx0 = 0.0f, gy0 = 0.0f;
-        if (r0 < S) ref_at(o, F0, gx0, gy0);
+        if (r0 < rb) ref_at(o, F0, gx0, gy0);
 #pragma unroll 1
-        for (int r = r0; r < S; r += 2) {
+        for (int r = r0; r < rb; r += 2) {
           const lds_float *t4 = t + 6 * wpitch, *t5 = t + 7 * wpitch;
           t4 = t4 > tlast ? tlast : t4;
           t5 = t5 > tlast ? tlast : t5;
@@ -2371,7 +2422,7 @@ struct Solver {
             b[k] = t5[k];
           }
           float F1 = 0.0f, gx1 = 0.0f, gy1 = 0.0f;
-          if (r + 2 < S) ref_at(o + ostep, F1, gx1, gy1);
+          if (r + 2 < rb) ref_at(o + ostep, F1, gx1, gy1);
           float vv = h0 * wyu[0];
           vv = fmaf(h1, wyu[1], vv);
           vv = fmaf(h2, wyu[2], vv);
@@ -2396,14 +2447,16 @@ struct Solver {
     };
     const int nfull = S >> 5;
 #pragma unroll 1
-    for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), lane >> 5, 2);
+    for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), ra + (lane >> 5));
     const int R = S & 31;
     if (R) {
       // the last columns R at a time, 64 / R rows per step (row-major, so that
       // the reference loads of a half-wave stay in few cache lines)
-      const int rows = kWave / R;
-      const int lr = (int)(((float)lane + 0.5f) / (float)R), lc = lane - lr * R;
-      if (lr < rows) {
+      const int per = kWave / R, rows = per * kNW;
+      int lr = (int)(((float)lane + 0.5f) / (float)R);
+      const int lc = lane - lr * R;
+      if (lr < per) {
+        lr += per * w;
         const int rx = x0 + (nfull << 5) + lc - ref.ox, ry0 = y0 + lr - ref.oy;
         int o = ry0 * ref.w + rx;
         const lds_float *t = win + (__umul24(ry0 + fv - 2 - wy0, wpitch) + (rx + fu - 2 - wx0));
@@ -2420,6 +2473,416 @@ struct Solver {
     }
     unc_record(pt, u, v, fields, nsub, gid);
     return true;
+  }
+
+  // -------------------------------------- translation-only Gauss-Newton ---
+  // With (u, v) as the only parameters (the reference's default) the warp is
+  // x' = cx + (u + dx), y' = cy + (v + dy): the x weights belong to a column of
+  // the subset and the y weights to a row, and the Keys sum separates.  A lane
+  // takes a column and steps down its rows; the row sums of the six window rows
+  // under its pixel stay in registers and each step adds one (12 multiply-adds,
+  // 6 taps and 8 broadcast words per value instead of 42, 36 and 34 operations
+  // for the weights) -- the products and their order are those of sample(), so
+  // the values are too.  The y weights of the rows are tabled once per pass.
+  // f(r, c, value) for every pixel of this wave's rows, and (one wave) g(r1)
+  // after each kTransChunk rows, r1 the rows done; returns after the group's
+  // sync.  S <= 64: a column per lane.
+  static constexpr int kTransChunk = 12;  // a multiple of the six rows that the unrolled walk turns its sums in
+  template <class F, class C>
+  __device__ __forceinline__ void trans_values(const Affine &A, F &&f, C &&g) {
+    const int lane = lid(), w = wid();
+    const int ra = S * w / kNW, rb = S * (w + 1) / kNW;
+    if constexpr (INTERP == 0) {
+      const float oxc = A.p[0] + (float)(lane - hw);
+#pragma unroll 1
+      for (int r0 = ra; r0 < rb; r0 += kTransChunk) {
+        const int r1 = min(r0 + kTransChunk, rb);
+        if (lane < S)
+          for (int r = r0; r < r1; ++r) f(r, lane, sample(oxc, A.p[1] + (float)(r - hw)));
+        if constexpr (kIsWave) g(r1);
+      }
+    } else {
+#pragma unroll 1
+      for (int r = grp.rank(); r < S; r += G::kSize) {
+        const float oy = A.p[1] + (float)(r - hw);
+        const float fly = floorf(oy);
+        float wy[6];
+        keys_weights(oy - fly, wy);
+        lds_float4 *q = (lds_float4 *)(ytab + 8 * r);
+        q[0] = float4v{wy[0], wy[1], wy[2], wy[3]};
+        q[1] = float4v{wy[4], wy[5], __int_as_float(cy - def.oy + (int)fly - 2 - wy0), 0.0f};
+      }
+      grp.sync();
+      auto row_of = [&](int r) { return __builtin_amdgcn_readfirstlane(__float_as_int(ytab[8 * r + 6])); };
+      // consecutive rows of the subset lie on consecutive window rows unless
+      // v + dy rounds across an integer
+      const int row0 = row_of(0);
+      const bool steady =
+          __ballot(lane < S && __float_as_int(ytab[8 * (lane < S ? lane : 0) + 6]) != row0 + lane) == 0ull;
+      const int c = min(lane, S - 1);  // the lanes past the last column repeat it
+      const float ox = A.p[0] + (float)(c - hw);
+      const float flx = floorf(ox);
+      float wx[6];
+      keys_weights(ox - flx, wx);
+      const lds_float *base = win + (cx - def.ox + (int)flx - 2 - wx0);
+      if (steady) {
+        auto rowsum = [&](const float (&a)[6]) {
+          float rs = a[0] * wx[0];
+#pragma unroll
+          for (int k = 1; k < 6; ++k) rs = fmaf(a[k], wx[k], rs);
+          return rs;
+        };
+        const lds_float *t = base + __umul24(row0 + ra, wpitch);
+        float h[6], a[6];
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+#pragma unroll
+          for (int k = 0; k < 6; ++k) a[k] = t[k];
+          h[m] = rowsum(a);
+          t += wpitch;
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k) a[k] = t[k];
+#pragma unroll 1
+        for (int r0 = ra; r0 < rb; r0 += kTransChunk) {
+          const int r1 = min(r0 + kTransChunk, rb);
+#pragma unroll 1
+          for (int r = r0; r < r1; r += 6) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+              if (r + j >= r1) break;
+              // the next row's taps first (past the last row: words of the slot, not used)
+              t += wpitch;
+              float b[6];
+#pragma unroll
+              for (int k = 0; k < 6; ++k) b[k] = t[k];
+              const lds_float4 *q = (const lds_float4 *)(ytab + 8 * (r + j));
+              const float4v w0 = q[0], w1 = q[1];
+              h[(j + 5) % 6] = rowsum(a);
+              float v = h[j] * w0.x;
+              v = fmaf(h[(j + 1) % 6], w0.y, v);
+              v = fmaf(h[(j + 2) % 6], w0.z, v);
+              v = fmaf(h[(j + 3) % 6], w0.w, v);
+              v = fmaf(h[(j + 4) % 6], w1.x, v);
+              v = fmaf(h[(j + 5) % 6], w1.y, v);
+              if (lane < S) f(r + j, lane, v);
+#pragma unroll
+              for (int k = 0; k < 6; ++k) a[k] = b[k];
+            }
+          }
+          if constexpr (kIsWave) g(r1);
+        }
+      } else {
+#pragma unroll 1
+        for (int r0 = ra; r0 < rb; r0 += kTransChunk) {
+          const int r1 = min(r0 + kTransChunk, rb);
+#pragma unroll 1
+          for (int r = r0; r < r1; ++r) {
+            const lds_float4 *q = (const lds_float4 *)(ytab + 8 * r);
+            const float4v w0 = q[0], w1 = q[1];
+            const float wy[6] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
+            const float v = keys_sum(base + __umul24(row_of(r), wpitch), wpitch, wx, wy);
+            if (lane < S) f(r, lane, v);
+          }
+          if constexpr (kIsWave) g(r1);
+        }
+      }
+    }
+    grp.sync();
+  }
+
+  // The reference values and gradients of a square subset into rtab (crew).
+  __device__ __forceinline__ void crew_tables() {
+    const int lane = lid(), w = wid();
+    const float inv = 1.0f / (float)S;
+    const unsigned o0 = (unsigned)((cy - hw - ref.oy) * ref.w + (cx - hw - ref.ox));
+#pragma unroll 2
+    for (int k0 = w * kWave; k0 < n; k0 += G::kSize) {
+      const int k = k0 + lane;
+      if (k < n) {
+        const int r = (int)(((float)k + 0.5f) * inv), c = k - r * S;  // exact: k < 2^14, S < 2^7
+        const unsigned o = o0 + (unsigned)(r * ref.w + c);
+        auto copy = [&](const gfloat *p, lds_float *to) {
+          __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void *)(p + o),
+                                           (__attribute__((address_space(3))) void *)(to + k0), 4, 0, 0);
+        };
+        if constexpr (std::is_same<T, float>::value) copy((const gfloat *)ref.pix, rtab);
+        else rtab[k] = Pix<T>::at_u(ref.pix, o);
+        copy((const gfloat *)ref.gx, rtab + n);
+        copy((const gfloat *)ref.gy, rtab + 2 * n);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    grp.sync();
+  }
+
+  // Per-subset constants of the translation-only solver in pers (kTrans*
+  // offsets), from the cache entry when it is current: sum(gx^2), sum(gx gy),
+  // sum(gy^2), sum(gx), sum(gy) and the mean reference intensity, in the order
+  // of precompute_phi (FP32 lane partials over pixels lane, lane + 64, ...), and
+  // the FP64 sums of F and F^2.  Returns false when the 2 x 2 matrix is not
+  // safely positive definite.
+  static constexpr int kTransS00 = 0, kTransS01 = 1, kTransS11 = 2, kTransPhi = 3, kTransMeanF = 5, kTransR = 6;
+  __device__ __forceinline__ bool trans_setup(int gid) {
+    const int lane = lid(), w = wid();
+    double *entry = kp.lean_cache ? kp.lean_cache + (size_t)gid * kLeanCacheDoubles : nullptr;
+    const double gen = (double)kp.lean_gen;
+    bool have = false;
+    if (entry) {
+      const double e = lane < kLeanCacheDoubles ? entry[lane] : 0.0;
+      have = lane_value(e, kLeanTag) == gen;
+      if (have && w == 0 && lane < 8) pers[lane] = e;
+    }
+    if (!have && w == 0) {
+      float pa[7];
+#pragma unroll
+      for (int k = 0; k < 7; ++k) pa[k] = 0.0f;
+      double rs[2] = {0.0, 0.0};
+      square_walk64([&](int, int o) {
+        float F, gx, gy;
+        ref_at(o, F, gx, gy);
+        pa[0] = fmaf(gx, gx, pa[0]);
+        pa[1] = fmaf(gx, gy, pa[1]);
+        pa[2] = fmaf(gy, gy, pa[2]);
+        pa[3] += gx;
+        pa[4] += gy;
+        pa[5] += F;
+        rs[0] += (double)F;
+        rs[1] = fma((double)F, (double)F, rs[1]);
+      });
+      double t[8];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) t[k] = wave_sum((double)pa[k]);
+      t[5] = (double)(float)(t[5] / (double)n);
+      t[6] = wave_sum(rs[0]);
+      t[7] = wave_sum(rs[1]);
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) pers[k] = t[k];
+        if (entry) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) entry[k] = t[k];
+          entry[kLeanTag] = gen;
+        }
+      }
+    }
+    grp.sync();
+    meanF = (float)uniform(pers[kTransMeanF]);
+    const double s00 = uniform(pers[kTransS00]), s01 = uniform(pers[kTransS01]), s11 = uniform(pers[kTransS11]);
+    // the pivots that ldlt_factor6 would test (the disabled parameters' are 1)
+    const double hmax = fmax(fmax(s00, s11), 1.0);
+    if (!(s00 > 1.0e-13 * hmax && hmax < 1.0e13)) return false;
+    const double l = s01 * (1.0 / s00);
+    return fma(-l, l * s00, s11) > 1.0e-13 * hmax;
+  }
+  // f(i, o) for pixels i = lane, lane + 64, ... of the square subset, o the
+  // reference pixel offset (one wave; the order of for_square in a wave).
+  template <class F>
+  __device__ __forceinline__ void square_walk64(F &&f) const {
+    const int lane = lid();
+    const float inv = 1.0f / (float)S;
+    const int drow = (int)(((float)kWave + 0.5f) * inv), dcol = kWave - drow * S;
+    const int row = (int)(((float)lane + 0.5f) * inv);
+    int col = lane - row * S;
+    int o = (cy - hw + row - ref.oy) * ref.w + (cx - hw + col - ref.ox);
+    const int ostep = drow * ref.w + dcol, owrap = ref.w - S;
+#pragma unroll 1
+    for (int i = lane; i < n; i += kWave) {
+      f(i, o);
+      o += ostep;
+      col += dcol;
+      if (col >= S) {
+        col -= S;
+        o += owrap;
+      }
+    }
+  }
+
+  // One Gauss-Newton pass at A: sum(gmf gx), sum(gmf gy), sum(G) into pers[
+  // kLeanPass, +3).  The lane partials are those of accumulate_gn_fast in a wave
+  // -- pixels lane, lane + 64, ... -- so the values go through gtab.  A crew's
+  // waves 0, 1 and 2 add one of the sums each.
+  __device__ __forceinline__ void accumulate_trans(const Affine &A, float shift) {
+    const int lane = lid();
+    if constexpr (kIsWave) {
+      // gtab holds kTransChunk rows: after each of them the lanes add their
+      // pixels of those rows (pixels lane, lane + 64, ... of the subset)
+      float pa[3] = {0.0f, 0.0f, 0.0f};
+      const float inv = 1.0f / (float)S;
+      const int drow = (int)(((float)kWave + 0.5f) * inv), dcol = kWave - drow * S;
+      const int row = (int)(((float)lane + 0.5f) * inv);
+      int i = lane, col = lane - row * S, done = 0;
+      int o = (cy - hw + row - ref.oy) * ref.w + (cx - hw + col - ref.ox);
+      const int ostep = drow * ref.w + dcol, owrap = ref.w - S;
+      trans_values(
+          A, [&](int r, int c, float v) { gtab[(r - done) * S + c] = v; },
+          [&](int r1) {
+            grp.sync();
+            const int end = r1 * S;
+            const lds_float *gt = gtab - done * S;
+            float F = 0.0f, gx = 0.0f, gy = 0.0f, Gv = 0.0f;
+            if (i < end) {
+              ref_at(o, F, gx, gy);
+              Gv = gt[i];
+            }
+#pragma unroll 1
+            while (i < end) {
+              // the next pixel's loads first: they are in flight during the sums
+              const float F0 = F, gx0 = gx, gy0 = gy, G0 = Gv;
+              i += kWave;
+              o += ostep;
+              col += dcol;
+              if (col >= S) {
+                col -= S;
+                o += owrap;
+              }
+              if (i < end) {
+                ref_at(o, F, gx, gy);
+                Gv = gt[i];
+              }
+              const float gmf = (G0 - shift) - (F0 - meanF);
+              pa[0] = fmaf(gmf, gx0, pa[0]);
+              pa[1] = fmaf(gmf, gy0, pa[1]);
+              pa[2] += G0;
+            }
+            done = r1;
+            grp.sync();
+          });
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double t = wave_sum((double)pa[k]);
+        if (lane == 0) pers[kLeanPass + k] = t;
+      }
+    } else {
+      trans_values(A, [&](int r, int c, float v) { gtab[r * S + c] = v; }, [](int) {});
+      const int w = wid();
+      if (w < 3) {
+        float p = 0.0f;
+        const lds_float *g = rtab + (w == 0 ? n : 2 * n);
+        if (w < 2) {
+#pragma unroll 4
+          for (int i = lane; i < n; i += kWave) {
+            const float gmf = (gtab[i] - shift) - (rtab[i] - meanF);
+            p = fmaf(gmf, g[i], p);
+          }
+        } else {
+#pragma unroll 4
+          for (int i = lane; i < n; i += kWave) p += gtab[i];
+        }
+        const double t = wave_sum((double)p);
+        if (lane == 0) pers[kLeanPass + w] = t;
+      }
+    }
+    grp.sync();
+  }
+
+  // Gauss-Newton of (u, v): gauss_newton's system with identity rows for the
+  // disabled parameters is the 2 x 2 one solved here.  kOverflow: as in
+  // gauss_newton_lean.
+  __device__ __forceinline__ int gauss_newton_trans(Affine &A, int &iters, double *fields, int nsub, int gid) {
+    const double s00 = uniform(pers[kTransS00]), s01 = uniform(pers[kTransS01]), s11 = uniform(pers[kTransS11]);
+    const float cond = wave_uniform_f(cond2x2(s00, s01, s01, s11));
+    const double inv0 = 1.0 / s00, l = s01 * inv0, inv1 = 1.0 / fma(-l, l * s00, s11);
+    float shift = meanF;
+    int it = 0;
+    A.prepare();  // (of the disabled parameters: the identity, at every step)
+#pragma unroll 1
+    for (; it <= kp.max_fast; ++it) {
+      iters = it;
+      if (!stage_affine(A) || !all_kept(A)) return kOverflow;
+      accumulate_trans(A, shift);
+      const float meanG = (float)(uniform(pers[kLeanPass + 2]) / (double)n);
+      const double corr = (double)meanG - (double)shift;
+      if (it == 0 && grp.rank() == 0) fields[(size_t)F_CONDITION * nsub + gid] = cond;
+      if (cond > 1.0e12f) return HESSIAN_SINGULAR;
+      const double q0 = uniform(pers[kLeanPass]) - corr * uniform(pers[kTransPhi]);
+      const double q1 = uniform(pers[kLeanPass + 1]) - corr * uniform(pers[kTransPhi + 1]);
+      const double d1 = fma(l, q0, -q1) * inv1;
+      const double d0 = fma(-l, d1, -q0 * inv0);
+      const float old0 = A.p[0], old1 = A.p[1];
+      A.p[0] += wave_uniform_f((float)d0);
+      A.p[1] += wave_uniform_f((float)d1);
+      // test_for_convergence (DICe_LocalShapeFunction.cpp:433-459)
+      if (fabsf(A.p[0] - old0) < kp.fast_tol && fabsf(A.p[1] - old1) < kp.fast_tol) {
+        if (kp.uncertainty) {
+          // a window that the general kernel's uncertainty pass would not fit hands the subset over there too
+          const int fu = (int)floorf(A.p[0]), fv = (int)floorf(A.p[1]);
+          const int ww = min(bx1 - ref.ox + fu + 4, def.w - 1) - max(bx0 - ref.ox + fu - 3, 0) + 1;
+          const int hh = min(by1 - ref.oy + fv + 4, def.h - 1) - max(by0 - ref.oy + fv - 3, 0) + 1;
+          if (ww > 0 && hh > 0 && ww * hh > win_cap) return kOverflow;
+          if (!lean_uncertainty(A, fields, nsub, gid)) return kOverflow;
+        }
+        break;
+      }
+      shift = meanG;
+    }
+    return it > kp.max_fast ? MAX_ITERATIONS_REACHED : CORRELATION_SUCCESSFUL;
+  }
+
+  // The gamma sums of gamma_sums_every at a translation (sd, sdd, sdr; the
+  // reference sums are per-subset constants).
+  __device__ __forceinline__ void gamma_sums_trans(const Affine &A, double (&acc)[6]) {
+    double t[3] = {0.0, 0.0, 0.0};
+    const int o0 = (cy - hw - ref.oy) * ref.w + (cx - hw - ref.ox);
+    trans_values(A, [&](int r, int c, float v) {
+      const double d = v;
+      const double rv = kIsWave ? Pix<T>::at_u(ref.pix, (unsigned)(o0 + r * ref.w + c)) : rtab[r * S + c];
+      t[0] += d;
+      t[1] = fma(d, d, t[1]);
+      t[2] = fma(d, rv, t[2]);
+    }, [](int) {});
+    grp.sum(t);
+    acc[1] = t[0];
+    acc[2] = t[1];
+    acc[3] = uniform(pers[kTransR]);
+    acc[4] = uniform(pers[kTransR + 1]);
+    acc[5] = t[2];
+  }
+
+  // A crew's pass of the six-parameter solver: accumulate_gn_fast<true> with the
+  // interpolation shared by the waves, the values through gtab, and the sums
+  // (each in one wave, in the order of for_strips) shared too.
+  __device__ __forceinline__ void accumulate_crew(const Affine &A, float shift) {
+    {
+      const float inv = 1.0f / (float)S;
+#pragma unroll 1
+      for (int k = grp.rank(); k < n; k += G::kSize) {
+        const int r = (int)(((float)k + 0.5f) * inv), c = k - r * S;  // exact: k < 2^14, S < 2^7
+        float ox, oy;
+        A.disp((float)(c - hw), (float)(r - hw), ox, oy);
+        gtab[k] = sample(ox, oy);
+      }
+    }
+    grp.sync();
+    const int w = wid(), lane = lid();
+    const int x0 = cx - hw, y0 = cy - hw;
+    if (w < 3) {
+      float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f;
+      const lds_float *g = rtab + (w == 0 ? n : 2 * n);
+      if (w < 2) {
+        for_strips<false>([&](int x, int y, float dx, float dy, int) {
+          const int i = (y - y0) * S + (x - x0);
+          const float gmf = (gtab[i] - shift) - (rtab[i] - meanF);
+          const float gv = g[i], g1 = gmf * gv;
+          p0 = DICE_CREW_ADD(gmf, gv, g1, p0);
+          p1 = fmaf(g1, dx, p1);
+          p2 = fmaf(g1, dy, p2);
+        });
+      } else {
+        for_strips<false>([&](int x, int y, float, float, int) { p0 += gtab[(y - y0) * S + (x - x0)]; });
+      }
+      // slots: gx 0, gy 1, dx gx 2, dy gx 3, dx gy 4, dy gy 5, G 6
+      const double t0 = wave_sum((double)p0);
+      if (lane == 0) pers[kLeanPass + (w == 2 ? 6 : w)] = t0;
+      if (w < 2) {
+        const double t1 = wave_sum((double)p1), t2 = wave_sum((double)p2);
+        if (lane == 0) {
+          pers[kLeanPass + 2 + 2 * w] = t1;
+          pers[kLeanPass + 3 + 2 * w] = t2;
+        }
+      }
+    }
+    grp.sync();
   }
 
   // Gauss-Newton of the lean kernel (all six parameters, no LM term or
@@ -2443,7 +2906,8 @@ struct Solver {
 #pragma unroll
       for (int k = 0; k < 6; ++k) p_state[k] = A.p[k];
       if (!stage_affine(A) || !all_kept(A)) return kOverflow;
-      accumulate_gn_fast<true>(A, shift, kLeanPass);
+      if constexpr (kIsWave) accumulate_gn_fast<true>(A, shift, kLeanPass);
+      else accumulate_crew(A, shift);
       const double cnt = (double)n_def_active;
       const float meanG = cnt > 0.0 ? (float)(uniform(pers[kLeanPass + 6]) / cnt) : 0.0f;
       const double corr = (double)meanG - (double)shift;
@@ -2520,44 +2984,23 @@ struct Solver {
       if (!stage_affine(A)) return kOverflow;
       float du[6];
       float meanG;
-      if constexpr (kTeam) {
-        // every pixel kept (else the PLAIN kernel takes the subset): H = M S M^T
-        // from the per-subset sums, q from the pass (see fast_system)
-        if (!all_kept(A)) return kOverflow;
-        last_fast = true;
-        double acc[7];
-        accumulate_gn_wide(A, shift, acc);
-        const double cnt = (double)n_def_active;
-        meanG = cnt > 0.0 ? (float)(acc[6] / cnt) : 0.0f;
-        const double corr = (double)meanG - (double)shift;
-        double H[6][6], q[6], sr[6];
-        fast_matrix(A, H);
-        fast_rows(A, [&](int l) { return (double)pers[36 + l]; }, sr);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) q[k] = acc[k] - corr * sr[k];
-        finish_system(H, q);
-        const float cond = cond2x2(H[0][0], H[0][1], H[0][1], H[1][1]);
-        if (grp.rank() == 0) fields[(size_t)F_CONDITION * nsub + gid] = cond;
-        if (cond > 1.0e12f) return HESSIAN_SINGULAR;
-        double dd[6];
-        if (!ldlt_update6(H, q, dd)) return kOverflow;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) du[k] = wave_uniform_f((float)dd[k]);
-      } else if constexpr (!kIsWave) {
+      if constexpr (!kIsWave) {
+        if constexpr (kTeam) last_fast = all_kept(A);
         double acc[35];
         accumulate_gn_block(A, shift, acc);
-        const double cnt = acc[34];
-        meanG = cnt > 0.0 ? (float)(acc[33] / cnt) : 0.0f;
+        auto tot = [&](int k) -> double { return kTeam ? (double)pers[kWideTot + k] : acc[k]; };
+        const double cnt = tot(34);
+        meanG = cnt > 0.0 ? (float)(tot(33) / cnt) : 0.0f;
         const double corr = (double)meanG - (double)shift;
         double q[6], H[6][6];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) q[k] = acc[k] - corr * acc[27 + k];
+        for (int k = 0; k < 6; ++k) q[k] = tot(k) - corr * tot(27 + k);
         {
           int h = 6;
 #pragma unroll
           for (int k = 0; k < 6; ++k)
 #pragma unroll
-            for (int l = k; l < 6; ++l) { H[k][l] = acc[h]; H[l][k] = acc[h]; ++h; }
+            for (int l = k; l < 6; ++l) { H[k][l] = H[l][k] = tot(h); ++h; }
         }
         // disabled parameters: identity rows, zero gradient (same solution as the
         // reduced N x N system of the reference)
@@ -2574,9 +3017,12 @@ struct Solver {
         if (grp.rank() == 0) fields[(size_t)F_CONDITION * nsub + gid] = cond;
         if (cond > 1.0e12f) return HESSIAN_SINGULAR;
         double dd[6];
-        if (!ldlt_update6(H, q, dd)) lu_update6(H, q, dd);
+        if (!ldlt_update6(H, q, dd)) {
+          if constexpr (kTeam) return kOverflow;  // the PLAIN kernel's pivoted LU
+          else lu_update6(H, q, dd);
+        }
 #pragma unroll
-        for (int k = 0; k < 6; ++k) du[k] = (float)dd[k];
+        for (int k = 0; k < 6; ++k) du[k] = kTeam ? wave_uniform_f((float)dd[k]) : (float)dd[k];
       } else {
         // every lane builds the whole system (the same values in all lanes) and
         // solves it by L D L^T; the pivoted LU is the fallback
@@ -2966,7 +3412,8 @@ struct Solver {
 
   // Immerkaer noise estimate (Subset::noise_std_dev, DICe_Subset.cpp:622-703)
   // over the bbox of the kept pixels at p_state, shifted by the final (u, v).
-  template <bool LEAN = false>
+  // LEAN: the separable walk for the common case, lane partials of type Part.
+  template <bool LEAN = false, typename Part = float>
   __device__ __forceinline__ float noise_std_dev(int min_x, int max_x, int min_y, int max_y, float u, float v) {
     min_x = (int)((float)min_x + u);
     max_x = (int)((float)max_x + u);
@@ -2990,21 +3437,23 @@ struct Solver {
       // row-filtered values of the rows around its pixel; FP32 lane partials
       const int lx0 = min_x - ox, ly0 = min_y - oy;
       if (bw > 0 && bh > 0 && lx0 >= 1 && ly0 >= 1 && lx0 + bw <= iw - 1 && ly0 + bh <= ih - 1 &&
-          stage(lx0 - 1, lx0 + bw, ly0 - 1, ly0 + bh, false)) {
-        const int lane = grp.rank();
-        float part = 0.0f;
+          stage(lx0 - 1, lx0 + bw, ly0 - 1, ly0 + bh, false) && (!kTeam || win_ok)) {
+        const int lane = lid(), w = wid();
+        const int ra = bh * w / kNW, rb = bh * (w + 1) / kNW;  // this wave's rows
+        Part part = 0;
         auto rowf = [&](const lds_float *p) { return (p[-1] + p[1]) - 2.0f * p[0]; };
-        auto column = [&](int c, int r0, int step) {
+        auto column = [&](int c, int r0) {
+          if (kNW > 1 && r0 >= rb) return;  // (one wave: r0 <= 1 lies in the staged rows)
           const lds_float *t = win + (__umul24(ly0 + r0 - wy0, wpitch) + (lx0 + c - wx0));
-          const int tstep = step * wpitch;
+          const int tstep = 2 * wpitch;
           {
             float cm = rowf(t - wpitch), c0 = rowf(t), cp = rowf(t + wpitch);
 #pragma unroll 1
-            for (int r = r0; r < bh; r += 2) {
-              part += fabsf((cm + cp) - 2.0f * c0);
+            for (int r = r0; r < rb; r += 2) {
+              part += (Part)fabsf((cm + cp) - 2.0f * c0);
               t += tstep;
               cm = cp;
-              if (r + 2 < bh) {
+              if (r + 2 < rb) {
                 c0 = rowf(t);
                 cp = rowf(t + wpitch);
               }
@@ -3013,19 +3462,21 @@ struct Solver {
         };
         const int nfull = bw >> 5;
 #pragma unroll 1
-        for (int st = 0; st < nfull; ++st) column((st << 5) + (lane & 31), lane >> 5, 2);
+        for (int st = 0; st < nfull; ++st) column((st << 5) + (lane & 31), ra + (lane >> 5));
         const int R = bw & 31;
         if (R) {
           // the last columns column-major over the lanes (consecutive rows: a
           // window pitch apart, distinct banks for an odd pitch)
-          int c = (int)(((float)lane + 0.5f) / (float)bh);
-          int r = lane - c * bh;
-          const int dc = kWave / bh, dr = kWave - dc * bh;
+          constexpr int all = kWave * kNW;
+          const int k0 = lane + kWave * w;
+          int c = (int)(((float)k0 + 0.5f) / (float)bh);
+          int r = k0 - c * bh;
+          const int dc = all / bh, dr = all - dc * bh;
           const lds_float *t = win + (__umul24(ly0 + r - wy0, wpitch) + (lx0 + (nfull << 5) + c - wx0));
           const int tstep = dc + dr * wpitch, twrap = 1 - bh * wpitch;
 #pragma unroll 1
-          for (int k = lane; k < R * bh; k += kWave) {
-            part += fabsf((rowf(t - wpitch) + rowf(t + wpitch)) - 2.0f * rowf(t));
+          for (int k = k0; k < R * bh; k += all) {
+            part += (Part)fabsf((rowf(t - wpitch) + rowf(t + wpitch)) - 2.0f * rowf(t));
             c += dc;
             r += dr;
             t += tstep;
@@ -3094,11 +3545,11 @@ struct Solver {
         // the last warp kept every active pixel: the gradient sums are
         // sum(phi phi^T)[0][0] and [1][1], the kept bbox is the bbox of the
         // active pixels (with the centroid, where the general path starts)
-        if (S > 0) noise = noise_std_dev(bx0, bx1, by0, by1, A.p[0], A.p[1]);
-        else noise = noise_std_dev(min(cx, abx0), max(cx, abx1), min(cy, aby0), max(cy, aby1), A.p[0], A.p[1]);
+        // (a workgroup: the separable walk with FP64 lane partials)
+        if (S > 0) noise = noise_std_dev<kTeam, double>(bx0, bx1, by0, by1, A.p[0], A.p[1]);
+        else noise = noise_std_dev<kTeam, double>(min(cx, abx0), max(cx, abx1), min(cy, aby0), max(cy, aby1), A.p[0], A.p[1]);
         if (noise < 0.0f) return -1.0f;
-        const float sgx = (float)uniform(kTeam ? pers[kWideSg] : pers[0]);
-        const float sgy = (float)uniform(kTeam ? pers[kWideSg + 1] : pers[7]);
+        const float sgx = (float)uniform(pers[0]), sgy = (float)uniform(pers[kTeam ? 1 : 7]);
         const float sg = sgx > sgy ? sgy : sgx;
         return sg > 0.0f ? (float)sqrt(2.0 * (double)noise * (double)noise / (double)sg) : -1.0f;
       }
@@ -3383,8 +3834,12 @@ struct Solver {
   // ov_list for the general kernel, which starts it again from its initial
   // guess: the lean pass has then written nothing but CONDITION and FIELD_1..7,
   // which that run writes again.
+  // TRANS: the translation-only solver for the same cases (u, v the only
+  // parameters), in the arithmetic of run() for them.  In a crew (one workgroup
+  // per subset) setup(gid) forms the six-parameter constants in wave 0.
+  template <bool TRANS, class Setup>
   __device__ __forceinline__ void run_lean(const DSubsets &ss, int gid, double *fields, int *fb_list,
-                                           int *fb_count, int *ov_list, int *ov_count) {
+                                           int *fb_count, int *ov_list, int *ov_count, Setup &&setup) {
     const int nsub = ss.n;
     set_subset(ss, gid);
     if (S <= 0 || !ref_in || cx - hw < 0 || cy - hw < 0 || mw > 0 || forced) {
@@ -3410,14 +3865,20 @@ struct Solver {
     Affine A;
     init_params(A, fields, nsub, gid);
     const int init_status = kp.guess ? (int)kp.guess[(size_t)7 * nsub + gid] : INITIALIZE_USING_PREVIOUS_FRAME_SUCCESSFUL;
-    if (!lean_setup(gid)) {
+    bool ready;
+    if constexpr (TRANS) ready = trans_setup(gid);
+    else ready = setup(gid);
+    if (!ready) {
       push(ov_list, ov_count, gid);
       return;
     }
+    if constexpr (!kIsWave) crew_tables();
     const float prev_u = (float)fv(F_DISP_X), prev_v = (float)fv(F_DISP_Y), prev_t = (float)fv(F_ROT_Z);
     float p_state[6];
     int iters = -1;
-    const int corr = gauss_newton_lean(A, iters, p_state, fields, nsub, gid);
+    int corr;
+    if constexpr (TRANS) corr = gauss_newton_trans(A, iters, fields, nsub, gid);
+    else corr = gauss_newton_lean(A, iters, p_state, fields, nsub, gid);
     if (corr == kOverflow) {
       push(ov_list, ov_count, gid);
       return;
@@ -3438,10 +3899,13 @@ struct Solver {
     // sigma with the last warp keeping every pixel: noise over the subset bbox
     // shifted by (u, v), gradient sums sum(gx^2), sum(gy^2) from S
     // (Objective::sigma, DICe_Objective.cpp:150-184)
-    const float noise = noise_std_dev<true>(bx0, bx1, by0, by1, A.p[0], A.p[1]);
+    // (TRANS: FP64 lane partials, as in noise_std_dev's general walk)
+    using Part = typename std::conditional<TRANS, double, float>::type;
+    const float noise = noise_std_dev<true, Part>(bx0, bx1, by0, by1, A.p[0], A.p[1]);
     float sig = -1.0f;
     if (noise >= 0.0f) {
-      const float sgx = (float)uniform(pers[kLeanS00]), sgy = (float)uniform(pers[kLeanS11]);
+      const float sgx = (float)uniform(pers[TRANS ? kTransS00 : kLeanS00]);
+      const float sgy = (float)uniform(pers[TRANS ? kTransS11 : kLeanS11]);
       const float sg = sgx > sgy ? sgy : sgx;
       sig = sg > 0.0f ? (float)sqrt(2.0 * (double)noise * (double)noise / (double)sg) : -1.0f;
     }
@@ -3449,14 +3913,18 @@ struct Solver {
       record_failed(fields, nsub, gid, FRAME_FAILED_DUE_TO_NEGATIVE_SIGMA, iters);
       return;
     }
-    A.prepare();
+    if constexpr (!TRANS) A.prepare();
     if (!stage_affine(A) || !all_kept(A)) {
       push(ov_list, ov_count, gid);
       return;
     }
     double acc[6] = {0, 0, 0, 0, 0, 0};
-    gamma_sums_every<true>(A, acc);
-    grp.sum(acc);
+    if constexpr (TRANS) {
+      gamma_sums_trans(A, acc);
+    } else {
+      gamma_sums_every<true>(A, acc);
+      grp.sum(acc);
+    }
     acc[0] = (double)n_def_active;
     int active;
     float contrast;
@@ -3518,6 +3986,8 @@ struct Items {
 struct LaneGroup {
   static constexpr int kSize = 1;
   static constexpr bool kWindow = false;
+  static constexpr bool kHandOver = false;
+  static constexpr bool kTight = false;
   __device__ __forceinline__ int rank() const { return 0; }
   __device__ __forceinline__ void sync() const {}
   template <int K>
@@ -4076,7 +4546,7 @@ struct BlockClaims {
 // 0.59 ms, and 0.95 against 1.08 ms for the polygons, measured with an earlier
 // reduction).
 #ifndef DICE_WIDE_WPE
-#define DICE_WIDE_WPE 4
+#define DICE_WIDE_WPE 3
 #endif
 template <typename T, int INTERP, bool SIMPLEX_OPT, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT > 512 ? 4 : DICE_WIDE_WPE))) void correlate_wide_kernel(
@@ -4193,7 +4663,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DICE_BATCHE
       ++visited;
       continue;
     }
-    s.run_lean(ss, items.at(k), fields, pa.fb_list, pa.fb_count, pa.ov_list, pa.ov_count);
+    s.template run_lean<false>(ss, items.at(k), fields, pa.fb_list, pa.fb_count, pa.ov_list, pa.ov_count,
+                               [&](int gid) { return s.lean_setup(gid); });
   }
 }
 
@@ -4203,6 +4674,124 @@ hipError_t launch_lean_variant(const Launch &L, const KParams &kp, const DImage 
   const size_t shm = (size_t)L.waves_per_group * L.lds_floats_per_wave * sizeof(float);
   hipLaunchKernelGGL((correlate_lean_kernel<T, INTERP>), dim3(L.groups), dim3(L.waves_per_group * kWave), shm,
                      stream, kp, ref, def, subs, fields, pa, L.lds_floats_per_wave);
+  return hipGetLastError();
+}
+
+// The window of a translated square subset: S + 6 pixels a side at most (the
+// taps and a fractional shift), S + 11 and S + 12 with the ring and the odd
+// pitch; a multiple of four floats.
+__host__ __device__ inline int trans_window_floats(int side, int cap) {
+  const int w = ((side + 12) * (side + 11) + 3) & ~3;
+  return w < cap ? w : cap & ~3;
+}
+
+#ifndef DICE_TRANS_WPE
+#define DICE_TRANS_WPE 3
+#endif
+// BATCHED translation-only Gauss-Newton pass: one wave per subset (and per
+// workgroup), Solver::run_lean<true>.  A wave's LDS: the slot, then gtab and ytab.
+template <typename T, int INTERP>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_WPE))) void correlate_trans_kernel(
+    KParams kp, DImage ref, DImage def, DSubsets ss, double *fields, PassArgs pa, int slot) {
+  extern __shared__ float lds[];
+  const Items items{pa.items, pa.item_count, ss.order};
+  TightWave g;
+  g.lane = (int)threadIdx.x;
+  lds_float *const base = (lds_float *)lds;
+  Solver<T, TightWave, INTERP, false> s(kp, ref, def, g, base, slot);
+  const int side = 2 * (ss.S / 2) + 1;
+  s.win_phys = trans_window_floats(side, s.win_cap);
+  s.pers = (lds_double *)(base + s.win_phys);
+  s.ytab = base + s.win_phys + kPersistFloats;
+  s.gtab = s.ytab + 8 * side;
+  const int total = items.total(ss.n);
+  if ((int)blockIdx.x >= total) return;  // as in correlate_batched_kernel
+  int range = (int)(blockIdx.x % kWorkRanges);
+#pragma unroll 1
+  for (int visited = 0; visited < kWorkRanges;) {
+    const int lo = (int)((long long)total * range / kWorkRanges);
+    const int hi = (int)((long long)total * (range + 1) / kWorkRanges);
+    int k = 0;
+    if (threadIdx.x == 0) k = atomicAdd(pa.counter + range * kCounterStride, 1);
+    k = __builtin_amdgcn_readfirstlane(k) + lo;
+    if (k >= hi) {
+      range = range + 1 == kWorkRanges ? 0 : range + 1;
+      ++visited;
+      continue;
+    }
+    s.template run_lean<true>(ss, items.at(k), fields, pa.fb_list, pa.fb_count, pa.ov_list, pa.ov_count,
+                              [](int) { return false; });
+  }
+}
+
+// The same two passes with few subsets: four waves per subset.
+template <typename T, int INTERP, bool TRANS>
+__global__ __launch_bounds__(256) void correlate_crew_kernel(KParams kp, DImage ref, DImage def, DSubsets ss,
+                                                             double *fields, PassArgs pa, int slot) {
+  extern __shared__ float lds[];
+  __shared__ double red[CrewGroup::kWaves * kTeamRed];
+  __shared__ int next;
+  const Items items{pa.items, pa.item_count, ss.order};
+  const int total = items.total(ss.n);
+  if ((int)blockIdx.x >= total) return;
+  CrewGroup g;
+  g.red = (lds_double *)red;
+  lds_float *const base = (lds_float *)lds;
+  Solver<T, CrewGroup, INTERP, false> s(kp, ref, def, g, base, slot - kPersistFloats);
+  s.pers = (lds_double *)(base + slot - kPersistFloats);
+  const int side = 2 * (ss.S / 2) + 1;
+  s.ytab = base + slot;
+  s.gtab = s.ytab + 8 * side;
+  s.rtab = s.gtab + side * side;
+  BlockClaims claims(pa.counter, total);
+#pragma unroll 1
+  for (int k = claims.take(&next); k >= 0; k = claims.take(&next)) {
+    s.template run_lean<TRANS>(ss, items.at(k), fields, pa.fb_list, pa.fb_count, pa.ov_list, pa.ov_count,
+                               [&](int gid) {
+                                 // wave 0 as a solver of its own on the same slot
+                                 if (s.wid() == 0) {
+                                   WaveGroup wg{(int)threadIdx.x};
+                                   Solver<T, WaveGroup, INTERP, false> one(kp, ref, def, wg, base, slot);
+                                   one.set_subset(ss, gid);
+                                   const bool ok = one.lean_setup(gid);
+                                   if (threadIdx.x == 0) next = ok ? 1 : 0;
+                                 }
+                                 __syncthreads();
+                                 const bool ok = __builtin_amdgcn_readfirstlane(next) != 0;
+                                 s.meanF = (float)uniform(s.pers[kLeanMeanF]);
+                                 __syncthreads();
+                                 return ok;
+                               });
+    __syncthreads();
+  }
+}
+
+// LDS floats of a wave of correlate_trans_kernel and of a crew: the slot (the
+// window and the per-subset constants), ytab, gtab, and a crew's reference tables.
+inline int trans_lds_floats(int S, int slot, bool crew) {
+  const int side = 2 * (S / 2) + 1;
+  if (crew) return slot + 8 * side + 4 * side * side;
+  return trans_window_floats(side, slot - kPersistFloats) + kPersistFloats +
+         (8 + Solver<float, TightWave, 2, false>::kTransChunk) * side;
+}
+
+template <typename T, int INTERP, bool TRANS>
+hipError_t launch_crew_variant(const Launch &L, const KParams &kp, const DImage &ref, const DImage &def,
+                               const DSubsets &subs, double *fields, const PassArgs &pa, hipStream_t stream) {
+  const size_t shm = (size_t)trans_lds_floats(subs.S, L.lds_floats_per_wave, true) * sizeof(float);
+  hipLaunchKernelGGL((correlate_crew_kernel<T, INTERP, TRANS>), dim3(subs.n), dim3(256), shm, stream, kp, ref, def,
+                     subs, fields, pa, L.lds_floats_per_wave);
+  return hipGetLastError();
+}
+
+template <typename T, int INTERP>
+hipError_t launch_trans_variant(const Launch &L, const KParams &kp, const DImage &ref, const DImage &def,
+                                const DSubsets &subs, double *fields, const PassArgs &pa, hipStream_t stream) {
+  const size_t shm = (size_t)trans_lds_floats(subs.S, L.lds_floats_per_wave, false) * sizeof(float);
+  const int per_cu = (int)((160 * 1024) / shm) < 4 * DICE_TRANS_WPE ? (int)((160 * 1024) / shm) : 4 * DICE_TRANS_WPE;
+  const int groups = subs.n < L.num_cus * per_cu ? subs.n : L.num_cus * per_cu;
+  hipLaunchKernelGGL((correlate_trans_kernel<T, INTERP>), dim3(groups), dim3(64), shm, stream, kp, ref, def, subs,
+                     fields, pa, L.lds_floats_per_wave);
   return hipGetLastError();
 }
 

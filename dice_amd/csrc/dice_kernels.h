@@ -137,6 +137,13 @@ struct Launch {
   int num_cus;
 };
 
+// Dynamic LDS of a launch without further attributes.
+constexpr size_t kMaxLaunchLds = 64 * 1024 - 2048;
+#ifndef DICE_CREW_MAX
+#define DICE_CREW_MAX 1024
+#endif
+constexpr int kCrewMaxSubsets = DICE_CREW_MAX;
+
 // Subsets of at most this many pixels run the Nelder-Mead iterations of the
 // BATCHED mode in rows of 16 lanes per subset (simplex_groups_kernel): a wave
 // then works on four subsets instead of spreading a few dozen pixels over 64

@@ -20,6 +20,11 @@ hipError_t launch_gn_lean(int, int, const Launch &, const KParams &, const DImag
                           double *, const PassArgs &, hipStream_t);
 hipError_t launch_simplex_batched(int, int, int, const Launch &, const KParams &, const DImage &, const DImage &,
                                   const DSubsets &, double *, const PassArgs &, hipStream_t);
+hipError_t launch_gn_trans(int, int, const Launch &, const KParams &, const DImage &, const DImage &, const DSubsets &,
+                           double *, const PassArgs &, hipStream_t);
+hipError_t launch_gn_crew(int, int, int, const Launch &, const KParams &, const DImage &, const DImage &,
+                          const DSubsets &, double *, const PassArgs &, hipStream_t);
+int trans_lds_floats(const Launch &, int, int);
 hipError_t launch_gn_wide(int, int, const Launch &, const KParams &, const DImage &, const DImage &, const DSubsets &,
                           double *, const PassArgs &, hipStream_t);
 hipError_t launch_simplex_wide(int, int, const Launch &, const KParams &, const DImage &, const DImage &,
@@ -693,20 +698,31 @@ static hipError_t launch_pass(bool simplex, int storage, const Launch &L, const 
   hipError_t e;
   const bool wide_only = L.wide_only && !defgrad;
   if (!wide_only) {
-    // Gauss-Newton pass 0 of square subsets with none of the options the lean
-    // kernel leaves out: the lean kernel takes every subset first and hands the
-    // others (and those that leave its common case) to the general kernel
+    // Gauss-Newton pass 0 of square subsets with none of the options that the
+    // common-case kernels leave out: they take every subset first and hand the
+    // others (and those that leave the common case) to the general kernel.  All
+    // six parameters: the lean kernel; translation only: its own kernel; few
+    // subsets of either kind: four waves each.
+    const int np = (kp.en_rot != 0) + (kp.en_normal != 0) + (kp.en_shear != 0);
     if (!simplex && pa.pass == 0 && subs.S > 0 && !subs.mbox && !kp.def_grads && kp.momentum == 0.0f &&
-        kp.init_gamma_thr == -1.0 && !kp.has_forced && kp.en_rot && kp.en_normal && kp.en_shear &&
-        kp.lm_alpha <= 0.0f) {
+        kp.init_gamma_thr == -1.0 && !kp.has_forced && kp.lm_alpha <= 0.0f && (np == 3 || np == 0)) {
       PassArgs pl = pa;
       pl.counter = work + kWorkSetLean * kWorkCounterInts;
       pl.ov_list = other;
       pl.ov_count = work + kWorkLeanCount;
-      e = launch_gn_lean(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
+      auto fits = [&](int crew) { return subs.S <= 64 && trans_lds_floats(L, subs.S, crew) * sizeof(float) <= kMaxLaunchLds; };
+      const bool crew = subs.n <= kCrewMaxSubsets && fits(1);
+      e = hipSuccess;
+      bool taken = true;
+      if (crew) e = launch_gn_crew(storage, kp.interp, np == 0, L, kp, ref, def, subs, fields, pl, stream);
+      else if (np == 3) e = launch_gn_lean(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
+      else if (fits(0)) e = launch_gn_trans(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
+      else taken = false;
       if (e != hipSuccess) return e;
-      pa.items = pl.ov_list;
-      pa.item_count = pl.ov_count;
+      if (taken) {
+        pa.items = pl.ov_list;
+        pa.item_count = pl.ov_count;
+      }
     }
     if (simplex && L.lane_simplex) {
       float *nm = reinterpret_cast<float *>(work + kWorkHeader + 3 * n);
