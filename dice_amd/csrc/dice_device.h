@@ -310,6 +310,8 @@ template <> struct Pix<float> {
   __device__ __forceinline__ static float at(const void *p, int i) { return ((const gfloat *)p)[i]; }
   __device__ __forceinline__ static float at_u(const void *p, unsigned i) { return ldf_u(p, i); }
   __device__ __forceinline__ static const gfloat *ptr(const void *p) { return (const gfloat *)p; }
+  typedef float Raw;
+  __device__ __forceinline__ static Raw raw_u(const void *p, unsigned i) { return ldf_u(p, i); }
 };
 template <> struct Pix<uint16_t> {
   typedef gu16 G;
@@ -318,6 +320,12 @@ template <> struct Pix<uint16_t> {
     return (float)*(const gu16 *)((const gchar *)p + (i << 1));
   }
   __device__ __forceinline__ static const gu16 *ptr(const void *p) { return (const gu16 *)p; }
+  // an element as it is loaded: a value kept for later use is converted there,
+  // since the conversion waits for the load
+  typedef unsigned Raw;
+  __device__ __forceinline__ static Raw raw_u(const void *p, unsigned i) {
+    return *(const gu16 *)((const gchar *)p + (i << 1));
+  }
 };
 // Kept for the image-level kernels.
 template <typename T> __device__ __forceinline__ float ldpix(const void *p, int i) { return Pix<T>::at(p, i); }
@@ -731,10 +739,10 @@ struct Solver {
   float meanF;
   float en[6];  // 1 for enabled parameters
   // Tables of correlate_trans_kernel / correlate_crew_kernel (LDS, square
-  // subsets, row-major): the interpolated values (n floats), per row of the
-  // subset its six y weights and its window row (8 floats each), and (crew) the
-  // reference values and gradients F, gx, gy (n floats each).
-  lds_float *gtab = nullptr, *ytab = nullptr, *rtab = nullptr;
+  // subsets, row-major): the interpolated values (n floats; a wave: four floats
+  // for each pixel of kTransChunk rows) and (crew) the reference values and gradients F, gx, gy (n
+  // floats each).
+  lds_float *gtab = nullptr, *rtab = nullptr;
   int win_phys = 0;  // G::kTight
 
   __device__ __forceinline__ Solver(const KParams &k, const DImage &r, const DImage &d, G g, lds_float *w, int cap)
@@ -862,6 +870,13 @@ struct Solver {
   // reference intensity and gradients at pixel offset o of the reference image
   __device__ __forceinline__ void ref_at(int o, float &F, float &gx, float &gy) const {
     F = Pix<T>::at_u(ref.pix, (unsigned)o);
+    gx = ldf_u(ref.gx, (unsigned)o);
+    gy = ldf_u(ref.gy, (unsigned)o);
+  }
+  // the same with the intensity as it is loaded
+  typedef typename Pix<T>::Raw Raw;
+  __device__ __forceinline__ void ref_raw(int o, Raw &F, float &gx, float &gy) const {
+    F = Pix<T>::raw_u(ref.pix, (unsigned)o);
     gx = ldf_u(ref.gx, (unsigned)o);
     gy = ldf_u(ref.gy, (unsigned)o);
   }
@@ -1075,7 +1090,7 @@ struct Solver {
       }
       __builtin_amdgcn_s_waitcnt(0);
     } else {
-#pragma unroll 4
+#pragma unroll 8
       for (int k = grp.rank(); k < tot; k += G::kSize) {
         const int r = (int)(((float)k + 0.5f) * inv);
         const int c = k - r * ww_s;
@@ -2408,8 +2423,9 @@ struct Solver {
         // are clamped to it (their sums are not used), so every step issues its
         // loads without a branch and they overlap the arithmetic
         const lds_float *tlast = win + (__umul24(wrows - 1, wpitch) + (rx + fu - 2 - wx0));
-        float F0 = 0.0f, gx0 = 0.0f, gy0 = 0.0f;
-        if (r0 < rb) ref_at(o, F0, gx0, gy0);
+        Raw F0 = 0;
+        float gx0 = 0.0f, gy0 = 0.0f;
+        if (r0 < rb) ref_raw(o, F0, gx0, gy0);
 #pragma unroll 1
         for (int r = r0; r < rb; r += 2) {
           const lds_float *t4 = t + 6 * wpitch, *t5 = t + 7 * wpitch;
@@ -2421,15 +2437,16 @@ struct Solver {
             a[k] = t4[k];
             b[k] = t5[k];
           }
-          float F1 = 0.0f, gx1 = 0.0f, gy1 = 0.0f;
-          if (r + 2 < rb) ref_at(o + ostep, F1, gx1, gy1);
+          Raw F1 = 0;
+          float gx1 = 0.0f, gy1 = 0.0f;
+          if (r + 2 < rb) ref_raw(o + ostep, F1, gx1, gy1);
           float vv = h0 * wyu[0];
           vv = fmaf(h1, wyu[1], vv);
           vv = fmaf(h2, wyu[2], vv);
           vv = fmaf(h3, wyu[3], vv);
           vv = fmaf(h4, wyu[4], vv);
           vv = fmaf(h5, wyu[5], vv);
-          unc_terms(u, v, gx0, gy0, vv - F0, *e - F0, pt);
+          unc_terms(u, v, gx0, gy0, vv - (float)F0, *e - (float)F0, pt);
           F0 = F1;
           gx0 = gx1;
           gy0 = gy1;
@@ -2481,46 +2498,72 @@ struct Solver {
   // the subset and the y weights to a row, and the Keys sum separates.  A lane
   // takes a column and steps down its rows; the row sums of the six window rows
   // under its pixel stay in registers and each step adds one (12 multiply-adds,
-  // 6 taps and 8 broadcast words per value instead of 42, 36 and 34 operations
-  // for the weights) -- the products and their order are those of sample(), so
-  // the values are too.  The y weights of the rows are tabled once per pass.
-  // f(r, c, value) for every pixel of this wave's rows, and (one wave) g(r1)
-  // after each kTransChunk rows, r1 the rows done; returns after the group's
-  // sync.  S <= 64: a column per lane.
-  static constexpr int kTransChunk = 12;  // a multiple of the six rows that the unrolled walk turns its sums in
-  template <class F, class C>
+  // 6 taps and 6 lane reads of y weights per value instead of 42, 36 and 34
+  // operations for the weights) -- the products and their order are those of
+  // sample(), so the values are too.  (The y weights as an LDS table read by all
+  // lanes made the LDS pipe the bound: 16 of its cycles per row and wave.)
+  // f(j, r, c, value, F, gx, gy) for every pixel of this wave's rows (j: its row
+  // in the chunk, a constant after unrolling) and, one wave only, g(r1) after each
+  // kTransChunk rows, r1 the rows done; returns after the group's sync.  REF: the
+  // reference loads that f needs (0 none, 1 F, 2 F, gx and gy).
+  // S <= 64: a column per lane; the lanes past the last column repeat it (no
+  // branch per row; f must bear the repeats).
+  static constexpr int kTransChunk = 6;  // the rows after which the unrolled walk has turned its six sums around
+  template <int REF, class F, class C>
   __device__ __forceinline__ void trans_values(const Affine &A, F &&f, C &&g) {
     const int lane = lid(), w = wid();
     const int ra = S * w / kNW, rb = S * (w + 1) / kNW;
+    const int c = min(lane, S - 1);
+    const float ox = A.p[0] + (float)(c - hw);
+    int o = (cy - hw + ra - ref.oy) * ref.w + (cx - hw + c - ref.ox);
+    // the loads run kAhead rows ahead of their use: with one row ahead every row
+    // waited for them (700 cycles a row against 290 without loads)
+    constexpr int kAhead = 3;  // divides kTransChunk
+    Raw Fr[kAhead];
+    float gxr[kAhead], gyr[kAhead];
+    int fr = ra;  // the row that o is at
+    auto fetch = [&](int k) {
+      if constexpr (REF == 1) Fr[k] = Pix<T>::raw_u(ref.pix, (unsigned)o);
+      if constexpr (REF == 2) ref_raw(o, Fr[k], gxr[k], gyr[k]);
+      o += fr + 1 < rb ? ref.w : 0;
+      ++fr;
+    };
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      Fr[k] = 0;
+      gxr[k] = gyr[k] = 0.0f;
+      if (REF > 0) fetch(k);
+    }
+    // row r0 + j with its value v
+    auto emit = [&](int j, int r, float v) {
+      const Raw F0 = Fr[j % kAhead];
+      const float gx0 = gxr[j % kAhead], gy0 = gyr[j % kAhead];
+      if (REF > 0) fetch(j % kAhead);
+      f(j, r, c, v, (float)F0, gx0, gy0);
+    };
     if constexpr (INTERP == 0) {
-      const float oxc = A.p[0] + (float)(lane - hw);
 #pragma unroll 1
       for (int r0 = ra; r0 < rb; r0 += kTransChunk) {
         const int r1 = min(r0 + kTransChunk, rb);
-        if (lane < S)
-          for (int r = r0; r < r1; ++r) f(r, lane, sample(oxc, A.p[1] + (float)(r - hw)));
+#pragma unroll
+        for (int j = 0; j < kTransChunk; ++j) {
+          if (r0 + j >= r1) break;
+          emit(j, r0 + j, sample(ox, A.p[1] + (float)(r0 + j - hw)));
+        }
         if constexpr (kIsWave) g(r1);
       }
     } else {
-#pragma unroll 1
-      for (int r = grp.rank(); r < S; r += G::kSize) {
-        const float oy = A.p[1] + (float)(r - hw);
-        const float fly = floorf(oy);
-        float wy[6];
-        keys_weights(oy - fly, wy);
-        lds_float4 *q = (lds_float4 *)(ytab + 8 * r);
-        q[0] = float4v{wy[0], wy[1], wy[2], wy[3]};
-        q[1] = float4v{wy[4], wy[5], __int_as_float(cy - def.oy + (int)fly - 2 - wy0), 0.0f};
-      }
-      grp.sync();
-      auto row_of = [&](int r) { return __builtin_amdgcn_readfirstlane(__float_as_int(ytab[8 * r + 6])); };
+      // lane r holds row r's y weights and window row
+      const float oy = A.p[1] + (float)(lane - hw);
+      const float fly = floorf(oy);
+      float wyl[6];
+      keys_weights(oy - fly, wyl);
+      const int yl = cy - def.oy + (int)fly - 2 - wy0;
+      auto wy_of = [&](int k, int r) { return __int_as_float(lane_value(__float_as_int(wyl[k]), r)); };
       // consecutive rows of the subset lie on consecutive window rows unless
       // v + dy rounds across an integer
-      const int row0 = row_of(0);
-      const bool steady =
-          __ballot(lane < S && __float_as_int(ytab[8 * (lane < S ? lane : 0) + 6]) != row0 + lane) == 0ull;
-      const int c = min(lane, S - 1);  // the lanes past the last column repeat it
-      const float ox = A.p[0] + (float)(c - hw);
+      const int row0 = lane_value(yl, 0);
+      const bool steady = __ballot(lane < S && yl != row0 + lane) == 0ull;
       const float flx = floorf(ox);
       float wx[6];
       keys_weights(ox - flx, wx);
@@ -2546,28 +2589,29 @@ struct Solver {
 #pragma unroll 1
         for (int r0 = ra; r0 < rb; r0 += kTransChunk) {
           const int r1 = min(r0 + kTransChunk, rb);
-#pragma unroll 1
-          for (int r = r0; r < r1; r += 6) {
+          // row r0 + j, its sums at h[j % 6] ...; the next row's taps first (past
+          // the last row: words of the slot, not used)
+          auto row = [&](int j) {
+            t += wpitch;
+            float b[6];
 #pragma unroll
-            for (int j = 0; j < 6; ++j) {
-              if (r + j >= r1) break;
-              // the next row's taps first (past the last row: words of the slot, not used)
-              t += wpitch;
-              float b[6];
+            for (int k = 0; k < 6; ++k) b[k] = t[k];
+            h[(j + 5) % 6] = rowsum(a);
+            float v = h[j % 6] * wy_of(0, r0 + j);
 #pragma unroll
-              for (int k = 0; k < 6; ++k) b[k] = t[k];
-              const lds_float4 *q = (const lds_float4 *)(ytab + 8 * (r + j));
-              const float4v w0 = q[0], w1 = q[1];
-              h[(j + 5) % 6] = rowsum(a);
-              float v = h[j] * w0.x;
-              v = fmaf(h[(j + 1) % 6], w0.y, v);
-              v = fmaf(h[(j + 2) % 6], w0.z, v);
-              v = fmaf(h[(j + 3) % 6], w0.w, v);
-              v = fmaf(h[(j + 4) % 6], w1.x, v);
-              v = fmaf(h[(j + 5) % 6], w1.y, v);
-              if (lane < S) f(r + j, lane, v);
+            for (int k = 1; k < 6; ++k) v = fmaf(h[(j + k) % 6], wy_of(k, r0 + j), v);
+            emit(j, r0 + j, v);
 #pragma unroll
-              for (int k = 0; k < 6; ++k) a[k] = b[k];
+            for (int k = 0; k < 6; ++k) a[k] = b[k];
+          };
+          if (r1 - r0 == kTransChunk) {
+#pragma unroll
+            for (int j = 0; j < kTransChunk; ++j) row(j);
+          } else {
+#pragma unroll
+            for (int j = 0; j < kTransChunk; ++j) {
+              if (r0 + j >= r1) break;
+              row(j);
             }
           }
           if constexpr (kIsWave) g(r1);
@@ -2576,13 +2620,14 @@ struct Solver {
 #pragma unroll 1
         for (int r0 = ra; r0 < rb; r0 += kTransChunk) {
           const int r1 = min(r0 + kTransChunk, rb);
-#pragma unroll 1
-          for (int r = r0; r < r1; ++r) {
-            const lds_float4 *q = (const lds_float4 *)(ytab + 8 * r);
-            const float4v w0 = q[0], w1 = q[1];
-            const float wy[6] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y};
-            const float v = keys_sum(base + __umul24(row_of(r), wpitch), wpitch, wx, wy);
-            if (lane < S) f(r, lane, v);
+#pragma unroll
+          for (int j = 0; j < kTransChunk; ++j) {
+            const int r = r0 + j;
+            if (r >= r1) break;
+            float wy[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) wy[k] = wy_of(k, r);
+            emit(j, r, keys_sum(base + __umul24(lane_value(yl, r), wpitch), wpitch, wx, wy));
           }
           if constexpr (kIsWave) g(r1);
         }
@@ -2705,47 +2750,37 @@ struct Solver {
   __device__ __forceinline__ void accumulate_trans(const Affine &A, float shift) {
     const int lane = lid();
     if constexpr (kIsWave) {
-      // gtab holds kTransChunk rows: after each of them the lanes add their
-      // pixels of those rows (pixels lane, lane + 64, ... of the subset)
+      // gtab holds (gmf, gx, gy, G) of kTransChunk rows: after each of them the
+      // lanes add their pixels of those rows (pixels lane, lane + 64, ... of the
+      // subset).  Loading the reference here instead, in that order, costs a mask
+      // and a column wrap per step, and the kernel is bound by instruction issue.
       float pa[3] = {0.0f, 0.0f, 0.0f};
-      const float inv = 1.0f / (float)S;
-      const int drow = (int)(((float)kWave + 0.5f) * inv), dcol = kWave - drow * S;
-      const int row = (int)(((float)lane + 0.5f) * inv);
-      int i = lane, col = lane - row * S, done = 0;
-      int o = (cy - hw + row - ref.oy) * ref.w + (cx - hw + col - ref.ox);
-      const int ostep = drow * ref.w + dcol, owrap = ref.w - S;
-      trans_values(
-          A, [&](int r, int c, float v) { gtab[(r - done) * S + c] = v; },
+      int i = lane, done = 0;  // the lane's next pixel; rows done
+      lds_float4 *const tab = (lds_float4 *)gtab;
+      lds_float4 *put = tab + min(lane, S - 1);
+      trans_values<2>(
+          A,
+          [&](int, int, int, float v, float F, float gx, float gy) {
+            *put = float4v{(v - shift) - (F - meanF), gx, gy, v};
+            put += S;
+          },
           [&](int r1) {
             grp.sync();
+            const lds_float4 *q = tab + (i - done * S);
             const int end = r1 * S;
-            const lds_float *gt = gtab - done * S;
-            float F = 0.0f, gx = 0.0f, gy = 0.0f, Gv = 0.0f;
-            if (i < end) {
-              ref_at(o, F, gx, gy);
-              Gv = gt[i];
-            }
-#pragma unroll 1
-            while (i < end) {
-              // the next pixel's loads first: they are in flight during the sums
-              const float F0 = F, gx0 = gx, gy0 = gy, G0 = Gv;
-              i += kWave;
-              o += ostep;
-              col += dcol;
-              if (col >= S) {
-                col -= S;
-                o += owrap;
-              }
+            constexpr int kPer = (kTransChunk * 64) / kWave + 1;
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) {
               if (i < end) {
-                ref_at(o, F, gx, gy);
-                Gv = gt[i];
+                const float4v t = q[k * kWave];
+                pa[0] = fmaf(t.x, t.y, pa[0]);
+                pa[1] = fmaf(t.x, t.z, pa[1]);
+                pa[2] += t.w;
+                i += kWave;
               }
-              const float gmf = (G0 - shift) - (F0 - meanF);
-              pa[0] = fmaf(gmf, gx0, pa[0]);
-              pa[1] = fmaf(gmf, gy0, pa[1]);
-              pa[2] += G0;
             }
             done = r1;
+            put = tab + min(lane, S - 1);
             grp.sync();
           });
 #pragma unroll
@@ -2754,7 +2789,8 @@ struct Solver {
         if (lane == 0) pers[kLeanPass + k] = t;
       }
     } else {
-      trans_values(A, [&](int r, int c, float v) { gtab[r * S + c] = v; }, [](int) {});
+      trans_values<0>(
+          A, [&](int, int r, int c, float v, float, float, float) { gtab[r * S + c] = v; }, [](int) {});
       const int w = wid();
       if (w < 3) {
         float p = 0.0f;
@@ -2823,14 +2859,16 @@ struct Solver {
   // reference sums are per-subset constants).
   __device__ __forceinline__ void gamma_sums_trans(const Affine &A, double (&acc)[6]) {
     double t[3] = {0.0, 0.0, 0.0};
-    const int o0 = (cy - hw - ref.oy) * ref.w + (cx - hw - ref.ox);
-    trans_values(A, [&](int r, int c, float v) {
-      const double d = v;
-      const double rv = kIsWave ? Pix<T>::at_u(ref.pix, (unsigned)(o0 + r * ref.w + c)) : rtab[r * S + c];
-      t[0] += d;
-      t[1] = fma(d, d, t[1]);
-      t[2] = fma(d, rv, t[2]);
-    }, [](int) {});
+    trans_values<kIsWave ? 1 : 0>(
+        A,
+        [&](int, int r, int c, float v, float F, float, float) {
+          const double d = v, rv = kIsWave ? F : rtab[r * S + c];
+          t[0] += d;
+          t[1] = fma(d, d, t[1]);
+          t[2] = fma(d, rv, t[2]);
+        },
+        [](int) {});
+    if (lid() >= S) t[0] = t[1] = t[2] = 0.0;  // the repeats of the last column
     grp.sum(t);
     acc[1] = t[0];
     acc[2] = t[1];
@@ -4689,7 +4727,11 @@ __host__ __device__ inline int trans_window_floats(int side, int cap) {
 #define DICE_TRANS_WPE 3
 #endif
 // BATCHED translation-only Gauss-Newton pass: one wave per subset (and per
-// workgroup), Solver::run_lean<true>.  A wave's LDS: the slot, then gtab and ytab.
+// workgroup), Solver::run_lean<true>.  A wave's LDS: the window, the per-subset
+// constants, then gtab.  27,264 subsets of 35 x 35 (u16): 1.13 ms in the general
+// kernel, 0.59 ms here; 11 k vector instructions per subset (24 k there), issued
+// in 73 % of the quad-cycles with three waves per SIMD.  More waves spill, and
+// fewer hide less: four per SIMD (35 spilled registers) 0.66 ms, two 0.93 ms.
 template <typename T, int INTERP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_WPE))) void correlate_trans_kernel(
     KParams kp, DImage ref, DImage def, DSubsets ss, double *fields, PassArgs pa, int slot) {
@@ -4702,8 +4744,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_W
   const int side = 2 * (ss.S / 2) + 1;
   s.win_phys = trans_window_floats(side, s.win_cap);
   s.pers = (lds_double *)(base + s.win_phys);
-  s.ytab = base + s.win_phys + kPersistFloats;
-  s.gtab = s.ytab + 8 * side;
+  s.gtab = base + s.win_phys + kPersistFloats;
   const int total = items.total(ss.n);
   if ((int)blockIdx.x >= total) return;  // as in correlate_batched_kernel
   int range = (int)(blockIdx.x % kWorkRanges);
@@ -4724,7 +4765,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_W
   }
 }
 
-// The same two passes with few subsets: four waves per subset.
+// The same two passes with at most kCrewMaxSubsets subsets: four waves per
+// subset.  One wave each leaves most SIMDs idle and the frame takes a subset's
+// whole latency: 49 subsets of 27 x 27, 87 us in the general kernel, 35 here.
+// With 2,116 subsets of 31 x 31 every SIMD has two waves of its own and the lean
+// kernel is the faster one (129 against 168 us with four waves per subset).
 template <typename T, int INTERP, bool TRANS>
 __global__ __launch_bounds__(256) void correlate_crew_kernel(KParams kp, DImage ref, DImage def, DSubsets ss,
                                                              double *fields, PassArgs pa, int slot) {
@@ -4740,8 +4785,7 @@ __global__ __launch_bounds__(256) void correlate_crew_kernel(KParams kp, DImage 
   Solver<T, CrewGroup, INTERP, false> s(kp, ref, def, g, base, slot - kPersistFloats);
   s.pers = (lds_double *)(base + slot - kPersistFloats);
   const int side = 2 * (ss.S / 2) + 1;
-  s.ytab = base + slot;
-  s.gtab = s.ytab + 8 * side;
+  s.gtab = base + slot;
   s.rtab = s.gtab + side * side;
   BlockClaims claims(pa.counter, total);
 #pragma unroll 1
@@ -4767,12 +4811,12 @@ __global__ __launch_bounds__(256) void correlate_crew_kernel(KParams kp, DImage 
 }
 
 // LDS floats of a wave of correlate_trans_kernel and of a crew: the slot (the
-// window and the per-subset constants), ytab, gtab, and a crew's reference tables.
+// window and the per-subset constants), gtab, and a crew's reference tables.
 inline int trans_lds_floats(int S, int slot, bool crew) {
   const int side = 2 * (S / 2) + 1;
-  if (crew) return slot + 8 * side + 4 * side * side;
+  if (crew) return slot + 4 * side * side;
   return trans_window_floats(side, slot - kPersistFloats) + kPersistFloats +
-         (8 + Solver<float, TightWave, 2, false>::kTransChunk) * side;
+         4 * Solver<float, TightWave, 2, false>::kTransChunk * side;
 }
 
 template <typename T, int INTERP, bool TRANS>
