@@ -4045,6 +4045,7 @@ struct LaneGroup {
 // table, the vertices' objective values and the initial point live in the
 // row's LDS (nm, kNmFloats floats), written by the row's lane 0.
 constexpr int kNmFloats = 56;  // pts 7 x 6, gv 7, init 6, one spare
+constexpr int kNmConst = 8;    // after them (simplex_groups_kernel): the reference's part of the objective
 template <typename T, int INTERP, bool SQUARE>
 struct LaneSimplex {
   enum : int { kVertex = 0, kReflect = 1, kExpand = 2, kContract = 3, kShrink = 4 };
@@ -4393,9 +4394,27 @@ __global__ __launch_bounds__(256) DICE_LANE_BOUNDS void simplex_groups_kernel(KP
   const int lane = (int)(threadIdx.x % kWave), l = lane & (W - 1);
   // the row's slot: the window, then the vertex table
   lds_float *const win = (lds_float *)lds + (size_t)(threadIdx.x / W) * slot;
-  const int cap = slot - kNmFloats;
+  const int cap = slot - kNmFloats - kNmConst;
   LaneSimplex<T, INTERP, SQUARE> m(kp, ref, def, win + cap, l == 0);
   auto &s = m.s;
+  // square subsets whose pixels are all kept (below): the reference mean, the
+  // norm of its deviations, and whether it is flat
+  lds_double *const rc = (lds_double *)(win + cap + kNmFloats);
+  // their pixels' offsets from the centre are those of the lane
+  // (two pixels to a word, each offset + 16 in a byte)
+  unsigned dk[SQUARE ? (KPER + 1) / 2 : 1];
+  const int side = 2 * (ss.S / 2) + 1, npix = side * side;
+  if constexpr (SQUARE) {
+#pragma unroll
+    for (int k = 0; k < (KPER + 1) / 2; ++k) dk[k] = 0;
+#pragma unroll
+    for (int k = 0; k < KPER; ++k) {
+      const int j = l + W * k, i = j < npix ? j : npix / 2;
+      const int r = (int)(((float)i + 0.5f) / (float)side);  // exact: i < 2^8, S <= 16
+      dk[k / 2] |= (unsigned)((i - r * side - ss.S / 2 + 16) | ((r - ss.S / 2 + 16) << 8)) << (16 * (k & 1));
+    }
+  }
+
   constexpr int kPer = KPER;
   constexpr int lead = INTERP == 0 ? 0 : 2, trail = INTERP == 0 ? 1 : 3;
   float rv[kPer];  // reference values of the lane's pixels
@@ -4420,6 +4439,25 @@ __global__ __launch_bounds__(256) DICE_LANE_BOUNDS void simplex_groups_kernel(KP
           m.start(ss, gid, fields);
           s.template small_walk<W, KPER>(l, [&](int q, int x, int y, bool) { rv[q] = s.ref_value(x - ref.ox, y - ref.oy); });
           wr = 0;
+          if constexpr (SQUARE) {
+            // sr and srr of small_partial, once per subset, and gamma_of's terms of them
+            double sr = 0.0, srr = 0.0;
+#pragma unroll
+            for (int q = 0; q < KPER; ++q)
+              if (l + W * q < s.n) {
+                const double r = rv[q];
+                sr += r;
+                srr = fma(r, r, srr);
+              }
+            sr = row_sum<W>(sr);
+            srr = row_sum<W>(srr);
+            const double cnt = (double)s.n, mr = sr / cnt, dev = fmax(fma(-(cnt * mr), mr, srr), 0.0);
+            if (l == 0) {
+              rc[0] = mr;
+              rc[1] = sqrt(dev);
+              rc[2] = dev <= 1e-13 * srr ? 1.0 : 0.0;
+            }
+          }
         }
         need = false;
       }
@@ -4429,12 +4467,27 @@ __global__ __launch_bounds__(256) DICE_LANE_BOUNDS void simplex_groups_kernel(KP
       m.A.prepare();
       // the deformed pixels under this point's footprint (as Solver::stage_affine)
       float lo_x, hi_x, lo_y, hi_y;
-      s.warp_bounds(m.A, lo_x, hi_x, lo_y, hi_y);
+      const bool centred = SQUARE && s.bx0 == s.cx - s.hw && s.by0 == s.cy - s.hw;  // no clamped pixel
+      if (centred) {
+        // the corners are +-hw: disp's products at opposite ones differ in sign only
+        const float h = (float)s.hw;
+        const float x = m.A.a11 * h, y = m.A.a21 * h;
+        const float ex = fmaxf(fabsf(fmaf(m.A.a12, h, x)), fabsf(fmaf(m.A.a12, h, -x)));
+        const float ey = fmaxf(fabsf(fmaf(m.A.a22, h, y)), fabsf(fmaf(m.A.a22, h, -y)));
+        lo_x = m.A.p[0] - ex;
+        hi_x = m.A.p[0] + ex;
+        lo_y = m.A.p[1] - ey;
+        hi_y = m.A.p[1] + ey;
+      } else {
+        s.warp_bounds(m.A, lo_x, hi_x, lo_y, hi_y);
+      }
       const float mg = 1e-3f;
-      const int nx0 = max(s.cx - def.ox + (int)floorf(lo_x - mg) - lead, 0);
-      const int nx1 = min(s.cx - def.ox + (int)floorf(hi_x + mg) + trail, def.w - 1);
-      const int ny0 = max(s.cy - def.oy + (int)floorf(lo_y - mg) - lead, 0);
-      const int ny1 = min(s.cy - def.oy + (int)floorf(hi_y + mg) + trail, def.h - 1);
+      const int fx0 = s.cx - def.ox + (int)floorf(lo_x - mg), fx1 = s.cx - def.ox + (int)floorf(hi_x + mg);
+      const int fy0 = s.cy - def.oy + (int)floorf(lo_y - mg), fy1 = s.cy - def.oy + (int)floorf(hi_y + mg);
+      const int nx0 = max(fx0 - lead, 0), nx1 = min(fx1 + trail, def.w - 1);
+      const int ny0 = max(fy0 - lead, 0), ny1 = min(fy1 + trail, def.h - 1);
+      // every rounded position passes kept()'s guard
+      const bool every = centred && s.mw == 0 && fx0 >= 5 && fx1 <= def.w - 6 && fy0 >= 5 && fy1 <= def.h - 6;
       const bool inwin = wr > 0 && nx0 >= wx0 && nx1 < wx0 + wp && ny0 >= wy0 && ny1 < wy0 + wr;
       bool fits = true;
       if (!inwin && nx1 >= nx0 && ny1 >= ny0) {
@@ -4483,13 +4536,71 @@ __global__ __launch_bounds__(256) DICE_LANE_BOUNDS void simplex_groups_kernel(KP
         keys_weights(ty, wy);
         return keys_sum(win + ((iy - 2) * wp + ix - 2), wp, wx, wy);
       };
-      double acc[6] = {0, 0, 0, 0, 0, 0};
-      s.template small_partial<W, KPER>(m.A, l, acc, smp, [&](int, int, int k) { return rv[k]; });
+      float g;
+      if (SQUARE && __ballot(!every || glob) == 0ull) {
+        // every row of the wave in the common case -- a square subset, all pixels
+        // kept, the window in LDS: small_partial's sums of d, and gamma_of with
+        // the reference's part from rc.  The tests of a pixel and the sums of r
+        // were more than half of its instructions: 188,468 subsets of 9 x 9
+        // (bilinear, u16) 11.7 -> 8.6 ms with the epilogue, 8.3 -> 5.7 G vector
+        // instructions.  The kernel is bound by their issue.
+        double sd = 0.0, sdd = 0.0, sdr = 0.0;
+        auto pixel = [&](int k) {
+          float ox, oy;
+          // (opaque: the conversions of the loop's constants stay inside it, or they
+          // would hold a register pair per pixel)
+          const unsigned b = (unsigned)opaque_lane((int)dk[k / 2]) >> (16 * (k & 1));
+          const float r = __int_as_float(opaque_lane(__float_as_int(rv[k])));
+          m.A.disp((float)(b & 255u) - 16.0f, (float)((b >> 8) & 255u) - 16.0f, ox, oy);
+          const float flx = floorf(ox), fly = floorf(oy);
+          const float tx = ox - flx, ty = oy - fly;
+          const int at = __mul24(s.cy - def.oy - wy0 - lead + (int)fly, wp) + (s.cx - def.ox - wx0 - lead + (int)flx);
+          float v;
+          if (INTERP == 0) {
+            v = bilinear_sum(win + at, wp, tx, ty);
+          } else {
+            float wx[6], wy[6];
+            keys_weights(tx, wx);
+            keys_weights(ty, wy);
+            v = keys_sum(win + at, wp, wx, wy);
+          }
+          // (a lane without a pixel k took the centre's: it adds zeros)
+          const double d = W * (k + 1) <= npix || l + W * k < npix ? v : 0.0f;
+          sd += d;
+          sdd = fma(d, d, sdd);
+          sdr = fma(d, (double)r, sdr);
+          if (INTERP != 0 || (k & 1)) __builtin_amdgcn_sched_barrier(0);  // few pixels' taps in flight: registers
+        };
 #pragma unroll
-      for (int k = 0; k < 6; ++k) acc[k] = row_sum<W>(acc[k]);
-      int active;
-      float contrast;
-      const float g = s.gamma_of(acc, active, contrast);
+        for (int k = 0; k < KPER; ++k)
+          if (W * k < npix) pixel(k);
+        sd = row_sum<W>(sd);
+        sdd = row_sum<W>(sdd);
+        sdr = row_sum<W>(sdr);
+        const double cnt = (double)s.n, md = sd / cnt;
+        const double dd = fmax(fma(-(cnt * md), md, sdd), 0.0);
+        const double dr = fma(-(cnt * md), rc[0], sdr);
+        if (dd <= 1e-13 * sdd || rc[2] != 0.0) {
+          g = -1.0f;
+        } else {
+          double gam = fma(-2.0, dr / (sqrt(dd) * rc[1]), 2.0);
+          if (gam < 0.0) gam = 0.0;
+          g = (float)gam;
+          if (kp.normalize_gamma) g = (float)((double)g / cnt);
+        }
+      } else {
+        double acc[6] = {0, 0, 0, 0, 0, 0};
+        if constexpr (SQUARE)  // rolled: a small body, with the reference from the image
+          s.template small_partial<W, KPER, false>(
+              m.A, l, acc, smp, [&](int x, int y, int) { return s.ref_value(x - ref.ox, y - ref.oy); });
+        else
+          s.template small_partial<W, KPER>(m.A, l, acc, smp, [&](int, int, int k) { return rv[k]; });
+#pragma unroll
+        for (int k = 0; k < 6; ++k) acc[k] = row_sum<W>(acc[k]);
+        int active;
+        float contrast;
+        g = s.gamma_of(acc, active, contrast);
+      }
       int iters = 0;
       const int st = m.step(g, iters);
       if (st >= 0) {
@@ -4507,12 +4618,12 @@ __global__ __launch_bounds__(256) DICE_LANE_BOUNDS void simplex_groups_kernel(KP
 }
 
 // LDS floats of one row's slot in simplex_groups_kernel, rows of W lanes: 16
-// rows of 16 lanes (600 floats each) or 32 rows of 8 lanes (312 floats: a 16 x 16
-// window and the vertex table) per 256-thread workgroup; four workgroups per
-// CU: 150 KB or 156 KB.
+// rows of 16 lanes (608 floats each) or 32 rows of 8 lanes (320 floats: a 16 x 16
+// window, the vertex table and the reference's constants) per 256-thread
+// workgroup; four workgroups per CU: 152 KB or 160 KB.
 template <int W>
 constexpr int group_slot_floats() {
-  return W == 8 ? 312 : 600;
+  return kNmConst + (W == 8 ? 312 : 600);
 }
 
 template <typename T, int INTERP, bool SQUARE, int W, int KPER>
