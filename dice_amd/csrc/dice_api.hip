@@ -884,9 +884,9 @@ int dice_hip_pass_counts(dice_hip_context *ctx, int *counts) {
 }
 
 // VSG strains: the subsets binned on the device into a uniform grid (cells of
-// side max(r, 1) px for radius windows, about k subsets each for k-nearest):
+// a quarter of the radius for radius windows, about k subsets each for k-nearest):
 // the bounds of the centres (read back, 40 B, to size the grid), a cell key per
-// subset, a stable radix sort of (cell, id), each cell's range and one packed
+// subset, a list ordered by (cell, id), each cell's range and one packed
 // record per subset, then one thread per subset on the context stream.  The
 // bounds read-back and the final wait make this call synchronous.
 static int vsg_enqueue(dice_hip_context *ctx, int window_size, double *d_fields, double *d_vsg) {
@@ -908,27 +908,31 @@ static int vsg_enqueue(dice_hip_context *ctx, int window_size, double *d_fields,
   dice_hip::VsgGrid g{};
   g.x0 = x0;
   g.y0 = y0;
-  // radius windows: cells of side >= r, so that every neighbour lies in the 3 x 3 cells around a
-  // subset; k-nearest: cells holding about k subsets; at most 4000 cells along a side
-  const double side = knn ? std::sqrt((x1 - x0 + 1.0) * (y1 - y0 + 1.0) * knn / n) : (double)radius;
+  g.slack = 0.05 + 0x1p-21 * std::max({std::fabs(x0), std::fabs(x1), std::fabs(y0), std::fabs(y1)});
+  // radius windows: cells of side >= r / kVsgRings, so that every neighbour lies in the kVsgRings rings
+  // of cells around a subset (with the rounding of the float centres and distances), and of about one subset
+  // at least; k-nearest: cells holding about k subsets; at most 4000 cells along a side
+  const double side = knn ? std::sqrt((x1 - x0 + 1.0) * (y1 - y0 + 1.0) * knn / n)
+                          : std::max(((double)radius + 4.0 * g.slack) / dice_hip::kVsgRings,
+                                     std::sqrt((x1 - x0 + 1.0) * (y1 - y0 + 1.0) / n));
   g.cell = std::max({side, 1.0, (x1 - x0) / 4000.0, (y1 - y0) / 4000.0});
   g.ncx = (int)std::floor((x1 - x0) / g.cell) + 1;
   g.ncy = (int)std::floor((y1 - y0) / g.cell) + 1;
   const long long ncells = (long long)g.ncx * g.ncy;
-  size_t temp_bytes = 0;
-  HIP_TRY(ctx, dice_hip::vsg_grid_temp_bytes(n, ncells, &temp_bytes), "VSG grid scratch size");
   const size_t nb = (size_t)n * sizeof(int);
-  HIP_TRY(ctx, ctx->vsg_cells.ensure(2 * (size_t)ncells * sizeof(int)), "hipMalloc VSG grid");
+  const size_t groups = ((size_t)ncells + 1023) / 1024;
+  HIP_TRY(ctx, ctx->vsg_cells.ensure((2 * (size_t)ncells + 1 + groups) * sizeof(int)), "hipMalloc VSG grid");
   HIP_TRY(ctx, ctx->vsg_ids.ensure(nb), "hipMalloc VSG grid");
   HIP_TRY(ctx, ctx->vsg_ids2.ensure(nb), "hipMalloc VSG grid");
   HIP_TRY(ctx, ctx->vsg_keys.ensure(nb), "hipMalloc VSG grid");
   HIP_TRY(ctx, ctx->vsg_keys2.ensure(nb), "hipMalloc VSG grid");
+  HIP_TRY(ctx, ctx->vsg_temp.ensure(nb), "hipMalloc VSG grid");
   HIP_TRY(ctx, ctx->vsg_rec.ensure((size_t)n * sizeof(float4)), "hipMalloc VSG grid");
-  HIP_TRY(ctx, ctx->vsg_temp.ensure(temp_bytes), "hipMalloc VSG grid");
-  const dice_hip::VsgWork w{ctx->vsg_keys.as<int>(), ctx->vsg_ids.as<int>(), ctx->vsg_keys2.as<int>(),
-                            ctx->vsg_ids2.as<int>(),  ctx->vsg_cells.as<int>(),   ctx->vsg_rec.as<float4>(),
-                            ctx->vsg_temp.p,          temp_bytes};
-  HIP_TRY(ctx, dice_hip::launch_vsg_grid(d_fields, n, g, w, ctx->stream), "VSG grid");
+  int *const count = ctx->vsg_cells.as<int>();
+  const dice_hip::VsgWork w{ctx->vsg_keys2.as<int>(), ctx->vsg_temp.as<int>(), ctx->vsg_ids2.as<int>(),
+                            ctx->vsg_keys.as<int>(),  ctx->vsg_ids.as<int>(),  ctx->vsg_rec.as<float4>(),
+                            count,                    count + ncells,          count + 2 * ncells + 1};
+  HIP_TRY(ctx, dice_hip::launch_vsg_grid(d_fields, n, knn == 0, g, w, ctx->stream), "VSG grid");
   HIP_TRY(ctx, dice_hip::launch_vsg_strain(g, radius, knn, d_fields, d_vsg, n, ctx->stream), "VSG strain kernel");
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream), "VSG strain");
   return DICE_HIP_OK;

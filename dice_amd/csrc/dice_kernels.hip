@@ -4,8 +4,6 @@
 
 #include <algorithm>
 
-#include <rocprim/device/device_radix_sort.hpp>
-
 namespace dice_hip {
 
 typedef hipError_t (*PassLauncher)(int, int, int, const Launch &, const KParams &, const DImage &, const DImage &,
@@ -322,69 +320,126 @@ __global__ __launch_bounds__(256) void vsg_bounds_final_kernel(const double *par
   vsg_bounds_fold(red, x0, y0, x1, y1, bad, out);
 }
 
-// Cell of every subset centre (the same arithmetic as vsg_strain_kernel's own
-// cell) and its id, the keys of the sort.
-__global__ void vsg_cells_kernel(const double *fields, int n, VsgGrid g, int *keys, int *ids) {
+// The cell-ordered list by counting: every subset's cell and its turn to arrive
+// there (an atomic per subset), the cells' first entries by a scan of the counts,
+// the ids at those places, and last each entry's rank by id among its cell's, so
+// that ids ascend within a cell whatever the order of arrival.  That rank reads
+// the entries of one cell per entry, never more than the strain's own scan does
+// after it.  Five launches of a few us: 155,236 subsets in 18,225 cells 27 us, a
+// library radix sort of (cell, id) and the cells' ranges from it 72 us.
+//
+// Cell of subset i (the same arithmetic as vsg_subset's own cell).
+__global__ void vsg_cells_kernel(const double *fields, int n, VsgGrid g, int *count, int *cells, int *turn) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double xi = fields[(size_t)F_COORD_X * n + i], yi = fields[(size_t)F_COORD_Y * n + i];
   const int ci = min(max((int)floor((xi - g.x0) / g.cell), 0), g.ncx - 1);
   const int cj = min(max((int)floor((yi - g.y0) / g.cell), 0), g.ncy - 1);
-  keys[i] = cj * g.ncx + ci;
-  ids[i] = i;
+  const int c = cj * g.ncx + ci;
+  cells[i] = c;
+  turn[i] = atomicAdd(count + c, 1);
 }
 
-// Cell ranges from the sorted keys: entry k opens its cell when the previous
-// key differs and closes it when the next one does (cells without entries keep
-// the empty range [0, 0) of the zero fill).
-__global__ void vsg_ranges_kernel(const int *keys, int n, int *begin, int *end) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int c = keys[k];
-  if (k == 0 || keys[k - 1] != c) begin[c] = k;
-  if (k == n - 1 || keys[k + 1] != c) end[c] = k + 1;
+// Exclusive scan of the counts in two launches: the sum of each group of
+// kVsgScan cells, then each workgroup adds up the groups before its own and
+// scans its cells.  start[ncells] = n.
+constexpr int kVsgScan = 1024;
+__device__ int vsg_block_sum(int v, int *red) {  // over 256 threads; every thread gets it
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
+  __syncthreads();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+__global__ __launch_bounds__(256) void vsg_sums_kernel(const int *count, int ncells, int *sums) {
+  __shared__ int red[4];
+  int v = 0;
+  for (int t = 0; t < kVsgScan / 256; ++t) {
+    const int c = blockIdx.x * kVsgScan + t * 256 + threadIdx.x;
+    if (c < ncells) v += count[c];
+  }
+  v = vsg_block_sum(v, red);
+  if (threadIdx.x == 0) sums[blockIdx.x] = v;
+}
+__global__ __launch_bounds__(256) void vsg_starts_kernel(const int *count, int ncells, int n, const int *sums,
+                                                         int *start) {
+  __shared__ int red[4];
+  __shared__ int scan[256];
+  int before = 0;
+  for (int t = threadIdx.x; t < (int)blockIdx.x; t += 256) before += sums[t];
+  before = vsg_block_sum(before, red);
+  // four consecutive cells per thread
+  const int c0 = blockIdx.x * kVsgScan + threadIdx.x * 4;
+  int v[4], own = 0;
+  for (int k = 0; k < 4; ++k) {
+    v[k] = c0 + k < ncells ? count[c0 + k] : 0;
+    own += v[k];
+  }
+  scan[threadIdx.x] = own;
+  __syncthreads();
+  for (int o = 1; o < 256; o <<= 1) {
+    const int add = (int)threadIdx.x >= o ? scan[threadIdx.x - o] : 0;
+    __syncthreads();
+    scan[threadIdx.x] += add;
+    __syncthreads();
+  }
+  int at = before + scan[threadIdx.x] - own;
+  for (int k = 0; k < 4; ++k) {
+    if (c0 + k < ncells) start[c0 + k] = at;
+    at += v[k];
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) start[ncells] = n;
+}
+__global__ void vsg_place_kernel(const int *cells, const int *turn, const int *start, int n, int *arrived) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) arrived[start[cells[i]] + turn[i]] = i;
 }
 
-// Entry k of the cell-ordered list: the centre and displacement of subset
-// ids[k] as float (the precision the strain uses), and ids[k] replaced by ~id
-// when the subset failed (SIGMA < 0), so that the neighbour loop reads one
-// 16-byte record and one word per candidate.
-__global__ void vsg_pack_kernel(const double *fields, int n, int *ids, float4 *rec) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int j = ids[k];
-  auto F = [&](int s) { return fields[(size_t)s * n + j]; };
-  rec[k] = make_float4((float)F(F_COORD_X), (float)F(F_COORD_Y), (float)F(F_DISP_X), (float)F(F_DISP_Y));
-  if (!(F(F_SIGMA) >= 0.0)) ids[k] = ~j;
+// Entry of subset i in the cell-ordered list: its cell, its id, ~id when it
+// failed (SIGMA < 0), and its centre and displacement as float (the precision
+// the strain uses).  hide: the centre of a failed subset as NaN, which fails
+// every distance test, so that a radius scan reads one 16-byte record per
+// candidate and nothing else.
+__global__ void vsg_pack_kernel(const double *fields, const int *cells, const int *start, const int *arrived, int n,
+                                int hide, int *keys, int *ids, float4 *rec) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int c = cells[i];
+  const int lo = start[c], hi = start[c + 1];
+  int k = lo;
+  for (int t = lo; t < hi; ++t) k += arrived[t] < i ? 1 : 0;
+  auto F = [&](int s) { return fields[(size_t)s * n + i]; };
+  const bool failed = !(F(F_SIGMA) >= 0.0);
+  const float x = failed && hide ? __int_as_float(0x7fc00000) : (float)F(F_COORD_X);
+  rec[k] = make_float4(x, (float)F(F_COORD_Y), (float)F(F_DISP_X), (float)F(F_DISP_Y));
+  keys[k] = c;
+  ids[k] = failed ? ~i : i;
 }
 
-// One subset per thread (see launch_vsg_strain).
 // Candidate records of the radius scan: straight from the cell-ordered list,
-// or from a workgroup's LDS copy of the three cell-row ranges it needs.
+// or from a workgroup's LDS copy of the ranges it needs, one per cell row.
+constexpr int kVsgMaxRows = 2 * kVsgRings + 1;
 struct VsgGlobalReader {
   const float4 *rec;
-  const int *ids;
-  __device__ float4 at(int, int k) const { return rec[k]; }
-  __device__ int id(int, int k) const { return ids[k]; }
+  __device__ const float4 *row(int) const { return rec; }
 };
 struct VsgTileReader {
   const float4 *rec;  // LDS
-  const int *ids;     // LDS
+  const int *shift;   // LDS: where entry 0 would be, per row
   int row0;           // cell row of range 0
-  int glo[3], loff[3];
-  __device__ int slot(int cy, int k) const {
-    const int r = cy - row0;
-    return loff[r] + (k - glo[r]);
-  }
-  __device__ float4 at(int cy, int k) const { return rec[slot(cy, k)]; }
-  __device__ int id(int cy, int k) const { return ids[slot(cy, k)]; }
+  __device__ const float4 *row(int cy) const { return rec + shift[cy - row0]; }
 };
 
 // Strain of subset i (see launch_vsg_strain); radius candidates through R.
 // L lanes of one wave per subset (L = 1, 2, 4, ...; lane `part` of them): the
-// radius scan deals the candidates of each cell out round-robin and the lanes'
-// sums are folded by butterfly shuffles; part 0 finishes.  Every lane of a
-// group must reach the fold.
+// radius scan deals the cell rows out round-robin and the lanes' sums are folded
+// by butterfly shuffles; part 0 finishes.  Every lane of a group must reach the
+// fold.  The candidates of a cell row are the cells within the circle's extent
+// there (plus g.slack for the rounding of the float distances): with cells of
+// a quarter of the radius three in four lie in the circle, against one in three
+// of the 3 x 3 cells of the radius.  The kernel is bound by the 11 FP64 sums per
+// neighbour and the LDS reads; 155,236 subsets at a step of 5 px, a window of
+// 121 px (460 neighbours each): 236 us with cells of the radius, 147 us with these.
 template <int L, class Reader>
 __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fields, double *vsg, int n, int i,
                            int part, const Reader &R) {
@@ -392,14 +447,14 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
   const double xi = F(F_COORD_X, i), yi = F(F_COORD_Y, i);
   const float xf = (float)xi, yf = (float)yi;
   const float r2 = radius * radius + 1.0e-5f;  // the reference's rad^2 + tiny in scalar_t
-  double s1 = 0, sx = 0, sy = 0, sxx = 0, sxy = 0, syy = 0, su = 0, sxu = 0, syu = 0, sv = 0, sxv = 0, syv = 0;
+  double sx = 0, sy = 0, sxx = 0, sxy = 0, syy = 0, su = 0, sxu = 0, syu = 0, sv = 0, sxv = 0, syv = 0;
   int valid = 0;
   // the reference keeps the neighbour offsets and the displacements as scalar_t (float)
   auto add = [&](float uf, float vf, float ddx, float ddy) {
     const double dx = ddx, dy = ddy;
     const double u = uf, v = vf;
     ++valid;
-    s1 += 1.0; sx += dx; sy += dy;
+    sx += dx; sy += dy;
     sxx += dx * dx; sxy += dx * dy; syy += dy * dy;
     su += u; sxu += dx * u; syu += dy * u;
     sv += v; sxv += dx * v; syv += dy * v;
@@ -407,15 +462,23 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
   const int ci = min(max((int)floor((xi - g.x0) / g.cell), 0), g.ncx - 1);
   const int cj = min(max((int)floor((yi - g.y0) / g.cell), 0), g.ncy - 1);
   if (F(F_SIGMA, i) >= 0.0 && knn == 0) {
-    for (int cy = max(cj - 1, 0); cy <= min(cj + 1, g.ncy - 1); ++cy)
-      for (int cx = max(ci - 1, 0); cx <= min(ci + 1, g.ncx - 1); ++cx) {
-        const int c = cy * g.ncx + cx;
-        for (int k = g.cell_begin[c] + part; k < g.cell_end[c]; k += L) {
-          const float4 q = R.at(cy, k);
-          const float ddx = q.x - xf, ddy = q.y - yf;
-          if (ddx * ddx + ddy * ddy < r2 && R.id(cy, k) >= 0) add(q.z, q.w, ddx, ddy);
-        }
+    const double rr = sqrt((double)r2) + g.slack;
+    for (int cy = cj - kVsgRings + part; cy <= min(cj + kVsgRings, g.ncy - 1); cy += L) {
+      if (cy < 0) continue;
+      const double ya = g.y0 + cy * g.cell, yb = ya + g.cell;
+      const double away = fmax(fmax(ya - yi, yi - yb) - g.slack, 0.0);
+      if (away > rr) continue;
+      const double half = sqrt(rr * rr - away * away) + g.slack;
+      const int ca = min(max((int)floor((xi - half - g.x0) / g.cell), 0), g.ncx - 1);
+      const int cb = min(max((int)floor((xi + half - g.x0) / g.cell), 0), g.ncx - 1);
+      const float4 *q = R.row(cy);
+      const int e = g.cell_begin[cy * g.ncx + cb + 1];
+      for (int k = g.cell_begin[cy * g.ncx + ca]; k < e; ++k) {
+        const float4 c = q[k];
+        const float ddx = c.x - xf, ddy = c.y - yf;
+        if (ddx * ddx + ddy * ddy < r2) add(c.z, c.w, ddx, ddy);
       }
+    }
   } else if (F(F_SIGMA, i) >= 0.0) {
     // the knn nearest subsets (this one included) by squared float distance, then id: rings of
     // cells around this one until no unvisited cell can hold a closer subset
@@ -430,7 +493,7 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
         for (int cx = ci - r; cx <= ci + r; cx += max(step, 1)) {
           if (cx < 0 || cx >= g.ncx) continue;
           const int c = cy * g.ncx + cx;
-          for (int k = g.cell_begin[c]; k < g.cell_end[c]; ++k) {
+          for (int k = g.cell_begin[c]; k < g.cell_begin[c + 1]; ++k) {
             const int j = g.cell_ids[k] < 0 ? ~g.cell_ids[k] : g.cell_ids[k];
             const float4 q = g.rec[k];
             const float ddx = q.x - xf, ddy = q.y - yf;
@@ -462,7 +525,7 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
 #pragma unroll
       for (int o = L / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o);
     };
-    fold(s1); fold(sx); fold(sy); fold(sxx); fold(sxy); fold(syy);
+    fold(sx); fold(sy); fold(sxx); fold(sxy); fold(syy);
     fold(su); fold(sxu); fold(syu); fold(sv); fold(sxv); fold(syv);
 #pragma unroll
     for (int o = L / 2; o >= 1; o >>= 1) valid += __shfl_xor(valid, o);
@@ -471,6 +534,7 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
   double out[kVsgFields] = {0, 0, 0, 0, 0, 0, 0};
   bool ok = valid >= 3;
   if (ok) {
+    const double s1 = valid;
     const double a[3][3] = {{s1, sx, sy}, {sx, sxx, sxy}, {sy, sxy, syy}};
     double inv[3][3];
     ok = inverse3(a, inv);
@@ -502,79 +566,64 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
 __global__ void vsg_strain_kernel(VsgGrid g, float radius, int knn, double *fields, double *vsg, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  vsg_subset<1>(g, radius, knn, fields, vsg, n, i, 0, VsgGlobalReader{g.rec, g.cell_ids});
-}
-
-__device__ int lower_bound_int(const int *a, int n, int v) {
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int m = (lo + hi) >> 1;
-    if (a[m] < v) lo = m + 1;
-    else hi = m;
-  }
-  return lo;
+  vsg_subset<1>(g, radius, knn, fields, vsg, n, i, 0, VsgGlobalReader{g.rec});
 }
 
 // Radius windows: kVsgLanes lanes per subset; workgroup b takes entries
-// [64 b, 64 b + 64) of the cell-ordered list.  When they lie in one row of cells, every candidate they
-// need lies in three contiguous ranges of the list (the cell rows above, at and
-// below, from one column left of the first cell to one right of the last),
+// [64 b, 64 b + 64) of the cell-ordered list.  When they lie in one row of cells,
+// the candidates they need lie in one contiguous range of the list per cell row
+// (from kVsgRings columns left of the first cell to kVsgRings right of the last),
 // which the workgroup copies to LDS once; otherwise, or when the ranges exceed
 // kVsgTileEntries, its threads read the list directly.  Both give the same
 // sums in the same order.
 constexpr int kVsgTileEntries = 2048;
-#ifndef DICE_VSG_LANES
-#define DICE_VSG_LANES 4
-#endif
-constexpr int kVsgLanes = DICE_VSG_LANES;
+constexpr int kVsgLanes = 4;
 constexpr int kVsgGroupSubsets = 256 / kVsgLanes;
 __global__ __launch_bounds__(256) void vsg_strain_tiled_kernel(VsgGrid g, float radius, double *fields, double *vsg,
                                                                int n) {
   __shared__ float4 srec[kVsgTileEntries];
-  __shared__ int sid[kVsgTileEntries];
-  __shared__ int sh[6];  // start and length of the three ranges
+  __shared__ int lo[kVsgMaxRows], len[kVsgMaxRows], shift[kVsgMaxRows];
+  __shared__ int total;
   const int k0 = blockIdx.x * kVsgGroupSubsets;
   const int k1 = min(k0 + kVsgGroupSubsets, n);
   const int cfirst = g.cell_keys[k0], clast = g.cell_keys[k1 - 1];
   const int cj = cfirst / g.ncx;
   bool tiled = false;
   if (clast / g.ncx == cj) {  // uniform over the workgroup
-    if (threadIdx.x < 3) {
-      const int cy = cj - 1 + (int)threadIdx.x;
-      int lo = 0, hi = 0;
+    if (threadIdx.x < kVsgMaxRows) {
+      const int r = (int)threadIdx.x, cy = cj - kVsgRings + r;
+      int a = 0, b = 0;
       if (cy >= 0 && cy < g.ncy) {
-        const int a = cy * g.ncx + max(cfirst - cj * g.ncx - 1, 0);
-        const int b = cy * g.ncx + min(clast - cj * g.ncx + 1, g.ncx - 1) + 1;
-        lo = lower_bound_int(g.cell_keys, n, a);
-        hi = lower_bound_int(g.cell_keys, n, b);
+        a = g.cell_begin[cy * g.ncx + max(cfirst - cj * g.ncx - kVsgRings, 0)];
+        b = g.cell_begin[cy * g.ncx + min(clast - cj * g.ncx + kVsgRings, g.ncx - 1) + 1];
       }
-      sh[threadIdx.x] = lo;
-      sh[3 + threadIdx.x] = hi - lo;
+      lo[r] = a;
+      len[r] = b - a;
     }
     __syncthreads();
-    tiled = sh[3] + sh[4] + sh[5] <= kVsgTileEntries;
-    if (tiled) {
+    if (threadIdx.x == 0) {
       int off = 0;
-      for (int r = 0; r < 3; ++r) {
-        for (int t = threadIdx.x; t < sh[3 + r]; t += blockDim.x) {
-          srec[off + t] = g.rec[sh[r] + t];
-          sid[off + t] = g.cell_ids[sh[r] + t];
-        }
-        off += sh[3 + r];
+      for (int r = 0; r < kVsgMaxRows; ++r) {
+        shift[r] = off - lo[r];
+        off += len[r];
       }
+      total = off;
     }
+    __syncthreads();
+    tiled = total <= kVsgTileEntries;
+    if (tiled)
+      for (int r = 0; r < kVsgMaxRows; ++r)
+        for (int t = threadIdx.x; t < len[r]; t += blockDim.x) srec[shift[r] + lo[r] + t] = g.rec[lo[r] + t];
     __syncthreads();
   }
   const int k = k0 + (int)threadIdx.x / kVsgLanes, part = (int)threadIdx.x % kVsgLanes;
   if (k >= n) return;  // whole groups of lanes
   const int e = g.cell_ids[k];
   const int i = e < 0 ? ~e : e;
-  if (tiled) {
-    const VsgTileReader R{srec, sid, cj - 1, {sh[0], sh[1], sh[2]}, {0, sh[3], sh[3] + sh[4]}};
-    vsg_subset<kVsgLanes>(g, radius, 0, fields, vsg, n, i, part, R);
-  } else {
-    vsg_subset<kVsgLanes>(g, radius, 0, fields, vsg, n, i, part, VsgGlobalReader{g.rec, g.cell_ids});
-  }
+  if (tiled)
+    vsg_subset<kVsgLanes>(g, radius, 0, fields, vsg, n, i, part, VsgTileReader{srec, shift, cj - kVsgRings});
+  else
+    vsg_subset<kVsgLanes>(g, radius, 0, fields, vsg, n, i, part, VsgGlobalReader{g.rec});
 }
 
 __global__ void uncertainty_kernel(const double *fields, double *out, int n) {
@@ -604,37 +653,22 @@ hipError_t launch_vsg_bounds(const double *fields, int n, double *bounds, hipStr
   return hipGetLastError();
 }
 
-static int vsg_key_bits(long long ncells) {
-  int bits = 1;
-  while ((1LL << bits) < ncells) ++bits;
-  return bits;
-}
-
-hipError_t vsg_grid_temp_bytes(int n, long long ncells, size_t *bytes) {
-  return rocprim::radix_sort_pairs(nullptr, *bytes, (const int *)nullptr, (int *)nullptr, (const int *)nullptr,
-                                   (int *)nullptr, (size_t)n, 0, vsg_key_bits(ncells));
-}
-
-hipError_t launch_vsg_grid(const double *fields, int n, VsgGrid &g, const VsgWork &w, hipStream_t stream) {
+hipError_t launch_vsg_grid(const double *fields, int n, bool radius_window, VsgGrid &g, const VsgWork &w,
+                           hipStream_t stream) {
   if (n <= 0) return hipErrorInvalidValue;
-  const long long ncells = (long long)g.ncx * g.ncy;
-  hipLaunchKernelGGL(zero_ints_kernel, dim3((int)((2 * ncells + 255) / 256)), dim3(256), 0, stream, w.cell_range,
-                     (int)(2 * ncells));
-  hipLaunchKernelGGL(vsg_cells_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, fields, n, g, w.keys, w.ids);
-  hipError_t e = hipGetLastError();
+  const int ncells = g.ncx * g.ncy, groups = (ncells + kVsgScan - 1) / kVsgScan;
+  const dim3 per_subset((n + 255) / 256), block(256);
+  hipError_t e = launch_zero_ints(w.count, ncells, stream);
   if (e != hipSuccess) return e;
-  // ids ordered by cell; the radix sort is stable, so ids ascend within a cell
-  size_t bytes = w.temp_bytes;
-  e = rocprim::radix_sort_pairs(w.temp, bytes, (const int *)w.keys, w.keys_sorted, (const int *)w.ids, w.ids_sorted,
-                                (size_t)n, 0, vsg_key_bits(ncells), stream);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(vsg_ranges_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, w.keys_sorted, n, w.cell_range,
-                     w.cell_range + ncells);
-  hipLaunchKernelGGL(vsg_pack_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, fields, n, w.ids_sorted, w.rec);
-  g.cell_begin = w.cell_range;
-  g.cell_end = w.cell_range + ncells;
-  g.cell_ids = w.ids_sorted;
-  g.cell_keys = w.keys_sorted;
+  hipLaunchKernelGGL(vsg_cells_kernel, per_subset, block, 0, stream, fields, n, g, w.count, w.cells, w.turn);
+  hipLaunchKernelGGL(vsg_sums_kernel, dim3(groups), block, 0, stream, w.count, ncells, w.sums);
+  hipLaunchKernelGGL(vsg_starts_kernel, dim3(groups), block, 0, stream, w.count, ncells, n, w.sums, w.cell_start);
+  hipLaunchKernelGGL(vsg_place_kernel, per_subset, block, 0, stream, w.cells, w.turn, w.cell_start, n, w.arrived);
+  hipLaunchKernelGGL(vsg_pack_kernel, per_subset, block, 0, stream, fields, w.cells, w.cell_start, w.arrived, n,
+                     radius_window ? 1 : 0, w.keys, w.ids, w.rec);
+  g.cell_begin = w.cell_start;
+  g.cell_ids = w.ids;
+  g.cell_keys = w.keys;
   g.rec = w.rec;
   return hipGetLastError();
 }
