@@ -4684,16 +4684,17 @@ struct BlockClaims {
 // are all kept, and hands the others to pa.ov_list for the PLAIN kernel.
 // PLAIN is bound by its taps: 36 scattered loads per pixel and pass through
 // the CU's one texture-address unit.  From LDS the kernel is bound by VALU issue
-// (84 % of the quad-cycles at four waves per SIMD), so the sums per pixel count:
-// Gauss-Newton adds q and sum(G) only (7 FP64 adds instead of 35) and takes H
-// from the per-subset S.  2,280 subsets of 75 x 75 (1500 x 1100, six
-// parameters): 1.49 -> 0.44 ms per frame; 8,000 polygons of 200-3000 px, half of
-// them too large for a slot: 1.91 -> 0.84 ms.  NT = 1024 when there is at most
-// one subset per CU (a subset's latency is then what counts): six 61 x 61
-// subsets by Nelder-Mead 0.99 -> 0.78 ms, bookkeeping in one wave only.
-// Registers: four waves per SIMD with some spills beat two without (0.53 against
-// 0.59 ms, and 0.95 against 1.08 ms for the polygons, measured with an earlier
-// reduction).
+// (84 % of the quad-cycles); Gauss-Newton adds PLAIN's 35 products per pixel in
+// FP64 and reads the totals from LDS.  (H from the per-subset S, with 7 sums per
+// pixel, takes the same time and rounds H differently.)  What Gauss-Newton
+// leaves to PLAIN are the systems that its L D L^T refuses.  2,280 subsets of
+// 75 x 75 (1500 x 1100, six parameters): 1.49 -> 0.44 ms per frame; 8,000
+// polygons of 200-3000 px, half of them too large for a slot: 1.91 -> 0.84 ms.
+// NT = 1024 when there is at most one subset per CU (a subset's latency is then
+// what counts): six 61 x 61 subsets by Nelder-Mead 0.99 -> 0.78 ms, bookkeeping
+// in one wave only.  Registers: three waves per SIMD beat two and, with its
+// spills, four (0.48 against 0.59 and 0.53 ms; 0.96 against 1.08 and 0.95 ms for
+// the polygons, measured with an earlier reduction).
 #ifndef DICE_WIDE_WPE
 #define DICE_WIDE_WPE 3
 #endif
