@@ -3716,7 +3716,7 @@ struct Solver {
   //           SIMPLEX_THEN_GRADIENT_BASED for the subsets that asked for it.
   // SIMPLEX_OPT selects which optimizer this instantiation runs.  A BATCHED
   // wave whose window overflows its LDS slot pushes the subset to ov_list and
-  // leaves it to the PLAIN kernel (nothing it wrote is an input of the solve).
+  // leaves it to the next kernel (nothing it wrote is an input of the solve).
   // nm: per-subset Nelder-Mead results of simplex_groups_kernel for this pass
   // (SIMPLEX_OPT only), or null to run the simplex here.  NM_ONLY: the
   // instantiation holds no simplex (and so needs far fewer registers); a
@@ -4680,8 +4680,8 @@ struct BlockClaims {
 // The subsets whose window outgrew a BATCHED wave's slot (or all of them when
 // the subset side says so in advance, pa.count_all): one workgroup of NT
 // threads per subset, in PLAIN's arithmetic -- FP64 sums -- with the deformed
-// window in LDS (cap floats).  Gauss-Newton takes the subsets whose pixels
-// are all kept, and hands the others to pa.ov_list for the PLAIN kernel.
+// window in LDS (cap floats).  Gauss-Newton hands what it cannot finish to
+// pa.ov_list for the PLAIN kernel.
 // PLAIN is bound by its taps: 36 scattered loads per pixel and pass through
 // the CU's one texture-address unit.  From LDS the kernel is bound by VALU issue
 // (84 % of the quad-cycles); Gauss-Newton adds PLAIN's 35 products per pixel in
