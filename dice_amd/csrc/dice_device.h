@@ -4686,12 +4686,13 @@ struct BlockClaims {
 // the CU's one texture-address unit.  From LDS the kernel is bound by VALU issue
 // (84 % of the quad-cycles); Gauss-Newton adds PLAIN's 35 products per pixel in
 // FP64 and reads the totals from LDS.  (H from the per-subset S, with 7 sums per
-// pixel, takes the same time and rounds H differently.)  What Gauss-Newton
-// leaves to PLAIN are the systems that its L D L^T refuses.  2,280 subsets of
-// 75 x 75 (1500 x 1100, six parameters): 1.49 -> 0.44 ms per frame; 8,000
-// polygons of 200-3000 px, half of them too large for a slot: 1.91 -> 0.84 ms.
+// pixel, is a tenth faster, but moves the last bit of 5-10 % of the parameters.)
+// What Gauss-Newton leaves to PLAIN are the systems that its L D L^T refuses.
+// 2,280 subsets of 75 x 75 (1500 x 1100, six parameters): 1.48 -> 0.48 ms per
+// frame; 8,000 polygons of 200-3000 px, half of them too large for a slot: 1.93 ->
+// 0.98 ms.
 // NT = 1024 when there is at most one subset per CU (a subset's latency is then
-// what counts): six 61 x 61 subsets by Nelder-Mead 0.99 -> 0.78 ms, bookkeeping
+// what counts): six 61 x 61 subsets by Nelder-Mead 1.01 -> 0.83 ms, bookkeeping
 // in one wave only.  Registers: three waves per SIMD beat two and, with its
 // spills, four (0.48 against 0.59 and 0.53 ms; 0.96 against 1.08 and 0.95 ms for
 // the polygons, measured with an earlier reduction).
@@ -4879,7 +4880,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_W
 
 // The same two passes with at most kCrewMaxSubsets subsets: four waves per
 // subset.  One wave each leaves most SIMDs idle and the frame takes a subset's
-// whole latency: 49 subsets of 27 x 27, 87 us in the general kernel, 35 here.
+// whole latency: 49 subsets of 27 x 27, 87 us in the general kernel, 32 here.
 // With 2,116 subsets of 31 x 31 every SIMD has two waves of its own and the lean
 // kernel is the faster one (129 against 168 us with four waves per subset).
 template <typename T, int INTERP, bool TRANS>
