@@ -2373,6 +2373,9 @@ struct Solver {
   // images with every sample x + u, y + v away from the border, so the Keys
   // weights are those of the fractional parts of (u, v) for every pixel and the
   // unshifted deformed pixel is in the window (otherwise false: hand over).
+  // PIXEL: the weights of each pixel's own rounded position x + u, y + v, as
+  // uncertainty() has them with bilinear images (S <= 64: a column per lane).
+  template <bool PIXEL = false>
   __device__ __forceinline__ bool lean_uncertainty(const Affine &A, double *fields, int nsub, int gid) {
     const float u = A.p[0], v = A.p[1];
     const int fu = (int)floorf(u), fv = (int)floorf(v);
@@ -2382,7 +2385,8 @@ struct Solver {
                            (float)ly0 + v > 2.5f + m && (float)ly1 + v < (float)def.h - 3.5f - m;
     if (!uniform_w || lx1 > def.w - 2 || ly1 > def.h - 2) return false;
     // the taps of x + u are x + fu - 2 .. x + fu + 3 (integer offsets: no rounding margin)
-    if (!stage(lx0 + fu - 2, lx1 + fu + 3, ly0 + fv - 2, ly1 + fv + 3)) return false;
+    const int pm = PIXEL ? 1 : 0;
+    if (!stage(lx0 + fu - 2 - pm, lx1 + fu + 3 + pm, ly0 + fv - 2 - pm, ly1 + fv + 3 + pm)) return false;
     if (!(wx0 <= lx0 && wx0 + wpitch > lx1 && wy0 <= ly0 && wy0 + wrows > ly1)) return false;
     float wxu[6], wyu[6];
     keys_weights(u - (float)fu, wxu);
@@ -2462,6 +2466,19 @@ struct Solver {
         }
       }
     };
+    if constexpr (PIXEL) {
+      if (lane < S) {
+        const int rx = x0 + lane - ref.ox;
+#pragma unroll 1
+        for (int r = ra; r < rb; ++r) {
+          const int ry = y0 + r - ref.oy;
+          pixel(ry * ref.w + rx, keys_single(win, wpitch, wx0, wy0, (float)rx + u, (float)ry + v),
+                win + (__umul24(ry - wy0, wpitch) + (rx - wx0)));
+        }
+      }
+      unc_record(pt, u, v, fields, nsub, gid);
+      return true;
+    }
     const int nfull = S >> 5;
 #pragma unroll 1
     for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), ra + (lane >> 5));
@@ -2846,7 +2863,7 @@ struct Solver {
           const int ww = min(bx1 - ref.ox + fu + 4, def.w - 1) - max(bx0 - ref.ox + fu - 3, 0) + 1;
           const int hh = min(by1 - ref.oy + fv + 4, def.h - 1) - max(by0 - ref.oy + fv - 3, 0) + 1;
           if (ww > 0 && hh > 0 && ww * hh > win_cap) return kOverflow;
-          if (!lean_uncertainty(A, fields, nsub, gid)) return kOverflow;
+          if (!lean_uncertainty<INTERP == 0>(A, fields, nsub, gid)) return kOverflow;
         }
         break;
       }

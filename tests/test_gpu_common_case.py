@@ -84,3 +84,33 @@ def test_same_results(scene, S, interp, dtype, affine):
         general = run(ctx, q, ref, de, cx, cy, S)
         ok = general[dh.F["STATUS"]] != 5  # flat or empty subsets fail the threshold
         same(wave[:, ok], general[:, ok])
+
+
+@pytest.mark.parametrize("step", [6, 55], ids=["wave", "crew"])
+def test_bilinear_uncertainty_far_from_the_origin(step):
+    """With bilinear images the uncertainty fields take each pixel's weights from the float sum x + u, which
+    rounds by 2^-13 px at x = 1100: the translation kernels follow the general one in that.  The terms are
+    positive and at most 64 pixels go to an FP32 lane sum in each kernel, in another order: 64 * 2^-24 on r_tot2
+    and the other sums, half of that after the root, twice for the two kernels: 4e-6."""
+    w, h, S = 1300, 200, 35
+    sp = synth.Speckle(w, h, seed=33)
+    ref = sp.frame(None)
+    de = sp.frame(synth.affine_field(0.37, -0.21, 0.0, 0.0, 0.0, 0.0), noise_sigma=1.0, noise_seed=34)
+    gx, gy = np.meshgrid(np.arange(22, w - 22, step), np.arange(22, h - 22, step))
+    cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
+    assert (len(cx) > 1024) == (step == 6)
+    p = dh.default_params()
+    p.optimization_method = dh.GRADIENT_BASED
+    p.interpolation_method = dh.BILINEAR
+    ctx = dh.Context(0)
+    a = run(ctx, p, ref, de, cx, cy, S)
+    p.initial_gamma_threshold = 1e9
+    b = run(ctx, p, ref, de, cx, cy, S)
+    ctx.close()
+    for name in EXACT:
+        assert np.array_equal(a[dh.F[name]], b[dh.F[name]]), name
+    ok = np.isin(a[dh.F["STATUS"]], dh.CONVERGED_STATUSES)
+    assert ok.mean() > 0.9
+    for k in (1, 3, 4, 5, 6, 7):
+        x, y = a[dh.F["FIELD_%d" % k]][ok], b[dh.F["FIELD_%d" % k]][ok]
+        assert np.all(np.abs(x - y) <= 4e-6 * np.abs(y)), k
