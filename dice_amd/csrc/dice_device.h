@@ -4707,10 +4707,11 @@ struct BlockClaims {
 // What Gauss-Newton leaves to PLAIN are the systems that its L D L^T refuses.
 // 2,280 subsets of 75 x 75 (1500 x 1100, six parameters): 1.48 -> 0.48 ms per
 // frame; 8,000 polygons of 200-3000 px, half of them too large for a slot: 1.93 ->
-// 0.98 ms.
-// NT = 1024 when there is at most one subset per CU (a subset's latency is then
-// what counts): six 61 x 61 subsets by Nelder-Mead 1.01 -> 0.83 ms, bookkeeping
-// in one wave only.  Registers: three waves per SIMD beat two and, with its
+// 0.98 ms.  NT = 1024 for Nelder-Mead when there is at most one subset per CU (a
+// subset's latency is then what counts): six 61 x 61 subsets 1.01 -> 0.83 ms,
+// bookkeeping in one wave only.  A Gauss-Newton step is too short for that: 108
+// subsets of 69 x 69 take 177 us with 1,024 threads each and 123 us with 256, and
+// about 240 of 71 x 71 163 and 119 us.  Registers: three waves per SIMD beat two and, with its
 // spills, four (0.48 against 0.59 and 0.53 ms; 0.96 against 1.08 and 0.95 ms for
 // the polygons, measured with an earlier reduction).
 #ifndef DICE_WIDE_WPE
@@ -4747,15 +4748,17 @@ template <typename T, int INTERP, bool SX>
 hipError_t launch_wide_variant(const Launch &L, const KParams &kp, const DImage &ref, const DImage &def,
                                const DSubsets &subs, double *fields, const PassArgs &pa, hipStream_t stream) {
   const size_t shm = (size_t)L.wide_floats * sizeof(float);
-  if (subs.n <= L.num_cus) {
-    // at most one subset per CU: its latency counts, so every SIMD gets four waves of it
-    hipLaunchKernelGGL((correlate_wide_kernel<T, INTERP, SX, 1024>), dim3(subs.n), dim3(1024), shm, stream, kp, ref,
-                       def, subs, fields, pa, L.wide_floats);
-  } else {
-    const int groups = subs.n < 4 * L.num_cus ? subs.n : 4 * L.num_cus;
-    hipLaunchKernelGGL((correlate_wide_kernel<T, INTERP, SX, 256>), dim3(groups), dim3(256), shm, stream, kp, ref, def,
-                       subs, fields, pa, L.wide_floats);
+  if constexpr (SX) {
+    if (subs.n <= L.num_cus) {
+      // at most one subset per CU: its latency counts, so every SIMD gets four waves of it
+      hipLaunchKernelGGL((correlate_wide_kernel<T, INTERP, SX, 1024>), dim3(subs.n), dim3(1024), shm, stream, kp, ref,
+                         def, subs, fields, pa, L.wide_floats);
+      return hipGetLastError();
+    }
   }
+  const int groups = subs.n < 4 * L.num_cus ? subs.n : 4 * L.num_cus;
+  hipLaunchKernelGGL((correlate_wide_kernel<T, INTERP, SX, 256>), dim3(groups), dim3(256), shm, stream, kp, ref, def,
+                     subs, fields, pa, L.wide_floats);
   return hipGetLastError();
 }
 
