@@ -2523,9 +2523,8 @@ struct Solver {
   // in the chunk, a constant after unrolling) and, one wave only, g(r1) after each
   // kTransChunk rows, r1 the rows done; returns after the group's sync.  REF: the
   // reference loads that f needs (0 none, 1 F, 2 F, gx and gy).
-  // S <= 64: a column per lane; the lanes past the last column repeat it (no
+  // S <= kTransMaxSide: a column per lane; the lanes past the last column repeat it (no
   // branch per row; f must bear the repeats).
-  static constexpr int kTransChunk = 6;  // the rows after which the unrolled walk has turned its six sums around
   template <int REF, class F, class C>
   __device__ __forceinline__ void trans_values(const Affine &A, F &&f, C &&g) {
     const int lane = lid(), w = wid();
@@ -4848,14 +4847,6 @@ hipError_t launch_lean_variant(const Launch &L, const KParams &kp, const DImage 
   return hipGetLastError();
 }
 
-// The window of a translated square subset: S + 6 pixels a side at most (the
-// taps and a fractional shift), S + 11 and S + 12 with the ring and the odd
-// pitch; a multiple of four floats.
-__host__ __device__ inline int trans_window_floats(int side, int cap) {
-  const int w = ((side + 12) * (side + 11) + 3) & ~3;
-  return w < cap ? w : cap & ~3;
-}
-
 #ifndef DICE_TRANS_WPE
 #define DICE_TRANS_WPE 3
 #endif
@@ -4941,15 +4932,6 @@ __global__ __launch_bounds__(256) void correlate_crew_kernel(KParams kp, DImage 
                                });
     __syncthreads();
   }
-}
-
-// LDS floats of a wave of correlate_trans_kernel and of a crew: the slot (the
-// window and the per-subset constants), gtab, and a crew's reference tables.
-inline int trans_lds_floats(int S, int slot, bool crew) {
-  const int side = 2 * (S / 2) + 1;
-  if (crew) return slot + 4 * side * side;
-  return trans_window_floats(side, slot - kPersistFloats) + kPersistFloats +
-         4 * Solver<float, TightWave, 2, false>::kTransChunk * side;
 }
 
 template <typename T, int INTERP, bool TRANS>

@@ -1,0 +1,57 @@
+// Which common-case Gauss-Newton kernel takes a pass over square subsets, and
+// the LDS that it asks for.  Host arithmetic only, so that it can be tested
+// without a GPU.
+#pragma once
+#include <cstddef>
+
+namespace dice_hip {
+
+// Per-subset constants of the BATCHED fast Gauss-Newton pass at the end of a
+// wave's slot: the 6 x 6 matrix sum(phi phi^T), sum(phi), sum(F) and the pixel
+// count (44 doubles), then the sums of the current pass, sum(gmf phi) and
+// sum(G) (7 doubles), and one double of padding.
+constexpr int kPersistFloats = 104;
+
+// The most dynamic LDS that the kernels below are launched with.
+constexpr size_t kMaxLaunchLds = 64 * 1024 - 2048;
+constexpr int kCrewMaxSubsets = 1024;
+// correlate_trans_kernel and its crew hold a column of the subset per lane.
+constexpr int kTransMaxSide = 64;
+// rows after which the translation walk's six row sums are back in their places
+constexpr int kTransChunk = 6;
+
+// The side of the square subsets of size S (DICe_Subset.cpp:90-92): odd, so
+// that an even S means S + 1 pixels.
+constexpr int square_side(int S) { return 2 * (S / 2) + 1; }
+
+// The window of a translated square subset: side + 6 pixels at most (the taps
+// and a fractional shift), side + 11 and side + 12 with the ring and the odd
+// pitch; a multiple of four floats.
+constexpr int trans_window_floats(int side, int cap) {
+  const int w = ((side + 12) * (side + 11) + 3) & ~3;
+  return w < cap ? w : cap & ~3;
+}
+
+// LDS floats of a wave of correlate_trans_kernel and of a crew: the slot (the
+// window and the per-subset constants), gtab, and a crew's reference tables.
+constexpr int trans_lds_floats(int S, int slot, bool crew) {
+  const int side = square_side(S);
+  if (crew) return slot + 4 * side * side;
+  return trans_window_floats(side, slot - kPersistFloats) + kPersistFloats + 4 * kTransChunk * side;
+}
+
+enum class CommonKernel { kNone, kLean, kTrans, kCrew };
+
+// The kernel for n subsets of size S, all six parameters (affine) or translation
+// only, with slot floats of LDS per wave.  All six parameters: the lean kernel;
+// translation only: its own kernel; few subsets of either kind: four waves each.
+inline CommonKernel common_kernel(int n, int S, bool affine, int slot) {
+  auto fits = [&](bool crew) {
+    return square_side(S) <= kTransMaxSide && trans_lds_floats(S, slot, crew) * sizeof(float) <= kMaxLaunchLds;
+  };
+  if (n <= kCrewMaxSubsets && fits(true)) return CommonKernel::kCrew;
+  if (affine) return CommonKernel::kLean;
+  return fits(false) ? CommonKernel::kTrans : CommonKernel::kNone;
+}
+
+}  // namespace dice_hip

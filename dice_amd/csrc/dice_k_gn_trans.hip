@@ -27,9 +27,4 @@ hipError_t launch_gn_crew(int storage, int interp, int trans, const Launch &L, c
 #undef V
 }
 
-// Dynamic LDS of the kernels above for subsets of side S, in floats.
-int trans_lds_floats(const Launch &L, int S, int crew) {
-  return dev::trans_lds_floats(S, L.lds_floats_per_wave, crew != 0);
-}
-
 }  // namespace dice_hip

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "dice_dispatch.h"
+
 namespace dice_hip {
 
 constexpr int kWave = 64;
@@ -106,11 +108,7 @@ constexpr int kGnSums = 35;
 constexpr int kGnRedStride = kWave + 1;
 constexpr int kGnTotOffset = kGnSums * kGnRedStride + 1;
 constexpr int kGnTotQ = 0, kGnTotH = 8, kGnTotR = 44;
-// Per-subset constants of the BATCHED fast Gauss-Newton pass at the end of a
-// wave's slot: the 6 x 6 matrix sum(phi phi^T), sum(phi), sum(F) and the pixel
-// count (44 doubles), then the sums of the current pass, sum(gmf phi) and
-// sum(G) (7 doubles), and one double of padding.
-constexpr int kPersistFloats = 104;
+// The per-subset constants at the end of a wave's slot: kPersistFloats.
 constexpr int kPersistPass = 44;  // double offset of the current pass's sums
 // The lean kernel's layout of the same area (double offsets): the L D L^T
 // factors of S (L strictly lower, packed by rows, 15; then 1/d, 6), sum(phi)
@@ -136,13 +134,6 @@ struct Launch {
   int wide_only;               // batched: no subset's window can fit a wave's slot
   int num_cus;
 };
-
-// Dynamic LDS of a launch without further attributes.
-constexpr size_t kMaxLaunchLds = 64 * 1024 - 2048;
-#ifndef DICE_CREW_MAX
-#define DICE_CREW_MAX 1024
-#endif
-constexpr int kCrewMaxSubsets = DICE_CREW_MAX;
 
 // Subsets of at most this many pixels run the Nelder-Mead iterations of the
 // BATCHED mode in rows of 16 lanes per subset (simplex_groups_kernel): a wave

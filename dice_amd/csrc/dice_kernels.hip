@@ -22,7 +22,6 @@ hipError_t launch_gn_trans(int, int, const Launch &, const KParams &, const DIma
                            double *, const PassArgs &, hipStream_t);
 hipError_t launch_gn_crew(int, int, int, const Launch &, const KParams &, const DImage &, const DImage &,
                           const DSubsets &, double *, const PassArgs &, hipStream_t);
-int trans_lds_floats(const Launch &, int, int);
 hipError_t launch_gn_wide(int, int, const Launch &, const KParams &, const DImage &, const DImage &, const DSubsets &,
                           double *, const PassArgs &, hipStream_t);
 hipError_t launch_simplex_wide(int, int, const Launch &, const KParams &, const DImage &, const DImage &,
@@ -734,9 +733,8 @@ static hipError_t launch_pass(bool simplex, int storage, const Launch &L, const 
   if (!wide_only) {
     // Gauss-Newton pass 0 of square subsets with none of the options that the
     // common-case kernels leave out: they take every subset first and hand the
-    // others (and those that leave the common case) to the general kernel.  All
-    // six parameters: the lean kernel; translation only: its own kernel; few
-    // subsets of either kind: four waves each.
+    // others (and those that leave the common case) to the general kernel
+    // (common_kernel says which of them).
     const int np = (kp.en_rot != 0) + (kp.en_normal != 0) + (kp.en_shear != 0);
     if (!simplex && pa.pass == 0 && subs.S > 0 && !subs.mbox && !kp.def_grads && kp.momentum == 0.0f &&
         kp.init_gamma_thr == -1.0 && !kp.has_forced && kp.lm_alpha <= 0.0f && (np == 3 || np == 0)) {
@@ -744,16 +742,16 @@ static hipError_t launch_pass(bool simplex, int storage, const Launch &L, const 
       pl.counter = work + kWorkSetLean * kWorkCounterInts;
       pl.ov_list = other;
       pl.ov_count = work + kWorkLeanCount;
-      auto fits = [&](int crew) { return subs.S <= 64 && trans_lds_floats(L, subs.S, crew) * sizeof(float) <= kMaxLaunchLds; };
-      const bool crew = subs.n <= kCrewMaxSubsets && fits(1);
+      const CommonKernel common = common_kernel(subs.n, subs.S, np == 3, L.lds_floats_per_wave);
       e = hipSuccess;
-      bool taken = true;
-      if (crew) e = launch_gn_crew(storage, kp.interp, np == 0, L, kp, ref, def, subs, fields, pl, stream);
-      else if (np == 3) e = launch_gn_lean(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
-      else if (fits(0)) e = launch_gn_trans(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
-      else taken = false;
+      if (common == CommonKernel::kCrew)
+        e = launch_gn_crew(storage, kp.interp, np == 0, L, kp, ref, def, subs, fields, pl, stream);
+      else if (common == CommonKernel::kLean)
+        e = launch_gn_lean(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
+      else if (common == CommonKernel::kTrans)
+        e = launch_gn_trans(storage, kp.interp, L, kp, ref, def, subs, fields, pl, stream);
       if (e != hipSuccess) return e;
-      if (taken) {
+      if (common != CommonKernel::kNone) {
         pa.items = pl.ov_list;
         pa.item_count = pl.ov_count;
       }

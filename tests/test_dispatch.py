@@ -1,0 +1,39 @@
+"""The rule that picks a common-case Gauss-Newton kernel (dice_amd/csrc/dice_dispatch.h), compiled for the host
+and swept over subset sizes, counts and LDS slots."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+NONE, LEAN, TRANS, CREW = range(4)
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("dispatch") / "dispatch")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-o", exe,
+                           os.path.join(ROOT, "tests", "cpp", "dispatch.cpp")])
+
+    def ask(rows):
+        text = "\n".join(" ".join(str(int(v)) for v in r) for r in rows)
+        out = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=60, check=True).stdout
+        return np.array(out.split(), dtype=np.int64).reshape(len(rows), -1)
+
+    return ask
+
+
+def sweep(ns=(1, 255, 1024, 1025, 5000), sizes=range(1, 100), slots=(2560, 2704, 2812, 5184, 6400, 16000)):
+    return [(n, S, affine, slot) for n in ns for S in sizes for affine in (0, 1) for slot in slots]
+
+
+def test_the_translation_kernels_have_a_lane_per_column(rule):
+    """A subset of even size S is S + 1 pixels wide: size 64 has 65 columns, one more than a wave has lanes."""
+    rows = sweep()
+    for (n, S, affine, slot), (kernel, wave_lds, crew_lds) in zip(rows, rule(rows)):
+        if kernel in (TRANS, CREW):
+            assert S // 2 * 2 + 1 <= 64, (n, S, affine, slot)
+            assert (crew_lds if kernel == CREW else wave_lds) <= 62 * 1024, (n, S, affine, slot)
+        assert kernel != TRANS or not affine, (n, S, affine, slot)
+        assert kernel != LEAN or affine, (n, S, affine, slot)
