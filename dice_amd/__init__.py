@@ -91,6 +91,7 @@ EXPORTS = [
     "dice_hip_correlate_points", "dice_hip_gamma", "dice_hip_gamma_adjoint", "dice_hip_gauss_filter",
     "dice_hip_neighbor_rounds", "dice_hip_vsg_strain", "dice_hip_vsg_strain_device",
     "dice_hip_uncertainty", "dice_hip_uncertainty_device", "dice_hip_objective", "dice_hip_pass_counts",
+    "dice_hip_handover_counts",
     "dice_hip_correlate_device_noalloc", "dice_hip_set_force_simplex", "dice_hip_set_subset_masks",
     "dice_hip_set_image_offsets",
 ]
@@ -153,6 +154,7 @@ def lib():
         L.dice_hip_gauss_filter.argtypes = [I, I, I, I, P, P, I]
         L.dice_hip_neighbor_rounds.argtypes = [P]
         L.dice_hip_pass_counts.argtypes = [P, P]
+        L.dice_hip_handover_counts.argtypes = [P, P]
         L.dice_hip_set_force_simplex.argtypes = [P, P]
         L.dice_hip_set_subset_masks.argtypes = [P, P, P, P]
         L.dice_hip_set_image_offsets.argtypes = [P, I, I, I, I]
@@ -360,6 +362,13 @@ class Context:
         of the last correlation launch."""
         c = np.zeros(3, dtype=np.int32)
         self._check(self._lib.dice_hip_pass_counts(self.h, _p(c)), "pass_counts")
+        return tuple(int(v) for v in c)
+
+    def handover_counts(self):
+        """dice_hip_handover_counts: subsets that the common-case kernel left to the general one and that the
+        workgroup-per-subset kernel left to the PLAIN one (primary pass, fallback pass) in the last launch."""
+        c = np.zeros(3, dtype=np.int32)
+        self._check(self._lib.dice_hip_handover_counts(self.h, _p(c)), "handover_counts")
         return tuple(int(v) for v in c)
 
     def synchronize(self):

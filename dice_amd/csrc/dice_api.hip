@@ -868,7 +868,8 @@ int dice_hip_correlate_device_noalloc(dice_hip_context *ctx, int mode, double *d
 
 int dice_hip_neighbor_rounds(dice_hip_context *ctx) { return ctx ? ctx->nb_rounds : DICE_HIP_EINVAL; }
 
-int dice_hip_pass_counts(dice_hip_context *ctx, int *counts) {
+// three counts of the work area's header, at the given indexes
+static int read_counts(dice_hip_context *ctx, int *counts, int a, int b, int c) {
   if (!ctx) return DICE_HIP_EINVAL;
   if (!counts) return ctx->fail(DICE_HIP_EINVAL, "null counts");
   counts[0] = counts[1] = counts[2] = 0;
@@ -877,10 +878,18 @@ int dice_hip_pass_counts(dice_hip_context *ctx, int *counts) {
   int h[dice_hip::kWorkHeader];
   HIP_TRY(ctx, hipMemcpyAsync(h, ctx->last_work, sizeof h, hipMemcpyDeviceToHost, ctx->stream), "hipMemcpy counts");
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream), "pass counts");
-  counts[0] = h[dice_hip::kWorkFbCount];
-  counts[1] = h[dice_hip::kWorkOv0Count];
-  counts[2] = h[dice_hip::kWorkOv1Count];
+  counts[0] = h[a];
+  counts[1] = h[b];
+  counts[2] = h[c];
   return DICE_HIP_OK;
+}
+
+int dice_hip_pass_counts(dice_hip_context *ctx, int *counts) {
+  return read_counts(ctx, counts, dice_hip::kWorkFbCount, dice_hip::kWorkOv0Count, dice_hip::kWorkOv1Count);
+}
+
+int dice_hip_handover_counts(dice_hip_context *ctx, int *counts) {
+  return read_counts(ctx, counts, dice_hip::kWorkLeanCount, dice_hip::kWorkWideCount, dice_hip::kWorkWideCount + 1);
 }
 
 // VSG strains: the subsets binned on the device into a uniform grid (cells of

@@ -259,6 +259,11 @@ int dice_hip_neighbor_rounds(dice_hip_context *ctx);
  * the primary and the fallback pass and were solved by a workgroup each.  No
  * counterpart in the reference: a diagnostic of this library's launches. */
 int dice_hip_pass_counts(dice_hip_context *ctx, int *counts);
+/* The hand-overs between the kernels of that launch: counts[0] subsets that a
+ * common-case Gauss-Newton kernel left to the general one, counts[1] and
+ * counts[2] those that the workgroup-per-subset kernel left to the PLAIN kernel
+ * in the primary and the fallback pass.  A diagnostic, as above. */
+int dice_hip_handover_counts(dice_hip_context *ctx, int *counts);
 
 /* A multi-frame sequence: the CLI frame loop of execute_correlation calls
  * (DICe_Main.cpp:324-374) for n_frames deformed frames already in device
