@@ -2375,7 +2375,12 @@ struct Solver {
   // unshifted deformed pixel is in the window (otherwise false: hand over).
   // PIXEL: the weights of each pixel's own rounded position x + u, y + v, as
   // uncertainty() has them with bilinear images (S <= 64: a column per lane).
-  template <bool PIXEL = false>
+  // FAR: an unshifted pixel outside the window is read from the image.  The
+  // window's ring is at most 2 px and the odd pitch's column, so that is any
+  // motion of more than 5 px, where handing the finished subset over solves it a
+  // second time: 14,664 subsets of 35 x 35 (8 bits) moved by 7 px, 0.66 ms in the
+  // general kernel alone, 0.95 ms with the hand-over, 0.35 ms here.
+  template <bool PIXEL = false, bool FAR = false>
   __device__ __forceinline__ bool lean_uncertainty(const Affine &A, double *fields, int nsub, int gid) {
     const float u = A.p[0], v = A.p[1];
     const int fu = (int)floorf(u), fv = (int)floorf(v);
@@ -2383,11 +2388,13 @@ struct Solver {
     const float m = 1e-3f;
     const bool uniform_w = (float)lx0 + u > 2.5f + m && (float)lx1 + u < (float)def.w - 3.5f - m &&
                            (float)ly0 + v > 2.5f + m && (float)ly1 + v < (float)def.h - 3.5f - m;
-    if (!uniform_w || lx1 > def.w - 2 || ly1 > def.h - 2) return false;
+    const bool edge = lx1 > def.w - 2 || ly1 > def.h - 2;
+    if (!uniform_w || (!FAR && edge)) return false;
     // the taps of x + u are x + fu - 2 .. x + fu + 3 (integer offsets: no rounding margin)
     const int pm = PIXEL ? 1 : 0;
     if (!stage(lx0 + fu - 2 - pm, lx1 + fu + 3 + pm, ly0 + fv - 2 - pm, ly1 + fv + 3 + pm)) return false;
-    if (!(wx0 <= lx0 && wx0 + wpitch > lx1 && wy0 <= ly0 && wy0 + wrows > ly1)) return false;
+    const bool e_in_win = !edge && wx0 <= lx0 && wx0 + wpitch > lx1 && wy0 <= ly0 && wy0 + wrows > ly1;
+    if (!FAR && !e_in_win) return false;
     float wxu[6], wyu[6];
     keys_weights(u - (float)fu, wxu);
     keys_weights(v - (float)fv, wyu);
@@ -2405,106 +2412,115 @@ struct Solver {
       for (int k = 1; k < 6; ++k) rs = fmaf(p[k], wxu[k], rs);
       return rs;
     };
-    auto pixel = [&](int o, float interp, const lds_float *e) {
-      float refv, gx, gy;
-      ref_at(o, refv, gx, gy);
-      unc_terms(u, v, gx, gy, interp - refv, *e - refv, pt);
-    };
-    auto column = [&](int x, int r0) {
-      if (kNW > 1 && r0 >= rb) return;
-      constexpr int step = 2;
-      const int rx = x - ref.ox, ry0 = y0 + r0 - ref.oy;
-      int o = ry0 * ref.w + rx;
-      const int ostep = step * ref.w;
-      // taps of (rx + u, ry + v): window rows ry + fv - 2 .. + 3, columns rx + fu - 2 .. + 3
-      const lds_float *t = win + (__umul24(ry0 + fv - 2 - wy0, wpitch) + (rx + fu - 2 - wx0));
-      const lds_float *e = win + (__umul24(ry0 - wy0, wpitch) + (rx - wx0));
-      const int tstep = step * wpitch;
-      {
-        float h0 = rowsum(t), h1 = rowsum(t + wpitch), h2 = rowsum(t + 2 * wpitch), h3 = rowsum(t + 3 * wpitch),
-              h4 = rowsum(t + 4 * wpitch), h5 = rowsum(t + 5 * wpitch);
-        // this column in the last row of the window: the rows read ahead at the last step
-        // are clamped to it (their sums are not used), so every step issues its
-        // loads without a branch and they overlap the arithmetic
-        const lds_float *tlast = win + (__umul24(wrows - 1, wpitch) + (rx + fu - 2 - wx0));
-        Raw F0 = 0;
-        float gx0 = 0.0f, gy0 = 0.0f;
-        if (r0 < rb) ref_raw(o, F0, gx0, gy0);
-#pragma unroll 1
-        for (int r = r0; r < rb; r += 2) {
-          const lds_float *t4 = t + 6 * wpitch, *t5 = t + 7 * wpitch;
-          t4 = t4 > tlast ? tlast : t4;
-          t5 = t5 > tlast ? tlast : t5;
-          float a[6], b[6];
-#pragma unroll
-          for (int k = 0; k < 6; ++k) {
-            a[k] = t4[k];
-            b[k] = t5[k];
-          }
-          Raw F1 = 0;
-          float gx1 = 0.0f, gy1 = 0.0f;
-          if (r + 2 < rb) ref_raw(o + ostep, F1, gx1, gy1);
-          float vv = h0 * wyu[0];
-          vv = fmaf(h1, wyu[1], vv);
-          vv = fmaf(h2, wyu[2], vv);
-          vv = fmaf(h3, wyu[3], vv);
-          vv = fmaf(h4, wyu[4], vv);
-          vv = fmaf(h5, wyu[5], vv);
-          unc_terms(u, v, gx0, gy0, vv - (float)F0, *e - (float)F0, pt);
-          F0 = F1;
-          gx0 = gx1;
-          gy0 = gy1;
-          o += ostep;
-          e += tstep;
-          t += tstep;
-          h0 = h2;
-          h1 = h3;
-          h2 = h4;
-          h3 = h5;
-          h4 = rowsum(a);
-          h5 = rowsum(b);
-        }
-      }
-    };
-    if constexpr (PIXEL) {
-      if (lane < S) {
-        const int rx = x0 + lane - ref.ox;
-#pragma unroll 1
-        for (int r = ra; r < rb; ++r) {
-          const int ry = y0 + r - ref.oy;
-          pixel(ry * ref.w + rx, keys_single(win, wpitch, wx0, wy0, (float)rx + u, (float)ry + v),
-                win + (__umul24(ry - wy0, wpitch) + (rx - wx0)));
-        }
-      }
-      unc_record(pt, u, v, fields, nsub, gid);
-      return true;
-    }
-    const int nfull = S >> 5;
-#pragma unroll 1
-    for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), ra + (lane >> 5));
-    const int R = S & 31;
-    if (R) {
-      // the last columns R at a time, 64 / R rows per step (row-major, so that
-      // the reference loads of a half-wave stay in few cache lines)
-      const int per = kWave / R, rows = per * kNW;
-      int lr = (int)(((float)lane + 0.5f) / (float)R);
-      const int lc = lane - lr * R;
-      if (lr < per) {
-        lr += per * w;
-        const int rx = x0 + (nfull << 5) + lc - ref.ox, ry0 = y0 + lr - ref.oy;
+    // near: the unshifted deformed pixel (rx, ry) at e in the window; else from the image, 0 past the last
+    // interpolated row and column, as in uncertainty()
+    auto walk = [&](auto near) {
+      auto unshifted = [&](const lds_float *e, int rx, int ry) -> float {
+        if constexpr (decltype(near)::value) return *e;
+        return rx <= def.w - 2 && ry <= def.h - 2 ? Pix<T>::at_u(def.pix, (unsigned)(ry * def.w + rx)) : 0.0f;
+      };
+      auto pixel = [&](int o, float interp, const lds_float *e, int rx, int ry) {
+        float refv, gx, gy;
+        ref_at(o, refv, gx, gy);
+        unc_terms(u, v, gx, gy, interp - refv, unshifted(e, rx, ry) - refv, pt);
+      };
+      auto column = [&](int x, int r0) {
+        if (kNW > 1 && r0 >= rb) return;
+        constexpr int step = 2;
+        const int rx = x - ref.ox, ry0 = y0 + r0 - ref.oy;
         int o = ry0 * ref.w + rx;
+        const int ostep = step * ref.w;
+        // taps of (rx + u, ry + v): window rows ry + fv - 2 .. + 3, columns rx + fu - 2 .. + 3
         const lds_float *t = win + (__umul24(ry0 + fv - 2 - wy0, wpitch) + (rx + fu - 2 - wx0));
         const lds_float *e = win + (__umul24(ry0 - wy0, wpitch) + (rx - wx0));
-        const int ostep = rows * ref.w, tstep = rows * wpitch;
+        const int tstep = step * wpitch;
+        {
+          float h0 = rowsum(t), h1 = rowsum(t + wpitch), h2 = rowsum(t + 2 * wpitch), h3 = rowsum(t + 3 * wpitch),
+                h4 = rowsum(t + 4 * wpitch), h5 = rowsum(t + 5 * wpitch);
+          // this column in the last row of the window: the rows read ahead at the last step
+          // are clamped to it (their sums are not used), so every step issues its
+          // loads without a branch and they overlap the arithmetic
+          const lds_float *tlast = win + (__umul24(wrows - 1, wpitch) + (rx + fu - 2 - wx0));
+          Raw F0 = 0;
+          float gx0 = 0.0f, gy0 = 0.0f;
+          if (r0 < rb) ref_raw(o, F0, gx0, gy0);
 #pragma unroll 1
-        for (int r = lr; r < S; r += rows) {
-          pixel(o, keys_sum(t, wpitch, wxu, wyu), e);
-          o += ostep;
-          e += tstep;
-          t += tstep;
+          for (int r = r0; r < rb; r += 2) {
+            const lds_float *t4 = t + 6 * wpitch, *t5 = t + 7 * wpitch;
+            t4 = t4 > tlast ? tlast : t4;
+            t5 = t5 > tlast ? tlast : t5;
+            float a[6], b[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+              a[k] = t4[k];
+              b[k] = t5[k];
+            }
+            Raw F1 = 0;
+            float gx1 = 0.0f, gy1 = 0.0f;
+            if (r + 2 < rb) ref_raw(o + ostep, F1, gx1, gy1);
+            float vv = h0 * wyu[0];
+            vv = fmaf(h1, wyu[1], vv);
+            vv = fmaf(h2, wyu[2], vv);
+            vv = fmaf(h3, wyu[3], vv);
+            vv = fmaf(h4, wyu[4], vv);
+            vv = fmaf(h5, wyu[5], vv);
+            unc_terms(u, v, gx0, gy0, vv - (float)F0, unshifted(e, rx, y0 + r - ref.oy) - (float)F0, pt);
+            F0 = F1;
+            gx0 = gx1;
+            gy0 = gy1;
+            o += ostep;
+            e += tstep;
+            t += tstep;
+            h0 = h2;
+            h1 = h3;
+            h2 = h4;
+            h3 = h5;
+            h4 = rowsum(a);
+            h5 = rowsum(b);
+          }
+        }
+      };
+      if constexpr (PIXEL) {
+        if (lane < S) {
+          const int rx = x0 + lane - ref.ox;
+#pragma unroll 1
+          for (int r = ra; r < rb; ++r) {
+            const int ry = y0 + r - ref.oy;
+            pixel(ry * ref.w + rx, keys_single(win, wpitch, wx0, wy0, (float)rx + u, (float)ry + v),
+                  win + (__umul24(ry - wy0, wpitch) + (rx - wx0)), rx, ry);
+          }
+        }
+        return;
+      }
+      const int nfull = S >> 5;
+#pragma unroll 1
+      for (int st = 0; st < nfull; ++st) column(x0 + (st << 5) + (lane & 31), ra + (lane >> 5));
+      const int R = S & 31;
+      if (R) {
+        // the last columns R at a time, 64 / R rows per step (row-major, so that
+        // the reference loads of a half-wave stay in few cache lines)
+        const int per = kWave / R, rows = per * kNW;
+        int lr = (int)(((float)lane + 0.5f) / (float)R);
+        const int lc = lane - lr * R;
+        if (lr < per) {
+          lr += per * w;
+          const int rx = x0 + (nfull << 5) + lc - ref.ox, ry0 = y0 + lr - ref.oy;
+          int o = ry0 * ref.w + rx;
+          const lds_float *t = win + (__umul24(ry0 + fv - 2 - wy0, wpitch) + (rx + fu - 2 - wx0));
+          const lds_float *e = win + (__umul24(ry0 - wy0, wpitch) + (rx - wx0));
+          const int ostep = rows * ref.w, tstep = rows * wpitch;
+#pragma unroll 1
+          for (int r = lr; r < S; r += rows) {
+            pixel(o, keys_sum(t, wpitch, wxu, wyu), e, rx, y0 + r - ref.oy);
+            o += ostep;
+            e += tstep;
+            t += tstep;
+          }
         }
       }
-    }
+    };
+    if (!FAR || e_in_win) walk(std::true_type{});
+    else if constexpr (FAR) walk(std::false_type{});
     unc_record(pt, u, v, fields, nsub, gid);
     return true;
   }
@@ -2862,7 +2878,7 @@ struct Solver {
           const int ww = min(bx1 - ref.ox + fu + 4, def.w - 1) - max(bx0 - ref.ox + fu - 3, 0) + 1;
           const int hh = min(by1 - ref.oy + fv + 4, def.h - 1) - max(by0 - ref.oy + fv - 3, 0) + 1;
           if (ww > 0 && hh > 0 && ww * hh > win_cap) return kOverflow;
-          if (!lean_uncertainty<INTERP == 0>(A, fields, nsub, gid)) return kOverflow;
+          if (!lean_uncertainty<INTERP == 0, true>(A, fields, nsub, gid)) return kOverflow;
         }
         break;
       }

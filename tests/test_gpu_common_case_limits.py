@@ -55,3 +55,32 @@ def test_widest_subsets(S, interp):
         a = run(ctx, p, ref, de, cx, cy, S, f0)
         b = run(ctx, q, ref, de, cx, cy, S, f0)
     check(a, b)
+
+
+@pytest.mark.parametrize("step", [6, 45], ids=["wave", "crew"])
+@pytest.mark.parametrize("interp", [dh.KEYS_FOURTH, dh.BILINEAR], ids=["keys", "bilinear"])
+@pytest.mark.parametrize("u,v", [(7.3, -3.6), (-9.4, 12.2), (0.2, -6.7)])
+def test_large_motion(u, v, interp, step):
+    """A translation of more than 5 px: the unshifted subset lies outside the window that the uncertainty fields
+    are formed from (in places in the image's last columns and rows, which count as 0 there), and the kernels
+    still finish every subset themselves."""
+    w, h, S = 340, 320, 35
+    ref, de = images(w, h, u, v, 53)
+
+    def centres(size, d):  # up to the border that the motion leads away from
+        return np.arange(S // 2 + max(0, int(7 - d)), size - S // 2 - max(0, int(d + 7)), step)
+
+    gx, gy = np.meshgrid(centres(w, u), centres(h, v)[::-1])
+    gx[:, -1] = w - 1 - S // 2 - max(0, int(u + 7))
+    gy[0] = h - 1 - S // 2 - max(0, int(v + 7))
+    cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
+    assert (len(cx) > 1024) == (step == 6)
+    f0 = dh.new_fields(cx, cy)
+    f0[dh.F["DISP_X"]], f0[dh.F["DISP_Y"]] = round(u), round(v)
+    p, q = params(interp), params(interp)
+    q.initial_gamma_threshold = 1e9  # the general kernel
+    with dh.Context(0) as ctx:
+        a = run(ctx, p, ref, de, cx, cy, S, f0)
+        assert ctx.pass_counts()[1] == 0 and ctx.handover_counts() == (0, 0, 0)
+        b = run(ctx, q, ref, de, cx, cy, S, f0)
+    check(a, b)
