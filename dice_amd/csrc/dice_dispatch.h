@@ -42,15 +42,38 @@ constexpr int trans_lds_floats(int S, int slot, bool crew) {
 
 enum class CommonKernel { kNone, kLean, kTrans, kCrew };
 
-// The kernel for n subsets of size S, all six parameters (affine) or translation
-// only, with slot floats of LDS per wave.  All six parameters: the lean kernel;
-// translation only: its own kernel; few subsets of either kind: four waves each.
-inline CommonKernel common_kernel(int n, int S, bool affine, int slot) {
+// What the choice depends on.
+struct CommonPass {
+  int n, S;          // subsets and their size
+  bool affine;       // all six parameters, or translation only
+  int slot;          // LDS floats per wave
+  bool keys;         // Keys fourth-order interpolation, or bilinear
+  bool uncertainty;  // the uncertainty fields are formed
+};
+
+// Can a subset that is translated by a fraction of a pixel be finished in the
+// slot?  The solve stages the side and its taps (5 px more, bilinear 1), the
+// uncertainty fields the Keys taps (5), in the translation kernels with the
+// margin that the general kernel's test has (7).  Where they do not fit, every
+// subset would be set up there only to be handed over: 14,910 subsets of 43 x 43
+// (default parameters) 2.71 ms with that launch, 2.34 ms without.
+inline bool common_window_fits(const CommonPass &p) {
+  const int taps = p.keys ? 5 : 1, unc = p.affine ? 5 : 7;
+  const long long w = square_side(p.S) + (p.uncertainty && unc > taps ? unc : taps);
+  return w * w <= p.slot - kPersistFloats;
+}
+
+// All six parameters: the lean kernel; translation only: its own kernel; few
+// subsets of either kind: four waves each.  (The lean kernel also where a plain
+// translation does not fit: subsets that shrink may.)
+inline CommonKernel common_kernel(const CommonPass &p) {
+  const bool window = common_window_fits(p);
   auto fits = [&](bool crew) {
-    return square_side(S) <= kTransMaxSide && trans_lds_floats(S, slot, crew) * sizeof(float) <= kMaxLaunchLds;
+    return window && square_side(p.S) <= kTransMaxSide &&
+           trans_lds_floats(p.S, p.slot, crew) * sizeof(float) <= kMaxLaunchLds;
   };
-  if (n <= kCrewMaxSubsets && fits(true)) return CommonKernel::kCrew;
-  if (affine) return CommonKernel::kLean;
+  if (p.n <= kCrewMaxSubsets && fits(true)) return CommonKernel::kCrew;
+  if (p.affine) return CommonKernel::kLean;
   return fits(false) ? CommonKernel::kTrans : CommonKernel::kNone;
 }
 

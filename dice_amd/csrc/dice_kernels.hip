@@ -742,7 +742,8 @@ static hipError_t launch_pass(bool simplex, int storage, const Launch &L, const 
       pl.counter = work + kWorkSetLean * kWorkCounterInts;
       pl.ov_list = other;
       pl.ov_count = work + kWorkLeanCount;
-      const CommonKernel common = common_kernel(subs.n, subs.S, np == 3, L.lds_floats_per_wave);
+      const CommonKernel common = common_kernel(
+          CommonPass{subs.n, subs.S, np == 3, L.lds_floats_per_wave, kp.interp != 0, kp.uncertainty != 0});
       e = hipSuccess;
       if (common == CommonKernel::kCrew)
         e = launch_gn_crew(storage, kp.interp, np == 0, L, kp, ref, def, subs, fields, pl, stream);

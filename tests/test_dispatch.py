@@ -25,15 +25,33 @@ def rule(tmp_path_factory):
 
 
 def sweep(ns=(1, 255, 1024, 1025, 5000), sizes=range(1, 100), slots=(2560, 2704, 2812, 5184, 6400, 16000)):
-    return [(n, S, affine, slot) for n in ns for S in sizes for affine in (0, 1) for slot in slots]
+    return [(n, S, affine, slot, keys, unc) for n in ns for S in sizes for affine in (0, 1) for slot in slots
+            for keys in (0, 1) for unc in (0, 1)]
 
 
 def test_the_translation_kernels_have_a_lane_per_column(rule):
     """A subset of even size S is S + 1 pixels wide: size 64 has 65 columns, one more than a wave has lanes."""
     rows = sweep()
-    for (n, S, affine, slot), (kernel, wave_lds, crew_lds) in zip(rows, rule(rows)):
+    for (n, S, affine, slot, _, _), (kernel, wave_lds, crew_lds) in zip(rows, rule(rows)):
         if kernel in (TRANS, CREW):
             assert S // 2 * 2 + 1 <= 64, (n, S, affine, slot)
             assert (crew_lds if kernel == CREW else wave_lds) <= 62 * 1024, (n, S, affine, slot)
         assert kernel != TRANS or not affine, (n, S, affine, slot)
         assert kernel != LEAN or affine, (n, S, affine, slot)
+
+
+def test_no_launch_whose_subsets_are_all_handed_over(rule):
+    """The window of a subset at a translation of (0.5, 0.5) px and, with uncertainty fields, the general kernel's
+    window of them (3 px before and 4 px after the box), counted pixel by pixel, against the slot less the
+    per-subset constants (104 floats)."""
+    rows = sweep()
+    for (n, S, affine, slot, keys, unc), (kernel, _, _) in zip(rows, rule(rows)):
+        h = S // 2
+        need = np.floor(h + 0.5) + (3 if keys else 1) - (np.floor(-h + 0.5) - (2 if keys else 0)) + 1
+        if unc:
+            need = max(need, 2 * h + (6 if affine else 8))
+        fits = need ** 2 <= slot - 104
+        if kernel in (TRANS, CREW):
+            assert fits, (n, S, affine, slot, keys, unc)
+        if not affine and fits and S <= 41 and n > 1024:
+            assert kernel == TRANS, (n, S, affine, slot, keys, unc)
