@@ -4905,7 +4905,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_W
   }
 }
 
-// The same two passes with at most kCrewMaxSubsets subsets: four waves per
+// The same two passes with few subsets (crew_max_subsets): four waves per
 // subset.  One wave each leaves most SIMDs idle and the frame takes a subset's
 // whole latency: 49 subsets of 27 x 27, 87 us in the general kernel, 32 here.
 // With 2,116 subsets of 31 x 31 every SIMD has two waves of its own and the lean

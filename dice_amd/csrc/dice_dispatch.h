@@ -14,7 +14,6 @@ constexpr int kPersistFloats = 104;
 
 // The most dynamic LDS that the kernels below are launched with.
 constexpr size_t kMaxLaunchLds = 64 * 1024 - 2048;
-constexpr int kCrewMaxSubsets = 1024;
 // correlate_trans_kernel and its crew hold a column of the subset per lane.
 constexpr int kTransMaxSide = 64;
 // rows after which the translation walk's six row sums are back in their places
@@ -49,6 +48,8 @@ struct CommonPass {
   int slot;          // LDS floats per wave
   bool keys;         // Keys fourth-order interpolation, or bilinear
   bool uncertainty;  // the uncertainty fields are formed
+  bool listed;       // a part of the subsets, from a list (rounds of neighbour initialization)
+  int num_cus;
 };
 
 // Can a subset that is translated by a fraction of a pixel be finished in the
@@ -63,6 +64,20 @@ inline bool common_window_fits(const CommonPass &p) {
   return w * w <= p.slot - kPersistFloats;
 }
 
+// The most subsets that a crew of four waves each is taken for.  A CU holds three
+// crews at a time, and the lean kernel, with four waves per SIMD, takes a
+// wave's latency for all that fit: 768 six-parameter subsets of 21 x 21, 31 x 31
+// and 43 x 43 take 71, 78 and 111 us there and 65, 69 and 86 us in crews, 1,024
+// of them 71, 80 and 114 us against 84, 94 and 118 us.  Small subsets give a crew
+// little to share: 9 x 9 px, 256 subsets 102 against 94 us, 384 104 against 108 us;
+// 11 x 11 px, 300 subsets 109 against 101 us, 768 110 against 109 us.
+// With translation only the kernel for many subsets has the longer wave: crews
+// win up to 1,024 at 9 to 41 px.  A list holds few of its subsets.
+inline int crew_max_subsets(const CommonPass &p) {
+  if (!p.affine || p.listed) return 4 * p.num_cus;
+  return (square_side(p.S) >= 11 ? 3 : 1) * p.num_cus;
+}
+
 // All six parameters: the lean kernel; translation only: its own kernel; few
 // subsets of either kind: four waves each.  (The lean kernel also where a plain
 // translation does not fit: subsets that shrink may.)
@@ -72,7 +87,7 @@ inline CommonKernel common_kernel(const CommonPass &p) {
     return window && square_side(p.S) <= kTransMaxSide &&
            trans_lds_floats(p.S, p.slot, crew) * sizeof(float) <= kMaxLaunchLds;
   };
-  if (p.n <= kCrewMaxSubsets && fits(true)) return CommonKernel::kCrew;
+  if (p.n <= crew_max_subsets(p) && fits(true)) return CommonKernel::kCrew;
   if (p.affine) return CommonKernel::kLean;
   return fits(false) ? CommonKernel::kTrans : CommonKernel::kNone;
 }

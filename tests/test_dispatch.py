@@ -25,14 +25,14 @@ def rule(tmp_path_factory):
 
 
 def sweep(ns=(1, 255, 1024, 1025, 5000), sizes=range(1, 100), slots=(2560, 2704, 2812, 5184, 6400, 16000)):
-    return [(n, S, affine, slot, keys, unc) for n in ns for S in sizes for affine in (0, 1) for slot in slots
-            for keys in (0, 1) for unc in (0, 1)]
+    return [(n, S, affine, slot, keys, unc, listed) for n in ns for S in sizes for affine in (0, 1) for slot in slots
+            for keys in (0, 1) for unc in (0, 1) for listed in (0, 1)]
 
 
 def test_the_translation_kernels_have_a_lane_per_column(rule):
     """A subset of even size S is S + 1 pixels wide: size 64 has 65 columns, one more than a wave has lanes."""
     rows = sweep()
-    for (n, S, affine, slot, _, _), (kernel, wave_lds, crew_lds) in zip(rows, rule(rows)):
+    for (n, S, affine, slot, *_), (kernel, wave_lds, crew_lds) in zip(rows, rule(rows)):
         if kernel in (TRANS, CREW):
             assert S // 2 * 2 + 1 <= 64, (n, S, affine, slot)
             assert (crew_lds if kernel == CREW else wave_lds) <= 62 * 1024, (n, S, affine, slot)
@@ -45,7 +45,7 @@ def test_no_launch_whose_subsets_are_all_handed_over(rule):
     window of them (3 px before and 4 px after the box), counted pixel by pixel, against the slot less the
     per-subset constants (104 floats)."""
     rows = sweep()
-    for (n, S, affine, slot, keys, unc), (kernel, _, _) in zip(rows, rule(rows)):
+    for (n, S, affine, slot, keys, unc, _), (kernel, _, _) in zip(rows, rule(rows)):
         h = S // 2
         need = np.floor(h + 0.5) + (3 if keys else 1) - (np.floor(-h + 0.5) - (2 if keys else 0)) + 1
         if unc:
@@ -55,3 +55,14 @@ def test_no_launch_whose_subsets_are_all_handed_over(rule):
             assert fits, (n, S, affine, slot, keys, unc)
         if not affine and fits and S <= 41 and n > 1024:
             assert kernel == TRANS, (n, S, affine, slot, keys, unc)
+
+
+@pytest.mark.parametrize("S,affine,listed,most", [(8, 1, 0, 256), (9, 1, 0, 256), (10, 1, 0, 768), (31, 1, 0, 768),
+                                                  (41, 1, 0, 768), (9, 1, 1, 1024), (31, 1, 1, 1024),
+                                                  (9, 0, 0, 1024), (41, 0, 0, 1024), (31, 0, 1, 1024)])
+def test_number_of_subsets_that_crews_take(rule, S, affine, listed, most):
+    """One crew per CU (of 256) for small six-parameter subsets, three for larger ones, four for translation only
+    and for lists."""
+    rows = [(n, S, affine, 2560, 1, 1, listed) for n in (1, most, most + 1, 1 << 17)]
+    many = LEAN if affine else TRANS
+    assert rule(rows)[:, 0].tolist() == [CREW, CREW, many, many]
