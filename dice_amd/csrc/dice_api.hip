@@ -123,6 +123,7 @@ struct dice_hip_context {
   // largest and 90th-percentile bounding-box side of the subsets (S for square subsets): the
   // autotuner sizes its LDS window candidates from them
   int max_side = 0, p90_side = 0;
+  int cx_lo = 0, cx_hi = 0, cy_lo = 0, cy_hi = 0;  // extremes of the centres
   int max_count = 0;  // most pixels in one subset
   DevBuf cx, cy, off, px, py, act, bbox, nact, pxy, abox;
   DevBuf order;         // conformal: the work order (Morton order of the centres)
@@ -304,6 +305,9 @@ Launch current_launch(dice_hip_context *ctx, int mode) {
   // square subsets whose window would outgrow a wave's slot even compressed by a fifth
   const long long small = (long long)(0.8 * ctx->S) + 1;
   L.wide_only = ctx->S > 0 && small * small > L.lds_floats_per_wave ? 1 : 0;
+  const int hw = ctx->S / 2;
+  L.border = ctx->S > 0 && (dice_hip::reaches_border(ctx->cx_lo, ctx->cx_hi, hw, ctx->dox, ctx->dw) ||
+                            dice_hip::reaches_border(ctx->cy_lo, ctx->cy_hi, hw, ctx->doy, ctx->dh));
   L.lane_simplex = ctx->max_count <= dice_hip::kLaneSimplexMaxPixels ? std::max(ctx->max_count, 1) : 0;
   return L;
 }
@@ -582,6 +586,11 @@ int dice_hip_set_subsets(dice_hip_context *ctx, int n, const double *coord_x, co
   if (!conf_offsets) {
     ctx->S = subset_size;
     ctx->max_side = ctx->p90_side = subset_size;
+    const auto ex = std::minmax_element(hx.begin(), hx.end()), ey = std::minmax_element(hy.begin(), hy.end());
+    ctx->cx_lo = *ex.first;
+    ctx->cx_hi = *ex.second;
+    ctx->cy_lo = *ey.first;
+    ctx->cy_hi = *ey.second;
     ctx->max_count = (2 * (subset_size / 2) + 1) * (2 * (subset_size / 2) + 1);
   } else {
     if (!conf_x || !conf_y) return ctx->fail(DICE_HIP_EINVAL, "conformal subsets need pixel lists");

@@ -49,8 +49,16 @@ struct CommonPass {
   bool keys;         // Keys fourth-order interpolation, or bilinear
   bool uncertainty;  // the uncertainty fields are formed
   bool listed;       // a part of the subsets, from a list (rounds of neighbour initialization)
+  bool border;       // a subset's box reaches the pixels that are dropped at the image border
   int num_cus;
 };
+
+// Does a box of centres [x0, x1] with half width hw reach the 4 px along the
+// border of an image of w pixels whose first has coordinate o, where warped
+// pixels are dropped?
+constexpr bool reaches_border(int x0, int x1, int hw, int o, int w) {
+  return (long long)x0 - hw < (long long)o + 4 || (long long)x1 + hw >= (long long)o + w - 4;
+}
 
 // Can a subset that is translated by a fraction of a pixel be finished in the
 // slot?  The solve stages the side and its taps (5 px more, bilinear 1), the
@@ -78,10 +86,25 @@ inline int crew_max_subsets(const CommonPass &p) {
   return (square_side(p.S) >= 11 ? 3 : 1) * p.num_cus;
 }
 
+// Translation only, subsets at the border: they lose pixels, need many steps and
+// go to the general kernel, whose launch then takes at least a subset's time
+// after the translation kernel's, while the general kernel alone works on them
+// beside the others.  That is the faster way up to about 20 subsets per CU with
+// Keys and 40 with bilinear interpolation: a full grid of 35 x 35 px (8 bits), 961
+// subsets 175 against 232 us, 3,969 271 against 308, 5,929 361 against 340;
+// bilinear 3,969 221 against 300, 10,000 604 against 669, 12,100 488 against 468.
+// A round of neighbour initialization has a few subsets, mostly inside (324 points
+// of 27 x 27 px: none at the border 3.97 ms in the general kernel and 2.46 ms in
+// crews, one column of them 4.36 and 3.65 ms, all four sides 4.00 and 4.57 ms).
+inline bool general_for_border(const CommonPass &p) {
+  return p.border && !p.affine && !p.listed && p.n <= (p.keys ? 20 : 40) * p.num_cus;
+}
+
 // All six parameters: the lean kernel; translation only: its own kernel; few
 // subsets of either kind: four waves each.  (The lean kernel also where a plain
 // translation does not fit: subsets that shrink may.)
 inline CommonKernel common_kernel(const CommonPass &p) {
+  if (general_for_border(p)) return CommonKernel::kNone;
   const bool window = common_window_fits(p);
   auto fits = [&](bool crew) {
     return window && square_side(p.S) <= kTransMaxSide &&

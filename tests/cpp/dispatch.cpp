@@ -1,14 +1,23 @@
-// Reads "n S affine slot keys uncertainty listed" lines and, for 256 CUs, prints the kernel that common_kernel (dice_dispatch.h) names for each
+// Reads "n S affine slot keys uncertainty listed border" lines and, for 256 CUs, prints the kernel that common_kernel (dice_dispatch.h) names for each
 // (0 none, 1 lean, 2 translation, 3 crew) and the dynamic LDS bytes of the translation and crew launches.
 #include <cstdio>
 
 #include "../../dice_amd/csrc/dice_dispatch.h"
 
+using dice_hip::reaches_border;
+static_assert(!reaches_border(21, 78, 17, 0, 100) && reaches_border(20, 50, 17, 0, 100) &&
+                  reaches_border(50, 79, 17, 0, 100),
+              "a box from 4 to 95 of 100 pixels keeps them all");
+static_assert(!reaches_border(71, 128, 17, 50, 100) && reaches_border(21, 78, 17, 50, 100) &&
+                  reaches_border(70, 71, 17, 50, 100) && reaches_border(128, 129, 17, 50, 100),
+              "the same in an image that begins at 50");
+
 int main() {
-  int n, S, affine, slot, keys, unc, listed;
-  while (std::scanf("%d %d %d %d %d %d %d", &n, &S, &affine, &slot, &keys, &unc, &listed) == 7)
+  int n, S, affine, slot, keys, unc, listed, border;
+  while (std::scanf("%d %d %d %d %d %d %d %d", &n, &S, &affine, &slot, &keys, &unc, &listed, &border) == 8)
     std::printf("%d %zu %zu\n",
-                (int)dice_hip::common_kernel({n, S, affine != 0, slot, keys != 0, unc != 0, listed != 0, 256}),
+                (int)dice_hip::common_kernel(
+                    {n, S, affine != 0, slot, keys != 0, unc != 0, listed != 0, border != 0, 256}),
                 sizeof(float) * dice_hip::trans_lds_floats(S, slot, false),
                 sizeof(float) * dice_hip::trans_lds_floats(S, slot, true));
   return 0;

@@ -25,7 +25,7 @@ def rule(tmp_path_factory):
 
 
 def sweep(ns=(1, 255, 1024, 1025, 5000), sizes=range(1, 100), slots=(2560, 2704, 2812, 5184, 6400, 16000)):
-    return [(n, S, affine, slot, keys, unc, listed) for n in ns for S in sizes for affine in (0, 1) for slot in slots
+    return [(n, S, affine, slot, keys, unc, listed, 0) for n in ns for S in sizes for affine in (0, 1) for slot in slots
             for keys in (0, 1) for unc in (0, 1) for listed in (0, 1)]
 
 
@@ -45,7 +45,7 @@ def test_no_launch_whose_subsets_are_all_handed_over(rule):
     window of them (3 px before and 4 px after the box), counted pixel by pixel, against the slot less the
     per-subset constants (104 floats)."""
     rows = sweep()
-    for (n, S, affine, slot, keys, unc, _), (kernel, _, _) in zip(rows, rule(rows)):
+    for (n, S, affine, slot, keys, unc, *_), (kernel, _, _) in zip(rows, rule(rows)):
         h = S // 2
         need = np.floor(h + 0.5) + (3 if keys else 1) - (np.floor(-h + 0.5) - (2 if keys else 0)) + 1
         if unc:
@@ -63,6 +63,18 @@ def test_no_launch_whose_subsets_are_all_handed_over(rule):
 def test_number_of_subsets_that_crews_take(rule, S, affine, listed, most):
     """One crew per CU (of 256) for small six-parameter subsets, three for larger ones, four for translation only
     and for lists."""
-    rows = [(n, S, affine, 2560, 1, 1, listed) for n in (1, most, most + 1, 1 << 17)]
+    rows = [(n, S, affine, 2560, 1, 1, listed, 0) for n in (1, most, most + 1, 1 << 17)]
     many = LEAN if affine else TRANS
     assert rule(rows)[:, 0].tolist() == [CREW, CREW, many, many]
+
+
+@pytest.mark.parametrize("keys,most", [(1, 5120), (0, 10240)])
+def test_border_subsets_of_small_frames_stay_with_the_others(rule, keys, most):
+    """Translation only with a subset at the border: the general kernel takes the whole frame up to a size; lists and
+    six-parameter frames (whose lean kernel there always was) as without one."""
+    for S in (9, 35, 41):
+        rows = [(n, S, 0, 2560, keys, 1, 0, 1) for n in (1, 1024, 1025, most, most + 1)]
+        assert rule(rows)[:, 0].tolist() == [NONE] * 4 + [TRANS]
+        for affine, listed in ((1, 0), (0, 1), (1, 1)):
+            rows = [[(n, S, affine, 2560, keys, 1, listed, border) for n in (1, 300, 5000)] for border in (0, 1)]
+            assert np.array_equal(rule(rows[0]), rule(rows[1])) and (rule(rows[1])[:, 0] != NONE).all()

@@ -4,7 +4,8 @@ import pytest
 
 import dice_amd as dh
 from dice_amd import synth
-from test_gpu_common_case import CLOSE, EXACT
+import test_gpu_common_case as common
+from test_gpu_common_case import CLOSE, EXACT, scene  # noqa: F401 (scene: the fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -57,24 +58,84 @@ def test_widest_subsets(S, interp):
     check(a, b)
 
 
-@pytest.mark.parametrize("step", [6, 45], ids=["wave", "crew"])
+@pytest.mark.parametrize("S,interp,dtype", [(5, dh.KEYS_FOURTH, np.float32), (31, dh.KEYS_FOURTH, np.uint16),
+                                            (33, dh.BILINEAR, np.float32), (37, dh.KEYS_FOURTH, np.float32),
+                                            (41, dh.KEYS_FOURTH, np.float32), (41, dh.BILINEAR, np.uint16)])
+def test_inside(scene, S, interp, dtype):
+    """Translation only, all subsets inside the image: one wave per subset, crews and the general kernel."""
+    ctx, ref, de = scene
+    if dtype == np.uint16:
+        ref, de = [np.clip(np.round(np.maximum(i, 0) * 16), 0, 4095).astype(np.uint16) for i in (ref, de)]
+    c = S // 2 + 6
+    gx, gy = np.meshgrid(np.arange(c, common.W - c, 9), np.arange(c, common.H - c, 9))
+    cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
+    assert len(cx) > 1024
+    p, q = params(interp), params(interp)
+    q.initial_gamma_threshold = 1e9  # the general kernel
+    wave = common.run(ctx, p, ref, de, cx, cy, S)
+    finished = ctx.handover_counts()[0] < 0.05 * len(cx)
+    few = np.arange(0, len(cx), 15)  # 15: the start values, which depend on the index, are those of the whole set
+    crew = common.run(ctx, p, ref, de, cx[few], cy[few], S)
+    general = common.run(ctx, q, ref, de, cx, cy, S)
+    keep = (np.arange(len(few)) % 3 == 0) & (np.arange(len(few)) % 5 == 0)
+    common.same(wave[:, few][:, keep], crew[:, keep])
+    ok = general[dh.F["STATUS"]] != 5
+    common.same(wave[:, ok], general[:, ok])
+    assert finished
+
+
+@pytest.mark.parametrize("S,interp,step", [(21, dh.KEYS_FOURTH, 4), (35, dh.KEYS_FOURTH, 4), (35, dh.BILINEAR, 3)])
+def test_border_of_a_large_frame(scene, S, interp, step):
+    """Enough subsets for the translation kernel although some reach the border, which it hands over."""
+    ctx, ref, de = scene
+    c = S // 2
+    gx, gy = np.meshgrid(np.arange(c, common.W - c, step), np.arange(c, common.H - c, step))
+    cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
+    assert len(cx) > (5120 if interp == dh.KEYS_FOURTH else 10240)
+    p, q = params(interp), params(interp)
+    q.initial_gamma_threshold = 1e9
+    a = common.run(ctx, p, ref, de, cx, cy, S)
+    assert 0 < ctx.handover_counts()[0] < 0.2 * len(cx)
+    general = common.run(ctx, q, ref, de, cx, cy, S)
+    ok = general[dh.F["STATUS"]] != 5
+    common.same(a[:, ok], general[:, ok])
+
+
+def test_border_of_a_small_frame(scene):
+    """Few subsets, some at the border: the general kernel takes them all."""
+    ctx, ref, de = scene
+    S = 21
+    gx, gy = np.meshgrid(np.arange(10, common.W - 10, 23), np.arange(10, common.H - 10, 23))
+    cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
+    p, q = params(), params()
+    q.initial_gamma_threshold = 1e9
+    a = common.run(ctx, p, ref, de, cx, cy, S)
+    assert ctx.handover_counts() == (0, 0, 0)
+    general = common.run(ctx, q, ref, de, cx, cy, S)
+    ok = general[dh.F["STATUS"]] != 5
+    for name in EXACT + CLOSE:
+        assert np.array_equal(a[dh.F[name]][ok], general[dh.F[name]][ok]), name
+
+
+@pytest.mark.parametrize("step", [3, 45], ids=["wave", "crew"])
 @pytest.mark.parametrize("interp", [dh.KEYS_FOURTH, dh.BILINEAR], ids=["keys", "bilinear"])
 @pytest.mark.parametrize("u,v", [(7.3, -3.6), (-9.4, 12.2), (0.2, -6.7)])
 def test_large_motion(u, v, interp, step):
     """A translation of more than 5 px: the unshifted subset lies outside the window that the uncertainty fields
     are formed from (in places in the image's last columns and rows, which count as 0 there), and the kernels
     still finish every subset themselves."""
-    w, h, S = 340, 320, 35
+    w, h, S = (340, 320, 35) if interp == dh.KEYS_FOURTH else (420, 400, 35)
     ref, de = images(w, h, u, v, 53)
 
-    def centres(size, d):  # up to the border that the motion leads away from
-        return np.arange(S // 2 + max(0, int(7 - d)), size - S // 2 - max(0, int(d + 7)), step)
+    edge = 0 if step == 3 else 4  # crews: clear of the border before the motion too
 
-    gx, gy = np.meshgrid(centres(w, u), centres(h, v)[::-1])
-    gx[:, -1] = w - 1 - S // 2 - max(0, int(u + 7))
-    gy[0] = h - 1 - S // 2 - max(0, int(v + 7))
+    def centres(size, d):  # up to the border that the motion leads away from
+        lo, hi = S // 2 + max(edge, int(7 - d)), size - 1 - S // 2 - max(edge, int(d + 7))
+        return np.append(np.arange(lo, hi, step), hi)
+
+    gx, gy = np.meshgrid(centres(w, u), centres(h, v))
     cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
-    assert (len(cx) > 1024) == (step == 6)
+    assert len(cx) > 5120 if step == 3 else len(cx) <= 1024
     f0 = dh.new_fields(cx, cy)
     f0[dh.F["DISP_X"]], f0[dh.F["DISP_Y"]] = round(u), round(v)
     p, q = params(interp), params(interp)
@@ -82,5 +143,7 @@ def test_large_motion(u, v, interp, step):
     with dh.Context(0) as ctx:
         a = run(ctx, p, ref, de, cx, cy, S, f0)
         assert ctx.pass_counts()[1] == 0 and ctx.handover_counts() == (0, 0, 0)
+        # (the rule sends a border frame of this size to the translation kernel; crews have none here)
+        assert len(cx) > (5120 if interp == dh.KEYS_FOURTH else 10240) or step == 45
         b = run(ctx, q, ref, de, cx, cy, S, f0)
     check(a, b)
