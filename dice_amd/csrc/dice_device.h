@@ -676,10 +676,6 @@ __device__ __forceinline__ float cond2x2(double h00, double h01, double h10, dou
   return c;
 }
 
-#ifndef DICE_CREW_ADD
-#define DICE_CREW_ADD(gmf, gv, g1, p) ((p) + (g1))
-#endif
-
 // Status of a wave that handed its subset over (never stored in a field).
 constexpr int kOverflow = -1000;
 
@@ -2934,7 +2930,7 @@ struct Solver {
           const int i = (y - y0) * S + (x - x0);
           const float gmf = (gtab[i] - shift) - (rtab[i] - meanF);
           const float gv = g[i], g1 = gmf * gv;
-          p0 = DICE_CREW_ADD(gmf, gv, g1, p0);
+          p0 += g1;
           p1 = fmaf(g1, dx, p1);
           p2 = fmaf(g1, dy, p2);
         });
@@ -4716,9 +4712,9 @@ struct BlockClaims {
 // pa.ov_list for the PLAIN kernel.
 // PLAIN is bound by its taps: 36 scattered loads per pixel and pass through
 // the CU's one texture-address unit.  From LDS the kernel is bound by VALU issue
-// (84 % of the quad-cycles); Gauss-Newton adds PLAIN's 35 products per pixel in
+// (75 % of the quad-cycles); Gauss-Newton adds PLAIN's 35 products per pixel in
 // FP64 and reads the totals from LDS.  (H from the per-subset S, with 7 sums per
-// pixel, is a tenth faster, but moves the last bit of 5-10 % of the parameters.)
+// pixel, moves the last bit of 5-10 % of the parameters.)
 // What Gauss-Newton leaves to PLAIN are the systems that its L D L^T refuses.
 // 2,280 subsets of 75 x 75 (1500 x 1100, six parameters): 1.48 -> 0.48 ms per
 // frame; 8,000 polygons of 200-3000 px, half of them too large for a slot: 1.93 ->
@@ -4727,13 +4723,11 @@ struct BlockClaims {
 // bookkeeping in one wave only.  A Gauss-Newton step is too short for that: 108
 // subsets of 69 x 69 take 177 us with 1,024 threads each and 123 us with 256, and
 // about 240 of 71 x 71 163 and 119 us.  Registers: three waves per SIMD beat two and, with its
-// spills, four (0.48 against 0.59 and 0.53 ms; 0.96 against 1.08 and 0.95 ms for
-// the polygons, measured with an earlier reduction).
-#ifndef DICE_WIDE_WPE
-#define DICE_WIDE_WPE 3
-#endif
+// spills, four (one run: 0.50 against 0.58 and 0.65 ms; 1.02 against 1.14 and
+// 1.12 ms for the polygons).
+constexpr int kWideWaves = 3;
 template <typename T, int INTERP, bool SIMPLEX_OPT, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT > 512 ? 4 : DICE_WIDE_WPE))) void correlate_wide_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT > 512 ? 4 : kWideWaves))) void correlate_wide_kernel(
     KParams kp, DImage ref, DImage def, DSubsets ss, double *fields, PassArgs pa, int cap) {
   extern __shared__ float lds[];
   __shared__ double red[NT / kWave * kTeamRed];
@@ -4863,17 +4857,15 @@ hipError_t launch_lean_variant(const Launch &L, const KParams &kp, const DImage 
   return hipGetLastError();
 }
 
-#ifndef DICE_TRANS_WPE
-#define DICE_TRANS_WPE 3
-#endif
+constexpr int kTransWaves = 3;  // per SIMD
 // BATCHED translation-only Gauss-Newton pass: one wave per subset (and per
 // workgroup), Solver::run_lean<true>.  A wave's LDS: the window, the per-subset
 // constants, then gtab.  27,264 subsets of 35 x 35 (u16): 1.13 ms in the general
 // kernel, 0.59 ms here; 11 k vector instructions per subset (24 k there), issued
-// in 73 % of the quad-cycles with three waves per SIMD.  More waves spill, and
-// fewer hide less: four per SIMD (35 spilled registers) 0.66 ms, two 0.93 ms.
+// in 74 % of the quad-cycles with three waves per SIMD.  More waves spill, and
+// fewer hide less (one run: three per SIMD 0.63 ms, four 0.68, two 0.80).
 template <typename T, int INTERP>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DICE_TRANS_WPE))) void correlate_trans_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTransWaves))) void correlate_trans_kernel(
     KParams kp, DImage ref, DImage def, DSubsets ss, double *fields, PassArgs pa, int slot) {
   extern __shared__ float lds[];
   const Items items{pa.items, pa.item_count, ss.order};
@@ -4963,7 +4955,7 @@ template <typename T, int INTERP>
 hipError_t launch_trans_variant(const Launch &L, const KParams &kp, const DImage &ref, const DImage &def,
                                 const DSubsets &subs, double *fields, const PassArgs &pa, hipStream_t stream) {
   const size_t shm = (size_t)trans_lds_floats(subs.S, L.lds_floats_per_wave, false) * sizeof(float);
-  const int per_cu = (int)((160 * 1024) / shm) < 4 * DICE_TRANS_WPE ? (int)((160 * 1024) / shm) : 4 * DICE_TRANS_WPE;
+  const int per_cu = (int)((160 * 1024) / shm) < 4 * kTransWaves ? (int)((160 * 1024) / shm) : 4 * kTransWaves;
   const int groups = subs.n < L.num_cus * per_cu ? subs.n : L.num_cus * per_cu;
   hipLaunchKernelGGL((correlate_trans_kernel<T, INTERP>), dim3(groups), dim3(64), shm, stream, kp, ref, def, subs,
                      fields, pa, L.lds_floats_per_wave);
