@@ -927,12 +927,9 @@ static int vsg_enqueue(dice_hip_context *ctx, int window_size, double *d_fields,
   g.x0 = x0;
   g.y0 = y0;
   g.slack = 0.05 + 0x1p-21 * std::max({std::fabs(x0), std::fabs(x1), std::fabs(y0), std::fabs(y1)});
-  // radius windows: cells of side >= r / kVsgRings, so that every neighbour lies in the kVsgRings rings
-  // of cells around a subset (with the rounding of the float centres and distances), and of about one subset
-  // at least; k-nearest: cells holding about k subsets; at most 4000 cells along a side
-  const double side = knn ? std::sqrt((x1 - x0 + 1.0) * (y1 - y0 + 1.0) * knn / n)
-                          : std::max(((double)radius + 4.0 * g.slack) / dice_hip::kVsgRings,
-                                     std::sqrt((x1 - x0 + 1.0) * (y1 - y0 + 1.0) / n));
+  // k-nearest: cells holding about k subsets; at most 4000 cells along a side
+  const double area = (x1 - x0 + 1.0) * (y1 - y0 + 1.0);
+  const double side = knn ? std::sqrt(area * knn / n) : dice_hip::vsg_radius_cell(radius, g.slack, area, n);
   g.cell = std::max({side, 1.0, (x1 - x0) / 4000.0, (y1 - y0) / 4000.0});
   g.ncx = (int)std::floor((x1 - x0) / g.cell) + 1;
   g.ncy = (int)std::floor((y1 - y0) / g.cell) + 1;

@@ -266,7 +266,6 @@ hipError_t launch_vsg_grid(const double *fields, int n, bool radius_window, VsgG
 // squared float distance broken by subset id), the grid of any cell side.
 hipError_t launch_vsg_strain(const VsgGrid &g, float radius, int knn, double *fields, double *vsg, int n,
                              hipStream_t stream);
-constexpr int kVsgRings = 4;  // rings of cells around a subset's own that its radius may reach
 constexpr int kVsgFields = 7;
 constexpr int kVsgMaxK = 64;
 

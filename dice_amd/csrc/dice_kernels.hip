@@ -323,8 +323,8 @@ __global__ __launch_bounds__(256) void vsg_bounds_final_kernel(const double *par
 // there (an atomic per subset), the cells' first entries by a scan of the counts,
 // the ids at those places, and last each entry's rank by id among its cell's, so
 // that ids ascend within a cell whatever the order of arrival.  That rank reads
-// the entries of one cell per entry, never more than the strain's own scan does
-// after it.  Five launches of a few us: 155,236 subsets in 18,225 cells 27 us, a
+// the entries of one cell per entry, never more than the strain's own scan of a
+// valid subset does after it.  Five launches of a few us: 155,236 subsets in 18,225 cells 27 us, a
 // library radix sort of (cell, id) and the cells' ranges from it 72 us.
 //
 // Cell of subset i (the same arithmetic as vsg_subset's own cell).
@@ -406,6 +406,8 @@ __global__ void vsg_pack_kernel(const double *fields, const int *cells, const in
   const int c = cells[i];
   const int lo = start[c], hi = start[c + 1];
   int k = lo;
+  // (eight loads in flight: a crowded cell is read at its latency otherwise)
+#pragma unroll 8
   for (int t = lo; t < hi; ++t) k += arrived[t] < i ? 1 : 0;
   auto F = [&](int s) { return fields[(size_t)s * n + i]; };
   const bool failed = !(F(F_SIGMA) >= 0.0);
@@ -431,9 +433,11 @@ struct VsgTileReader {
 
 // Strain of subset i (see launch_vsg_strain); radius candidates through R.
 // L lanes of one wave per subset (L = 1, 2, 4, ...; lane `part` of them): the
-// radius scan deals the cell rows out round-robin and the lanes' sums are folded
-// by butterfly shuffles; part 0 finishes.  Every lane of a group must reach the
-// fold.  The candidates of a cell row are the cells within the circle's extent
+// radius scan deals the cell rows out round-robin, or the candidates of a row
+// when there are fewer than about five rows (8,000 subsets in 60 x 60 px and three far
+// away, window 61: 1.10 ms by rows, 0.52 ms by candidates), and the lanes' sums
+// are folded by butterfly shuffles; part 0 finishes.  Every lane of a group must
+// reach the fold.  The candidates of a cell row are the cells within the circle's extent
 // there (plus g.slack for the rounding of the float distances): with cells of
 // a quarter of the radius three in four lie in the circle, against one in three
 // of the 3 x 3 cells of the radius.  The kernel is bound by the 11 FP64 sums per
@@ -462,7 +466,10 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
   const int cj = min(max((int)floor((yi - g.y0) / g.cell), 0), g.ncy - 1);
   if (F(F_SIGMA, i) >= 0.0 && knn == 0) {
     const double rr = sqrt((double)r2) + g.slack;
-    for (int cy = cj - kVsgRings + part; cy <= min(cj + kVsgRings, g.ncy - 1); cy += L) {
+    const bool rows = 2.0 * g.cell <= (double)radius;  // (the same in every lane)
+    const int rings = rows ? kVsgRings : min(kVsgRings, (int)(rr / g.cell) + 1);
+    const int row0 = rows ? part : 0, row_step = rows ? L : 1, first = rows ? 0 : part, step = rows ? 1 : L;
+    for (int cy = cj - rings + row0; cy <= min(cj + rings, g.ncy - 1); cy += row_step) {
       if (cy < 0) continue;
       const double ya = g.y0 + cy * g.cell, yb = ya + g.cell;
       const double away = fmax(fmax(ya - yi, yi - yb) - g.slack, 0.0);
@@ -472,7 +479,7 @@ __device__ void vsg_subset(const VsgGrid &g, float radius, int knn, double *fiel
       const int cb = min(max((int)floor((xi + half - g.x0) / g.cell), 0), g.ncx - 1);
       const float4 *q = R.row(cy);
       const int e = g.cell_begin[cy * g.ncx + cb + 1];
-      for (int k = g.cell_begin[cy * g.ncx + ca]; k < e; ++k) {
+      for (int k = g.cell_begin[cy * g.ncx + ca] + first; k < e; k += step) {
         const float4 c = q[k];
         const float ddx = c.x - xf, ddy = c.y - yf;
         if (ddx * ddx + ddy * ddy < r2) add(c.z, c.w, ddx, ddy);

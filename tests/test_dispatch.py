@@ -1,5 +1,5 @@
 """The rule that picks a common-case Gauss-Newton kernel (dice_amd/csrc/dice_dispatch.h), compiled for the host
-and swept over subset sizes, counts and LDS slots."""
+and swept over subset sizes, counts and LDS slots, and the cell size of VSG radius windows there."""
 import os
 import subprocess
 
@@ -21,6 +21,7 @@ def rule(tmp_path_factory):
         out = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=60, check=True).stdout
         return np.array(out.split(), dtype=np.int64).reshape(len(rows), -1)
 
+    ask.exe = exe
     return ask
 
 
@@ -78,3 +79,16 @@ def test_border_subsets_of_small_frames_stay_with_the_others(rule, keys, most):
         for affine, listed in ((1, 0), (0, 1), (1, 1)):
             rows = [[(n, S, affine, 2560, keys, 1, listed, border) for n in (1, 300, 5000)] for border in (0, 1)]
             assert np.array_equal(rule(rows[0]), rule(rows[1])) and (rule(rows[1])[:, 0] != NONE).all()
+
+
+@pytest.mark.parametrize("radius", [1.0, 7.0, 20.0, 60.0, 300.0])
+@pytest.mark.parametrize("extent,n", [(60.0, 30000), (445.0, 8000), (1900.0, 445), (1900.0, 155236), (4096.0, 7)])
+def test_vsg_cells_between_a_quarter_of_the_radius_and_the_radius(rule, radius, extent, n):
+    """Four rings of cells reach the radius, and no cell is wider than it however few subsets there are for their
+    bounds (the one subset per cell on average in between)."""
+    slack = 0.05
+    cell = float(subprocess.check_output([rule.exe, str(radius), str(slack), str(extent ** 2), str(n)]))
+    assert 4.0 * cell >= radius + 4.0 * slack - 1e-9
+    assert cell <= max(radius, (radius + 4.0 * slack) / 4.0)
+    if radius / 2 < extent / n ** 0.5 < radius:
+        assert abs(cell - extent / n ** 0.5) < 1e-9
