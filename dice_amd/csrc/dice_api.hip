@@ -306,8 +306,9 @@ Launch current_launch(dice_hip_context *ctx, int mode) {
   const long long small = (long long)(0.8 * ctx->S) + 1;
   L.wide_only = ctx->S > 0 && small * small > L.lds_floats_per_wave ? 1 : 0;
   const int hw = ctx->S / 2;
-  L.border = ctx->S > 0 && (dice_hip::reaches_border(ctx->cx_lo, ctx->cx_hi, hw, ctx->dox, ctx->dw) ||
-                            dice_hip::reaches_border(ctx->cy_lo, ctx->cy_hi, hw, ctx->doy, ctx->dh));
+  L.border = ctx->S > 0 ? dice_hip::reaches_border(ctx->cx_lo, ctx->cx_hi, hw, ctx->dox, ctx->dw) |
+                              dice_hip::reaches_border(ctx->cy_lo, ctx->cy_hi, hw, ctx->doy, ctx->dh) << 2
+                        : 0;
   L.lane_simplex = ctx->max_count <= dice_hip::kLaneSimplexMaxPixels ? std::max(ctx->max_count, 1) : 0;
   return L;
 }

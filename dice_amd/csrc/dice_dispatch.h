@@ -51,15 +51,16 @@ struct CommonPass {
   bool keys;         // Keys fourth-order interpolation, or bilinear
   bool uncertainty;  // the uncertainty fields are formed
   bool listed;       // a part of the subsets, from a list (rounds of neighbour initialization)
-  bool border;       // a subset's box reaches the pixels that are dropped at the image border
+  int border;        // the sides of the image, 1 left, 2 right, 4 top and 8 bottom, at which a subset's
+                     // box reaches the pixels that are dropped there
   int num_cus;
 };
 
-// Does a box of centres [x0, x1] with half width hw reach the 4 px along the
-// border of an image of w pixels whose first has coordinate o, where warped
-// pixels are dropped?
-constexpr bool reaches_border(int x0, int x1, int hw, int o, int w) {
-  return (long long)x0 - hw < (long long)o + 4 || (long long)x1 + hw >= (long long)o + w - 4;
+// The ends, 1 low and 2 high, at which centres in [x0, x1] with half width hw
+// reach the 4 px along the border of an image of w pixels whose first has
+// coordinate o, where warped pixels are dropped.
+constexpr int reaches_border(int x0, int x1, int hw, int o, int w) {
+  return ((long long)x0 - hw < (long long)o + 4 ? 1 : 0) | ((long long)x1 + hw >= (long long)o + w - 4 ? 2 : 0);
 }
 
 // Can a subset that is translated by a fraction of a pixel be finished in the
@@ -95,11 +96,17 @@ inline int crew_max_subsets(const CommonPass &p) {
 // Keys and 40 with bilinear interpolation: a full grid of 35 x 35 px (8 bits), 961
 // subsets 175 against 232 us, 3,969 271 against 308, 5,929 361 against 340;
 // bilinear 3,969 221 against 300, 10,000 604 against 669, 12,100 488 against 468.
-// A round of neighbour initialization has a few subsets, mostly inside (324 points
-// of 27 x 27 px: none at the border 3.97 ms in the general kernel and 2.46 ms in
-// crews, one column of them 4.36 and 3.65 ms, all four sides 4.00 and 4.57 ms).
+// A round of neighbour initialization has a few subsets, and what counts is whether
+// nearly every round has one at the border, as where both ends of the columns that
+// the chain runs along do (361 points of 27 x 27 px, general kernel and crews: no
+// border 3.96 and 2.29 ms; left 4.38 and 3.67; left and right 4.45 and 3.83; top
+// and bottom 5.28 and 6.22; all four 5.35 and 6.32; three sides without the bottom
+// 5.06 and 4.81, 21 x 21 px 3.26 and 3.57, 35 x 35 px 3.65 and 3.73).
 inline bool general_for_border(const CommonPass &p) {
-  return p.border && !p.affine && !p.listed && p.n <= (p.keys ? 20 : 40) * p.num_cus;
+  if (!p.border || p.affine) return false;
+  const bool x = (p.border & 3) == 3, y = (p.border & 12) == 12;
+  if (p.listed) return y || (x && (p.border & 12) != 0);
+  return p.n <= (p.keys ? 20 : 40) * p.num_cus;
 }
 
 // All six parameters: the lean kernel; translation only: its own kernel; few

@@ -133,7 +133,7 @@ struct Launch {
   int wide_floats;             // batched: LDS window of correlate_wide_kernel
   int wide_only;               // batched: no subset's window can fit a wave's slot
   int num_cus;
-  int border;                  // batched: square subsets of which one reaches the deformed image's border
+  int border;                  // batched: the sides of the deformed image that square subsets reach (CommonPass)
 };
 
 // Subsets of at most this many pixels run the Nelder-Mead iterations of the

@@ -751,7 +751,7 @@ static hipError_t launch_pass(bool simplex, int storage, const Launch &L, const 
       pl.ov_count = work + kWorkLeanCount;
       const CommonKernel common = common_kernel(
           CommonPass{subs.n, subs.S, np == 3, L.lds_floats_per_wave, kp.interp != 0, kp.uncertainty != 0,
-                     pa.items != nullptr, L.border != 0, L.num_cus});
+                     pa.items != nullptr, L.border, L.num_cus});
       e = hipSuccess;
       if (common == CommonKernel::kCrew)
         e = launch_gn_crew(storage, kp.interp, np == 0, L, kp, ref, def, subs, fields, pl, stream);

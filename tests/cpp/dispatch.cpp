@@ -6,11 +6,11 @@
 #include "../../dice_amd/csrc/dice_dispatch.h"
 
 using dice_hip::reaches_border;
-static_assert(!reaches_border(21, 78, 17, 0, 100) && reaches_border(20, 50, 17, 0, 100) &&
-                  reaches_border(50, 79, 17, 0, 100),
+static_assert(reaches_border(21, 78, 17, 0, 100) == 0 && reaches_border(20, 50, 17, 0, 100) == 1 &&
+                  reaches_border(50, 79, 17, 0, 100) == 2 && reaches_border(0, 99, 17, 0, 100) == 3,
               "a box from 4 to 95 of 100 pixels keeps them all");
-static_assert(!reaches_border(71, 128, 17, 50, 100) && reaches_border(21, 78, 17, 50, 100) &&
-                  reaches_border(70, 71, 17, 50, 100) && reaches_border(128, 129, 17, 50, 100),
+static_assert(reaches_border(71, 128, 17, 50, 100) == 0 && reaches_border(21, 78, 17, 50, 100) == 1 &&
+                  reaches_border(70, 71, 17, 50, 100) == 1 && reaches_border(128, 129, 17, 50, 100) == 2,
               "the same in an image that begins at 50");
 
 int main(int argc, char **argv) {
@@ -23,7 +23,7 @@ int main(int argc, char **argv) {
   while (std::scanf("%d %d %d %d %d %d %d %d", &n, &S, &affine, &slot, &keys, &unc, &listed, &border) == 8)
     std::printf("%d %zu %zu\n",
                 (int)dice_hip::common_kernel(
-                    {n, S, affine != 0, slot, keys != 0, unc != 0, listed != 0, border != 0, 256}),
+                    {n, S, affine != 0, slot, keys != 0, unc != 0, listed != 0, border, 256}),
                 sizeof(float) * dice_hip::trans_lds_floats(S, slot, false),
                 sizeof(float) * dice_hip::trans_lds_floats(S, slot, true));
   return 0;

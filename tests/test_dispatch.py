@@ -69,16 +69,30 @@ def test_number_of_subsets_that_crews_take(rule, S, affine, listed, most):
     assert rule(rows)[:, 0].tolist() == [CREW, CREW, many, many]
 
 
+LEFT, RIGHT, TOP, BOTTOM = 1, 2, 4, 8
+
+
 @pytest.mark.parametrize("keys,most", [(1, 5120), (0, 10240)])
 def test_border_subsets_of_small_frames_stay_with_the_others(rule, keys, most):
-    """Translation only with a subset at the border: the general kernel takes the whole frame up to a size; lists and
+    """Translation only with a subset at the border: the general kernel takes the whole frame up to a size;
     six-parameter frames (whose lean kernel there always was) as without one."""
     for S in (9, 35, 41):
-        rows = [(n, S, 0, 2560, keys, 1, 0, 1) for n in (1, 1024, 1025, most, most + 1)]
-        assert rule(rows)[:, 0].tolist() == [NONE] * 4 + [TRANS]
-        for affine, listed in ((1, 0), (0, 1), (1, 1)):
-            rows = [[(n, S, affine, 2560, keys, 1, listed, border) for n in (1, 300, 5000)] for border in (0, 1)]
-            assert np.array_equal(rule(rows[0]), rule(rows[1])) and (rule(rows[1])[:, 0] != NONE).all()
+        for border in range(1, 16):
+            rows = [(n, S, 0, 2560, keys, 1, 0, border) for n in (1, 1024, 1025, most, most + 1)]
+            assert rule(rows)[:, 0].tolist() == [NONE] * 4 + [TRANS]
+            for listed in (0, 1):
+                rows = [[(n, S, 1, 2560, keys, 1, listed, b) for n in (1, 300, 5000)] for b in (0, border)]
+                assert np.array_equal(rule(rows[0]), rule(rows[1])) and (rule(rows[1])[:, 0] != NONE).all()
+
+
+def test_border_of_a_chain(rule):
+    """Rounds of neighbour initialization, translation only: the general kernel where the chain's columns reach the
+    border at both ends or three sides do, crews elsewhere."""
+    for border in range(16):
+        ends = border & (TOP | BOTTOM) == TOP | BOTTOM
+        three = bin(border).count("1") >= 3
+        got = rule([(n, 27, 0, 2560, 1, 1, 1, border) for n in (1, 361, 1024)])[:, 0].tolist()
+        assert got == [NONE if ends or three else CREW] * 3, border
 
 
 @pytest.mark.parametrize("radius", [1.0, 7.0, 20.0, 60.0, 300.0])
