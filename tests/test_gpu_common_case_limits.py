@@ -147,3 +147,30 @@ def test_large_motion(u, v, interp, step):
         assert len(cx) > (5120 if interp == dh.KEYS_FOURTH else 10240) or step == 45
         b = run(ctx, q, ref, de, cx, cy, S, f0)
     check(a, b)
+
+
+@pytest.mark.parametrize("step", [6, 45], ids=["wave", "crew"])
+@pytest.mark.parametrize("interp", [dh.KEYS_FOURTH, dh.BILINEAR], ids=["keys", "bilinear"])
+def test_sub_images_at_offsets(interp, step):
+    """Reference and deformed images cut out at different places, so that the unshifted pixel lies 11 and 7 px from
+    where the subset is found."""
+    w, h, S = 360, 340, 31
+    full_ref, full_def = images(w, h, 0.4, -0.3, 57)
+    ref, de = full_ref[9:, 20:], full_def[16:330, 31:350]
+    gx, gy = np.meshgrid(np.arange(60, 300, step), np.arange(50, 290, step))
+    cx, cy = gx.ravel().astype(float), gy.ravel().astype(float)
+    f0 = dh.new_fields(cx, cy)
+    p, q = params(interp), params(interp)
+    q.initial_gamma_threshold = 1e9  # the general kernel
+    with dh.Context(0) as ctx:
+        out = []
+        for k in (p, q):
+            ctx.set_params(k)
+            ctx.set_ref_image(np.ascontiguousarray(ref))
+            ctx.set_def_image(np.ascontiguousarray(de))
+            ctx.set_image_offsets(20, 9, 31, 16)
+            ctx.set_subsets(cx, cy, S)
+            out.append(ctx.correlate(f0.copy(), first_frame=False))
+            if k is p:
+                assert ctx.handover_counts() == (0, 0, 0)
+    check(*out)
